@@ -374,8 +374,8 @@ class Context:
         return m
 
     def set_skew(self, skew, rotate=False):
-        """Height skew of the work items (< 0: automatic) and the per-strip
-        rotation of its levels; results do not depend on either."""
+        """Height skew of the work items (< 0: automatic) and whether the
+        strips are cut running on; results do not depend on either."""
         _check(load().fivonagi_set_skew(self._h, C.c_double(skew), int(bool(rotate))))
 
     def autotune(self, trial_steps=20):

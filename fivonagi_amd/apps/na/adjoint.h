@@ -55,10 +55,11 @@ __device__ __forceinline__ void lim_part(float n, float dot, float& h, float& qd
 // The limited fluxes of interface f as the step kernel forms them (same
 // call), and the transpose's quantities.  dl_p = W_p . W_p(k-1),
 // dr_p = W_p . W_p(k+1).
+template <bool kL3Product>
 __device__ __forceinline__ void limiter_rec(const Iface& f, float dl1, float dr1, float dl2,
                                             float dr2, float dl3, float dr3, float dtd,
                                             float P[3], float M[3], LimT& t) {
-  fvna::limited_flux(f, dl1, dr1, dl2, dr2, dl3, dr3, dtd, P, M);
+  fvna::limited_flux<kL3Product>(f, dl1, dr1, dl2, dr2, dl3, dr3, dtd, P, M);
   const Waves& w = f.w;
   const float n1 = fvna::fma_(w.a1, w.a1, fvna::fma_(w.w21, w.w21, w.w31 * w.w31));
   const float n2 = fvna::fma_(w.a2, w.a2, fvna::fma_(w.w22, w.w22, w.w32 * w.w32));

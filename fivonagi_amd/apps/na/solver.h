@@ -20,6 +20,9 @@
 //     (see limited_flux).
 //   * the two sweep updates (step + writeLimiters) are fused into one:
 //     q - dtd*((apdq - fadd)(k) + (amdq + fadd)(k+1)).
+//   * every multiply-add is written out (fma_) and contraction is off in these
+//     bodies: which products fuse is part of the result, and it must not
+//     depend on how a kernel that inlines them is laid out.
 #ifndef FIVONAGI_APPS_NA_SOLVER_H
 #define FIVONAGI_APPS_NA_SOLVER_H
 
@@ -64,6 +67,12 @@ __device__ __forceinline__ R add_nc(R a, R b) {
   return a + b;
 }
 
+// q - d * flux in one rounding: a sweep's update of a cell
+template <typename R>
+__device__ __forceinline__ R sub_prod(R q, R d, R flux) {
+  return fma_(-d, flux, q);
+}
+
 // max(a, b) of finite values as one v_med3_f32 (median of a, b, FLT_MAX;
 // with +inf the intrinsic is folded back into a maxnum).
 // fmaxf must quiet signalling NaNs in IEEE mode, so on values the compiler
@@ -90,47 +99,61 @@ template <typename R>
 struct IfaceT {
   WavesT<R> w;
   R L1, L2, L3;         // speeds s1, s2, s3
+  R s2, rS;             // L3 = s2 * rS (limited_flux's kL3Product)
   R smax;               // max |s_p| (|L3| <= max(|L1|,|L2|) since L3 is their mean)
   bool bad;             // tmp3 < 0: imaginary eigenvalue (simError = 2)
 };
 typedef WavesT<float> Waves;
 typedef IfaceT<float> Iface;
 
-// Riemann solve at the interface between cell L and cell R.
-// r1 = rho', n = normal momentum, t = tangential momentum,
-// un/ut = n/rho, t/rho of the same cell (precomputed once per cell).
-// hbeta = BETA - 1.  The fluctuations amdq/apdq (fv.h:141-180) are not
-// formed here: limited_flux() folds them with the correction flux.
+// Sums and differences of the two cells L, R of an interface, all that its
+// Riemann solve needs of them.  r1 = rho', n = normal momentum, t = tangential
+// momentum, un/ut = n/rho, t/rho of the same cell (precomputed once per cell).
 // Every L operand enters only sums and differences with its R partner, so
 // when L is the neighbouring lane's value the cross-lane move folds into
 // the add/subtract (DPP operand).
 template <typename R>
-__device__ __forceinline__ void riemann(R r1L, R nL, R tL, R unL, R utL, R r1R, R nR, R tR,
-                                        R unR, R utR, R hbeta, IfaceT<R>& f) {
-  const R s1 = add_nc(r1L, r1R);                    // 2 (Z1 - 1)   fv.h:91
-  const R s2 = add_nc(unL, unR);                    // 2 Z2         fv.h:92
-  const R s3 = add_nc(utL, utR);                    // 2 Z3         fv.h:93
-  const R drho = r1R - r1L, dn = nR - nL, dtg = tR - tL;
+struct JumpT {
+  R s1, s2, s3;         // 2 (Z1 - 1), 2 Z2, 2 Z3   fv.h:91-93
+  R drho, dn, dtg;
+};
+typedef JumpT<float> Jump;
+template <typename R>
+__device__ __forceinline__ JumpT<R> jump(R r1L, R nL, R tL, R unL, R utL, R r1R, R nR, R tR,
+                                         R unR, R utR) {
+#pragma clang fp contract(off)
+  return JumpT<R>{r1L + r1R, unL + unR, utL + utR, r1R - r1L, nR - nL, tR - tL};
+}
+
+// Riemann solve at an interface.  hbeta = BETA - 1.  The fluctuations
+// amdq/apdq (fv.h:141-180) are not formed here: limited_flux() folds them with
+// the correction flux.
+template <typename R>
+__device__ __forceinline__ void riemann(const JumpT<R>& j, R hbeta, IfaceT<R>& f) {
+#pragma clang fp contract(off)
+  const R s1 = j.s1, s2 = j.s2, s3 = j.s3, drho = j.drho, dn = j.dn, dtg = j.dtg;
   const R S1 = s1 + R(2);                           // 2 Z1
-  const R tmp1 = s2 * rcp(S1);                      // Z2/Z1        fv.h:96
+  const R rS = rcp(S1);
+  const R tmp1 = s2 * rS;                           // Z2/Z1        fv.h:96
   // tmp1^2 - 2 Z2 tmp1 + 1 + 2 (BETA-1)(Z1-1)                      fv.h:97-101
-  const R tmp3 = fma_(tmp1, tmp1 - s2, fma_(hbeta, s1, R(1)));
+  const R tmp3 = fma_(tmp1, fma_(s2, rS, -s2), fma_(hbeta, s1, R(1)));
   f.bad = !(tmp3 >= R(0));                          // fv.h:102
   const R rs = rsq(tmp3);
-  const R sq = tmp3 * rs;                           // sqrt(tmp3)
-  const R L1 = tmp1 + sq, L2 = tmp1 - sq;           // fv.h:105-107
+  const R L1 = fma_(tmp3, rs, tmp1), L2 = fma_(-tmp3, rs, tmp1);   // tmp1 +- sqrt, fv.h:105-107
   f.L1 = L1; f.L2 = L2; f.L3 = tmp1;
+  f.s2 = s2; f.rS = rS;
   // fv.h:110-113: A_p = (L_p Z3 - 2 Z2 Z3)/(L_p Z1 - Z3) = s3 (L_p - s2)/(L_p S1 - s3),
   // with one reciprocal for both denominators (each is ~ +-2)
   const R d1 = fma_(L1, S1, -s3), d2 = fma_(L2, S1, -s3);
   const R srd = s3 * rcp(d1 * d2);
   const R A1 = (L1 - s2) * (d2 * srd);
   const R A2 = (L2 - s2) * (d1 * srd);
-  const R a1 = fma_(-drho, L2, dn) * (R(0.5) * rs);             // fv.h:116-117
-  const R a2 = drho - a1;                                       // fv.h:118
+  const R hrs = R(0.5) * rs, dnl = fma_(-drho, L2, dn);
+  const R a1 = dnl * hrs;                                       // fv.h:116-117
+  const R a2 = fma_(-dnl, hrs, drho);                           // fv.h:118
   f.w.a1 = a1; f.w.w21 = a1 * L1; f.w.w31 = a1 * A1;
   f.w.a2 = a2; f.w.w22 = a2 * L2; f.w.w32 = a2 * A2;
-  f.w.a3 = dtg - (f.w.w31 + f.w.w32);                           // fv.h:119-125
+  f.w.a3 = dtg - fma_(a1, A1, f.w.w32);                         // fv.h:119-125
   f.smax = fmax2(fabs(L1), fabs(L2));
 }
 
@@ -142,6 +165,7 @@ __device__ __forceinline__ void riemann(R r1L, R nL, R tL, R unL, R utL, R r1R, 
 // turns into 0 (finite), and the select is skipped.
 template <typename R>
 __device__ __forceinline__ R philim_half(R wnorm2, R dot) {
+#pragma clang fp contract(off)
   const R r = dot * rcp(wnorm2);
   return clamp01(min_(fma_(R(0.25), r, R(0.25)), r));
 }
@@ -150,10 +174,12 @@ __device__ __forceinline__ R philim_half(R wnorm2, R dot) {
 // (mul, then multiply-accumulates with b as the plain multiplicand)
 template <typename R>
 __device__ __forceinline__ R dot1(const WavesT<R>& a, const WavesT<R>& b) {
+#pragma clang fp contract(off)
   return fma_(b.a1, a.a1, fma_(b.w21, a.w21, b.w31 * a.w31));
 }
 template <typename R>
 __device__ __forceinline__ R dot2(const WavesT<R>& a, const WavesT<R>& b) {
+#pragma clang fp contract(off)
   return fma_(b.a2, a.a2, fma_(b.w22, a.w22, b.w32 * a.w32));
 }
 
@@ -164,10 +190,14 @@ __device__ __forceinline__ R dot2(const WavesT<R>& a, const WavesT<R>& b) {
 // with c_p = |s_p| (1 - |s_p| dt/d) phi_p / 2 = |s_p| (1 - |s_p| dt/d) philim_half.  A wave with s_p = 0 enters
 // neither fluctuation, as in the reference.
 // dotl_p = W_p . W_p(k-1), dotr_p = W_p . W_p(k+1); upwind by sign(s_p).
-template <typename R>
+// kL3Product: be_3 = L3 - al_3 from the product L3 = s2 rS with one rounding
+// (the x sweep, which has both factors at hand; the y sweep keeps L3 alone
+// in its window).
+template <bool kL3Product, typename R>
 __device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R dotl1, R dotr1, R dotl2,
                                              R dotr2, R dotl3, R dotr3, R dtd, R P[3],
                                              R M[3]) {
+#pragma clang fp contract(off)
   const WavesT<R>& w = f.w;
   const R n1 = fma_(w.a1, w.a1, fma_(w.w21, w.w21, w.w31 * w.w31));
   const R n2 = fma_(w.a2, w.a2, fma_(w.w22, w.w22, w.w32 * w.w32));
@@ -176,13 +206,15 @@ __device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R dotl1, R dotr
   const R h2 = philim_half(n2, f.L2 > R(0) ? dotl2 : dotr2);
   const R h3 = philim_half(n3, f.L3 > R(0) ? dotl3 : dotr3);
   const R s1 = fabs(f.L1), s2 = fabs(f.L2), s3 = fabs(f.L3);
-  const R c1 = s1 * fma_(-s1, dtd, R(1)) * h1;
-  const R c2 = s2 * fma_(-s2, dtd, R(1)) * h2;
-  const R c3 = s3 * fma_(-s3, dtd, R(1)) * h3;
+  // c_p = g_p h_p
+  const R g1 = s1 * fma_(-s1, dtd, R(1));
+  const R g2 = s2 * fma_(-s2, dtd, R(1));
+  const R g3 = s3 * fma_(-s3, dtd, R(1));
   // al_p = max(s_p, 0) - c_p; be_p = min(s_p, 0) + c_p = s_p - al_p
-  const R al1 = fmax2(f.L1, R(0)) - c1, be1 = f.L1 - al1;
-  const R al2 = fmax2(f.L2, R(0)) - c2, be2 = f.L2 - al2;
-  const R al3 = fmax2(f.L3, R(0)) - c3, be3 = f.L3 - al3;
+  const R al1 = fma_(-g1, h1, fmax2(f.L1, R(0))), be1 = f.L1 - al1;
+  const R al2 = fma_(-g2, h2, fmax2(f.L2, R(0))), be2 = f.L2 - al2;
+  const R al3 = fma_(-g3, h3, fmax2(f.L3, R(0)));
+  const R be3 = kL3Product ? fma_(f.s2, f.rS, -al3) : f.L3 - al3;
   P[0] = fma_(al1, w.a1, al2 * w.a2);
   P[1] = fma_(al1, w.w21, al2 * w.w22);
   P[2] = fma_(al3, w.a3, fma_(al1, w.w31, al2 * w.w32));

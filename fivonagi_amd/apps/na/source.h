@@ -19,6 +19,7 @@ namespace fvna {
 // turns that into a drift of T.
 template <typename R>
 __device__ __forceinline__ R source_increment(R ddx2, R ddy2, R u, R u_we, R u_s, R u_n) {
+#pragma clang fp contract(off)
   return fma_(ddx2, fma_(R(-2), u, u_we), ddy2 * (fma_(R(-2), u, u_s) + u_n));
 }
 

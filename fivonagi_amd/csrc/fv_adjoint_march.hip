@@ -235,7 +235,9 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
 
     // ---- y interface r (rows r-1 | r): normal = q3, tangential = q2 ----
     fvna::Iface fn;
-    fvna::riemann(b1.q1, b1.q3, b1.q2, b1.un, b1.ut, bn.q1, bn.q3, bn.q2, bn.un, bn.ut, hbeta, fn);
+    fvna::riemann(fvna::jump(b1.q1, b1.q3, b1.q2, b1.un, b1.ut, bn.q1, bn.q3, bn.q2, bn.un,
+                             bn.ut),
+                  hbeta, fn);
     float dln[3];
     dln[0] = fvna::dot1(fn.w, f1.w);
     dln[1] = fvna::dot2(fn.w, f1.w);
@@ -243,7 +245,7 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
     // ---- y limiter at interface r-1 ----
     float P1[3], M[3];
     fvad::LimT lim1;
-    fvad::limiter_rec(f1, dl1[0], dln[0], dl1[1], dln[1], dl1[2], dln[2], dty, P1, M, lim1);
+    fvad::limiter_rec<false>(f1, dl1[0], dln[0], dl1[1], dln[1], dl1[2], dln[2], dty, P1, M, lim1);
 
     // The rows before y0 only warm up the windows of the forward recompute
     // (the y interfaces and limiters the first emitted rows need); everything
@@ -260,9 +262,9 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
       const bool row_int = m >= 2 && m <= ny - 3;
       const bool upd = col_int && row_int;
       const float dtyu = row_int ? dty_c : 0.0f, dtxu = row_int ? dtx_c : 0.0f;
-      const float y1q = b2.q1 - dtyu * (Pp[0] + M[0]);
-      const float y3q = b2.q3 - dtyu * (Pp[1] + M[1]);
-      const float y2q = b2.q2 - dtyu * (Pp[2] + M[2]);
+      const float y1q = fvna::sub_prod(b2.q1, dtyu, Pp[0] + M[0]);
+      const float y3q = fvna::sub_prod(b2.q3, dtyu, Pp[1] + M[1]);
+      const float y2q = fvna::sub_prod(b2.q2, dtyu, Pp[2] + M[2]);
 
       // ---- x sweep on row m: normal = q2, tangential = q3 ----
       const float ir = fvna::rcp(1.0f + y1q);
@@ -270,7 +272,8 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
       const float l1 = shr1(y1q), l2 = shr1(y2q), l3 = shr1(y3q);
       const float lun = shr1(un), lut = shr1(ut);
       fvna::Iface fx;
-      fvna::riemann(l1, l2, l3, lun, lut, y1q, y2q, y3q, un, ut, hbeta, fx);
+      const fvna::Jump jx = fvna::jump(l1, l2, l3, lun, lut, y1q, y2q, y3q, un, ut);
+      fvna::riemann(jx, hbeta, fx);
       fvna::Waves wl;
       wl.a1 = shr1(fx.w.a1); wl.w21 = shr1(fx.w.w21); wl.w31 = shr1(fx.w.w31);
       wl.a2 = shr1(fx.w.a2); wl.w22 = shr1(fx.w.w22); wl.w32 = shr1(fx.w.w32);
@@ -280,12 +283,12 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
       const float drx1 = shl1(dlx1), drx2 = shl1(dlx2), drx3 = shl1(dlx3);
       float PX[3], MX[3];
       fvad::LimT limx;
-      fvad::limiter_rec(fx, dlx1, drx1, dlx2, drx2, dlx3, drx3, dtx, PX, MX, limx);
+      fvad::limiter_rec<true>(fx, dlx1, drx1, dlx2, drx2, dlx3, drx3, dtx, PX, MX, limx);
       const float mr0 = shl1(MX[0]), mr1 = shl1(MX[1]), mr2 = shl1(MX[2]);
       XRow xc;
-      xc.q1 = y1q - dtxu * (mr0 + PX[0]);
-      xc.q2 = y2q - dtxu * (mr1 + PX[1]);
-      xc.q3 = y3q - dtxu * (mr2 + PX[2]);
+      xc.q1 = fvna::sub_prod(y1q, dtxu, mr0 + PX[0]);
+      xc.q2 = fvna::sub_prod(y2q, dtxu, mr1 + PX[1]);
+      xc.q3 = fvna::sub_prod(y3q, dtxu, mr2 + PX[2]);
       const float ir2 = fvna::rcp(1.0f + xc.q1);
       xc.u = xc.q2 * ir2;
       xc.v = xc.q3 * ir2;
@@ -357,8 +360,7 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
         fvad::add_scaled(gx, kl, wl);
         fvad::add_scaled(gx, kr, wr);
       }
-      fvad::SumAdj sx = fvad::riemann_bw(fvna::add_nc(l1, y1q), fvna::add_nc(lun, un),
-                                         fvna::add_nc(lut, ut), y1q - l1, y2q - l2, hbeta, fx, gx);
+      fvad::SumAdj sx = fvad::riemann_bw(jx.s1, jx.s2, jx.s3, jx.drho, jx.dn, hbeta, fx, gx);
       sx = keep_if(col_x, sx);
       {
         // cell k: interface k's R part and interface k+1's L part (lane k+1)

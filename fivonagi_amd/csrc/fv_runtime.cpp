@@ -23,7 +23,7 @@
 #include "fv_types.h"
 
 extern "C" hipError_t fv_launch_step(const fv::InstDesc* insts, const fv::WorkItem* items,
-                                     const uint64_t* rowmask, int n_items, int phase,
+                                     const uint64_t* rowmask, int n_groups, int phase,
                                      int n_inst, fv::Ctl* ctl0, fv::SyncSlots* sync0, int bc0,
                                      int ext, int fp64, hipStream_t stream);
 extern "C" hipError_t fv_launch_settle(const fv::InstDesc* insts, int n_inst, int phase,
@@ -73,14 +73,15 @@ struct fivonagi_ctx {
   int n_inst = 0;
   std::vector<fivonagi_params> params;
   std::vector<fv::InstDesc> desc;          // host copy of the instance table
-  std::vector<fv::WorkItem> items;
-  std::vector<uint64_t> rowmask;           // CFL lane mask per item row (fv::WorkItem::mrow)
+  std::vector<fv::WorkItem> items;         // kGroupWaves places per workgroup
+  std::vector<uint64_t> rowmask;           // CFL lane mask per strip row (fv::WorkItem::mrow)
+  int n_groups() const { return (int)(items.size() / fv::kGroupWaves); }
   bool fp64 = false;                       // state and arithmetic in double
   bool md_any = false;                     // some instance has a moving window
   bool ext_any = false;                    // ... or the HIFU boundary (extended kernel)
   float skew = -1.0f;                      // height skew of the work items (< 0: automatic)
   float skew_used = 0.0f;                  // the skew of the current work list
-  bool rotate = false;                     // level pattern rotated per strip (chunk_bounds)
+  bool rotate = false;                     // strips cut running on (build_work)
   bool rotate_used = false;
   long cus = 256;                          // CUs of the device
   int per_cu = 16;                         // resident step waves per CU
@@ -169,8 +170,9 @@ void build_items(fivonagi_ctx* c, int auto_h, float skew, bool rotate) {
   std::vector<int> masks(c->n_inst);
   for (int k = 0; k < c->n_inst; ++k) masks[k] = c->desc[k].cfl_mask;
   fvh::WorkList wl;
-  fvh::build_work(c->params, masks, c->fold_bits, c->cus, c->per_cu, auto_h, skew, rotate, wl);
-  c->items = std::move(wl.items);
+  fvh::build_work(c->params, masks, c->fold_bits, c->cus, c->per_cu, auto_h, skew, rotate, wl,
+                  c->fp64 ? 48 : 24);
+  c->items = fvh::launch_items(wl, c->cus);
   c->rowmask = std::move(wl.rowmask);
   for (int k = 0; k < c->n_inst; ++k) c->desc[k].n_items = wl.n_items[k];
   c->skew_used = wl.skew_used;
@@ -265,7 +267,7 @@ hipError_t launch_phase(fivonagi_ctx* c, int phase) {
         fv_launch_taylor_ghosts(c->d_desc, c->n_inst, c->taylor_ring, phase, c->stream);
     if (e != hipSuccess) return e;
   }
-  hipError_t e = fv_launch_step(c->d_desc, c->d_items, c->d_rowmask, (int)c->items.size(),
+  hipError_t e = fv_launch_step(c->d_desc, c->d_items, c->d_rowmask, c->n_groups(),
                                 phase, c->n_inst, c->d_ctl, c->d_sync, c->params[0].bc,
                                 c->ext_any || c->keep_hist ? 1 : 0, c->fp64 ? 1 : 0,
                                 c->stream);
@@ -1255,7 +1257,7 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
       const fv::InstDesc* di = d_rdesc + (size_t)s * ni;
       if (c->taylor_ring > 0)
         HIP_TRY(fv_launch_taylor_ghosts(di, ni, c->taylor_ring, 0, c->stream));
-      HIP_TRY(fv_launch_step(di, c->d_items, c->d_rowmask, (int)c->items.size(), 0, ni,
+      HIP_TRY(fv_launch_step(di, c->d_items, c->d_rowmask, c->n_groups(), 0, ni,
                              one ? d_rctl + 2 * (size_t)s : nullptr, one ? d_rsync : nullptr,
                              c->params[0].bc, c->ext_any ? 1 : 0, 0, c->stream));
     }
@@ -1361,13 +1363,20 @@ int fivonagi_step_noalloc(const fivonagi_params* p, float* const q[6], int64_t n
   build_items(&tmp, auto_rows(tmp.params, tmp.cus * tmp.per_cu), tmp.skew, tmp.rotate);
   fv::InstDesc d = tmp.desc[0];
 
-  // the buffer's layout, each part 256-byte aligned
+  // the buffer's layout, each part 256-byte aligned.  Where the rest leaves too
+  // little room for the items (grids of a few rows and very many strips), the
+  // tallest ones
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t o = off;
     off = (off + bytes + 255) & ~(size_t)255;
     return o;
   };
+  const size_t others = sizeof(fv::InstDesc) + 2 * sizeof(fv::Ctl) + 3 * sizeof(fv::SyncSlots) +
+                        sizeof(float) * (h.ec.size() + h.es.size() + h.tab.size()) +
+                        sizeof(uint64_t) * tmp.rowmask.size() + 8 * 256;
+  if (others + sizeof(fv::WorkItem) * tmp.items.size() > cap)
+    build_items(&tmp, 1 << 20, 0.0f, false);
   const size_t o_desc = take(sizeof(fv::InstDesc));
   const size_t o_ctl = take(2 * sizeof(fv::Ctl));
   const size_t o_sync = take(3 * sizeof(fv::SyncSlots));
@@ -1420,7 +1429,7 @@ int fivonagi_step_noalloc(const fivonagi_params* p, float* const q[6], int64_t n
   const fv::InstDesc* d_desc = (const fv::InstDesc*)(dev + o_desc);
   const fv::WorkItem* d_items = (const fv::WorkItem*)(dev + o_items);
   const uint64_t* d_mask = (const uint64_t*)(dev + o_mask);
-  const int n_items = (int)tmp.items.size();
+  const int n_groups = tmp.n_groups();
   const int ext = h.ext ? 1 : 0;
   int64_t a = 0;                 // attempts launched by this call (phase = a mod 6)
   fv::Ctl now = c0;
@@ -1431,7 +1440,7 @@ int fivonagi_step_noalloc(const fivonagi_params* p, float* const q[6], int64_t n
       const int phase = (int)(a % 6);
       if (h.taylor_ring > 0)
         HIP_TRY(fv_launch_taylor_ghosts(d_desc, 1, h.taylor_ring, phase, stream));
-      HIP_TRY(fv_launch_step(d_desc, d_items, d_mask, n_items, phase, 1, d.ctl, d.sync, p->bc,
+      HIP_TRY(fv_launch_step(d_desc, d_items, d_mask, n_groups, phase, 1, d.ctl, d.sync, p->bc,
                              ext, 0, stream));
     }
     // the control block after the last attempt (fv_settle_kernel), read back

@@ -6,19 +6,35 @@
 // in x, 21 reduceCFL launches, reduceCFL2, source, update_T, update_dt and the
 // seven blocking device->host copies.
 //
-// Work decomposition ("march"): one wave64 per work item.  Lane l owns column
-// x0 - 3 + l; the wave marches upward through rows [y0-3, y1+3) of its strip:
+// Work decomposition ("march"): one wave64 per work item, up to four items of
+// a strip, one above the other, per workgroup.  Lane l owns column x0 - 3 + l;
+// the wave marches upward through the rows of its strip:
 //   load row r+1 (prefetch; boundary rules applied when the row is consumed)
 //   -> y-Riemann at interface r        (registers, same lane)
 //   -> y-limiter at interface r-1      (3-interface register window)
 //   -> q_y(r-2)                        (first + second order, fused)
 //   -> x-Riemann/limiter on row r-2    (neighbours via DPP wave_shr/wave_shl)
 //   -> q_xy(r-2)
-//   -> source on row r-3               (3-row register window + DPP)
-//   -> store row r-3 (lanes 3..60)
+//   -> source on row r-4               (3-row register window + DPP)
+//   -> store row r-4 (lanes 3..60)
 // The loop is unrolled three times so the period-3 register windows rotate
-// by renaming instead of moves.  No LDS and no barriers: the 3-column halo on
-// each side makes the waves independent.
+// by renaming instead of moves.
+//
+// Seams: output row y needs interfaces y-2 .. y+3, so a lone item of H rows
+// solves H+5 y interfaces, H+3 y limiters and H+2 x rows.  Inside a workgroup
+// nothing is solved twice: each wave leaves what its first rows make (the
+// first interface, the next one's dot products and M, the first two rows of
+// q_xy) in LDS, one barrier after its sixth row publishes it, and the wave
+// below ends its march on those values.  Only the topmost wave of a workgroup
+// marches the five rows past its last.
+//
+// The march is bound by VALU issue (about 270 instructions per row of a wave)
+// and, on small grids, by the length of the longest wave's march, so both gain
+// from rows not repeated: a wave of 18 rows marched 21.3 rows' worth alone and
+// 18.8 in a group of four, and a group of 16 rows marches 6 steps where a lone
+// item needed 17.  Per step, one wave per workgroup against groups of four:
+// 4096x1024 40.7 -> 36.9 us, 2048x2048 43.2 -> 37.5, 1024x1024 20.9 -> 16.6,
+// 400x400 16.4 -> 8.7 (FP32).  Waves per group: two gave 38.4 on 4096x1024.
 //
 // CFL and accept/reject: each wave reduces its cells' cfl to one float and
 // folds it into its group's 128-byte line (8 groups per instance) with one
@@ -96,8 +112,8 @@ __device__ __forceinline__ void stg(gdouble* base, uint32_t off, double v) {
   *(gdouble*)((gchar*)base + off) = v;
 }
 
-// s_waitcnt vmcnt(0) with expcnt and lgkmcnt left at their maxima (gfx9 encoding)
-constexpr int kWaitVm0 = 0x0F70;
+// s_waitcnt vmcnt(0) lgkmcnt(0) with expcnt left at its maximum (gfx9 encoding)
+constexpr int kWaitLoads = 0x0070;
 
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ int64_t uni64(int64_t v) {
@@ -352,6 +368,7 @@ template <typename R>
 struct Row {         // one cell of a row as the y sweep sees it
   R q1, q2, q3;      // rho', rho u, rho v
   R un, ut;          // y normal velocity v = q3/rho, tangential u = q2/rho
+  uint64_t cm;       // the row's CFL lane mask (uniform)
 };
 
 template <typename R>
@@ -365,6 +382,29 @@ template <typename R>
 struct XY {          // one cell of q_xy, with its velocities for the source
   R q1, q2, q3, u, v;
 };
+
+// What a wave hands to the wave below it, per lane: the waves and speeds of its
+// first interface (y0-2), the dot products of the next (y0-1), that
+// interface's M, and its first rows of q_xy (y0-1: the cell and its
+// velocities; y0: the velocities).
+constexpr int kSeamW = 0, kSeamL = 7, kSeamDl = 10, kSeamM = 13, kSeamX = 16, kSeamFields = 23;
+template <typename R>
+__device__ __forceinline__ void seam_put(R* s, int field, R v) {
+  s[field * kLanes] = v;
+}
+template <typename R>
+__device__ __forceinline__ R seam_get(const R* s, int field) {
+  return s[field * kLanes];
+}
+// every wave's seam values are in LDS and visible to its workgroup (LDS only:
+// the prefetched row stays in flight)
+__device__ __forceinline__ void seam_publish() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+template <int kT>
+using At = std::integral_constant<int, kT>;
 
 // One work item of attempt `phase` (mod 6) of an instance whose ghost cells
 // follow the boundary policy BC (apps/<app>/boundary.h).
@@ -387,10 +427,12 @@ template <typename R, bool kOne, bool kExt, class BC>
 __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, const WorkItem& it,
                                           const uint64_t* __restrict__ rowmask, int phase,
                                           const Ctl* __restrict__ ctl_in,
-                                          const SyncSlots* __restrict__ sync_in) {
+                                          const SyncSlots* __restrict__ sync_in,
+                                          R (*seam)[kSeamFields][kLanes]) {
+#pragma clang fp contract(off)
   const InstDesc& D = insts[kOne ? 0 : it.inst];
   const int local = it.local;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & (kLanes - 1);
 
   // ---- the previous attempt's reduction, folded: accept/reject decides
   // which buffer this attempt reads, so its first row can be requested
@@ -434,7 +476,7 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
   const bool col_int = (i >= 2) && (i <= nx - 3);
   const bool out_lane = (lane >= kHalo) && (lane < kLanes - kHalo) && (i < nx);
   const int y0 = it.y0, y1 = it.y1;
-  // CFL lane masks of the item's rows: cm[j], j in [y0, y1)
+  // CFL lane masks of the strip's rows: cm[j], j in [0, ny)
   const uint64_t* __restrict__ cm = rowmask + (it.mrow - y0);
 
   // the lane's ghost-cell source columns (the app's boundary policy; Taylor
@@ -445,20 +487,22 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
   BC::lane(ic, nx, lm, kSz);
   const uint32_t row_bytes = kSz * (uint32_t)nx;
 
-  // raw (unpatched) load of row r, with the row's table entries; the
+  // raw (unpatched) load of row r, with its CFL lane mask and table entries; the
   // boundary patch is applied when the row is consumed one iteration later,
   // so the load latency overlaps a full step
-  auto load_raw = [&](int r, R& a, R& b, R& c, fvbc::RowData<R>& h) {
+  auto load_raw = [&](int r, R& a, R& b, R& c, uint64_t& k, fvbc::RowData<R>& h) {
     const int rc = min(max(r, 0), ny - 1);
     const uint32_t o = BC::offset(rc, ny, lm, row_bytes);
     a = ldg(in1, o);
     b = ldg(in2, o);
     c = ldg(in3, o);
+    k = cm[rc];
     if (BC::kRowData) BC::template load_row<R>(tb, rc, h);
   };
   R n1, n2, n3;
+  uint64_t nk;
   fvbc::RowData<R> nh{R(0), R(0), R(0), R(0), R(0), R(0)};
-  load_raw(it.y0 - kHalo, n1, n2, n3, nh);   // in flight during advance()
+  load_raw(it.y0 - kHalo, n1, n2, n3, nk, nh);   // in flight during advance()
 
   // ---- control block of this attempt ----
   Ctl P = advance<R>(D, F, local == 0);
@@ -593,64 +637,120 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
   const uint64_t in_mask = __builtin_amdgcn_ballot_w64(col_in);
   const uint64_t x_mask = __builtin_amdgcn_ballot_w64(col_x);
 
-  // One march step, r <= y1 + 2.  bn/bm/bo: q_b rows r, r-1, r-2; fn/fc/fl:
-  // y interfaces r, r-1, r-2.  xn/xo/xm hold q_xy rows r-5, r-4, r-3 on
-  // entry; the x sweep overwrites xn with row r-2.  n1..n3 (nec, nes) hold the
-  // raw prefetched row r on entry and row r+1 on exit.  Order: consume the
-  // prefetch, store row r-4, issue the next prefetch -- so each store has a
-  // whole step to drain before the next step waits for its prefetch (stores
-  // and loads share one in-order counter).
-  auto body = [&](int r, Row<R>& bn, Row<R>& bm, Row<R>& bo, YI<R>& fn, YI<R>& fc, YI<R>& fl,
-                  XY<R>& xn, XY<R>& xm, XY<R>& xo) {
-    // every load of the prefetch (and every store before it) is done: an
-    // explicit vmcnt(0) here keeps the compiler's own wait for the prefetched
-    // registers from landing after this step's stores
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
-    bn.q1 = n1; bn.q2 = n2; bn.q3 = n3;
-    patch(bn, nh, r);
-    if (r >= y0 + 4) source_store(r - 4, xn, xo, xm);
+  // What this wave leaves for the wave below it, and finds of the wave above
+  // (kSeam* fields, one value per lane).
+  R* const s_out = &seam[it.role & kRoleIndex][0][lane];
+  const R* const s_in = s_out + kSeamFields * kLanes;
+  const bool above = (it.role & kRoleAbove) != 0;   // a wave above in the workgroup
+
+  // One march step.  bn/bm/bo: q_b rows r, r-1, r-2; fn/fc/fl: y interfaces
+  // r, r-1, r-2.  xn/xo/xm hold q_xy rows r-5, r-4, r-3 on entry; the x sweep
+  // overwrites xn with row r-2.  n1..n3 (nh) hold the raw prefetched row r on
+  // entry and row r+1 on exit.  Order: consume the prefetch, store row r-4,
+  // issue the next prefetch -- so each store has a whole step to drain before
+  // the next step waits for its prefetch (stores and loads share one in-order
+  // counter).  kT: the step's place in the march.
+  //   0..5    the first rows, r = y0 - 3 + kT: each stage starts where the
+  //           item's first outputs need it, and what the wave below needs is
+  //           left in LDS
+  //   6       every later row
+  //   7..9    the last three rows below a seam (r = y1-2, y1-1, y1): the
+  //           interfaces y1-2 and up are the upper wave's
+  auto body = [&](auto kTc, int r, Row<R>& bn, Row<R>& bm, Row<R>& bo, YI<R>& fn, YI<R>& fc,
+                  YI<R>& fl, XY<R>& xn, XY<R>& xm, XY<R>& xo) {
+    constexpr int kT = decltype(kTc)::value;
+    if constexpr (kT <= 7) {
+      // every load of the prefetch (and every store before it) is done: an
+      // explicit vmcnt(0) here keeps the compiler's own wait for the prefetched
+      // registers from landing after this step's stores, and lgkmcnt(0) its
+      // wait for the row's scalars (which return in any order, so that it could
+      // only wait for all) from landing after the next row's are requested
+      __builtin_amdgcn_s_waitcnt(kWaitLoads);
+      bn.q1 = n1; bn.q2 = n2; bn.q3 = n3; bn.cm = nk;
+      patch(bn, nh, r);
+    }
+    if constexpr (kT >= 6) {
+      if (r >= y0 + 4) source_store(r - 4, xn, xo, xm);
+    }
     // the next row, also past the item's last row: the row index is clamped
     // to the grid, and an unconditional load needs no copy of the registers
     // it replaces
-    load_raw(r + 1, n1, n2, n3, nh);
-    if (r < y0 - 2) return;
+    if constexpr (kT <= 6) load_raw(r + 1, n1, n2, n3, nk, nh);
+    if constexpr (kT == 0) return;
     const int m = r - 2;
-    // CFL lane masks of rows r (y interfaces) and m (x interfaces); the index
-    // is clamped so the loads are unconditional, the row test selects 0
-    const uint64_t mYr = cm[min(max(r, y0), y1 - 1)];
-    const uint64_t mXr = cm[min(max(m, y0), y1 - 1)];
-    const uint64_t mY = (r >= y0 && r < y1 && r >= 1) ? mYr : 0;
-    const uint64_t mX = (m >= y0 && m < y1) ? mXr : 0;
 
     // ---- y interface r (rows r-1 | r): normal = q3, tangential = q2 ----
-    fvna::riemann(bm.q1, bm.q3, bm.q2, bm.un, bm.ut, bn.q1, bn.q3, bn.q2, bn.un, bn.ut,
-                  hbeta, fn.f);
-    // branch-free (a branch here would split the block and stop the
-    // cross-lane moves of the x sweep from folding into their users)
-    err |= __builtin_amdgcn_ballot_w64(fn.f.bad) & ((r >= 1 && r < ny) ? in_mask : 0);
-    Sy = fvna::fmax2(Sy, lane_sel(mY, fn.f.smax));
+    if constexpr (kT <= 6) {
+      // CFL lane mask of row r (its y interfaces).  Rows next to a workgroup's
+      // own are counted there too: the same values, so the same maximum
+      const uint64_t mY = (r >= 1 && r < ny) ? bn.cm : 0;
+      fvna::riemann(fvna::jump(bm.q1, bm.q3, bm.q2, bm.un, bm.ut, bn.q1, bn.q3, bn.q2, bn.un,
+                               bn.ut),
+                    hbeta, fn.f);
+      // branch-free (a branch here would split the block and stop the
+      // cross-lane moves of the x sweep from folding into their users)
+      err |= __builtin_amdgcn_ballot_w64(fn.f.bad) & ((r >= 1 && r < ny) ? in_mask : 0);
+      Sy = fvna::fmax2(Sy, lane_sel(mY, fn.f.smax));
+      if constexpr (kT == 1) {
+        seam_put(s_out, kSeamW + 0, fn.f.w.a1);  seam_put(s_out, kSeamW + 1, fn.f.w.w21);
+        seam_put(s_out, kSeamW + 2, fn.f.w.w31); seam_put(s_out, kSeamW + 3, fn.f.w.a2);
+        seam_put(s_out, kSeamW + 4, fn.f.w.w22); seam_put(s_out, kSeamW + 5, fn.f.w.w32);
+        seam_put(s_out, kSeamW + 6, fn.f.w.a3);
+        seam_put(s_out, kSeamL + 0, fn.f.L1);
+        seam_put(s_out, kSeamL + 1, fn.f.L2);
+        seam_put(s_out, kSeamL + 2, fn.f.L3);
+        return;
+      }
+    } else if constexpr (kT == 7) {
+      fn.f.w.a1 = seam_get(s_in, kSeamW + 0);  fn.f.w.w21 = seam_get(s_in, kSeamW + 1);
+      fn.f.w.w31 = seam_get(s_in, kSeamW + 2); fn.f.w.a2 = seam_get(s_in, kSeamW + 3);
+      fn.f.w.w22 = seam_get(s_in, kSeamW + 4); fn.f.w.w32 = seam_get(s_in, kSeamW + 5);
+      fn.f.w.a3 = seam_get(s_in, kSeamW + 6);
+      fn.f.L1 = seam_get(s_in, kSeamL + 0);
+      fn.f.L2 = seam_get(s_in, kSeamL + 1);
+      fn.f.L3 = seam_get(s_in, kSeamL + 2);
+    }
 
     // W(r).W(r-1): the left product of interface r, the right one of r-1
-    fn.dl[0] = fvna::dot1(fn.f.w, fc.f.w);
-    fn.dl[1] = fvna::dot2(fn.f.w, fc.f.w);
-    fn.dl[2] = fn.f.w.a3 * fc.f.w.a3;
-    if (r < y0) return;
+    if constexpr (kT <= 7) {
+      fn.dl[0] = fvna::dot1(fn.f.w, fc.f.w);
+      fn.dl[1] = fvna::dot2(fn.f.w, fc.f.w);
+      fn.dl[2] = fn.f.w.a3 * fc.f.w.a3;
+    } else if constexpr (kT == 8) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) fn.dl[p] = seam_get(s_in, kSeamDl + p);
+    }
+    if constexpr (kT == 2) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) seam_put(s_out, kSeamDl + p, fn.dl[p]);
+      return;
+    }
 
     // ---- y limiter at interface r-1 ----
     R M[3];
-    fvna::limited_flux(fc.f, fc.dl[0], fn.dl[0], fc.dl[1], fn.dl[1], fc.dl[2], fn.dl[2], dty,
-                       fc.P, M);
-    if (r < y0 + 1) return;
+    if constexpr (kT <= 8) {
+      fvna::limited_flux<false>(fc.f, fc.dl[0], fn.dl[0], fc.dl[1], fn.dl[1], fc.dl[2], fn.dl[2],
+                                dty, fc.P, M);
+    } else {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) M[p] = seam_get(s_in, kSeamM + p);
+    }
+    if constexpr (kT == 3) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) seam_put(s_out, kSeamM + p, M[p]);
+      return;
+    }
 
     // ---- q_y on row m = r-2 (components: density, normal=q3, tangential=q2)
+    const uint64_t mX = (m >= 0 && m < ny) ? bo.cm : 0;
     const bool row_int = (m >= 2) && (m <= ny - 3);
     // ghost cells keep their value: dt/d is 0 there (the fluxes are finite
     // wherever the attempt is valid, so q - 0*flux == q exactly); the column
     // test is folded in once per item (dty_c, dtx_c), the row test here
     const R dtyu = row_int ? dty_c : R(0), dtxu = row_int ? dtx_c : R(0);
-    const R y1q = bo.q1 - dtyu * (fl.P[0] + M[0]);
-    const R y3q = bo.q3 - dtyu * (fl.P[1] + M[1]);
-    const R y2q = bo.q2 - dtyu * (fl.P[2] + M[2]);
+    const R y1q = fvna::sub_prod(bo.q1, dtyu, fl.P[0] + M[0]);
+    const R y3q = fvna::sub_prod(bo.q3, dtyu, fl.P[1] + M[1]);
+    const R y2q = fvna::sub_prod(bo.q2, dtyu, fl.P[2] + M[2]);
 
     // ---- x sweep on row m: normal = q2, tangential = q3 ----
     const R ir = fvna::rcp(R(1) + y1q);
@@ -658,7 +758,11 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
     const R l1 = shr1(y1q), l2 = shr1(y2q), l3 = shr1(y3q);
     const R lun = shr1(un), lut = shr1(ut);
     fvna::IfaceT<R> fx;
-    fvna::riemann(l1, l2, l3, lun, lut, y1q, y2q, y3q, un, ut, hbeta, fx);
+    // pinned together: the compiler folds a cross-lane move only into users
+    // within a few instructions of it
+    fvna::JumpT<R> jx = fvna::jump(l1, l2, l3, lun, lut, y1q, y2q, y3q, un, ut);
+    pin(jx.s1); pin(jx.s2); pin(jx.s3); pin(jx.drho); pin(jx.dn); pin(jx.dtg);
+    fvna::riemann(jx, hbeta, fx);
     err |= __builtin_amdgcn_ballot_w64(fx.bad) & ((m >= 0 && m < ny) ? x_mask : 0);
     Sx = fvna::fmax2(Sx, lane_sel(mX, fx.smax));
     // waves of the interface to the left (k-1)
@@ -671,36 +775,71 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
     // W(k).W(k+1) is the right neighbour's W(k+1).W(k)
     const R dr1 = shl1(dl1), dr2 = shl1(dl2), dr3 = shl1(dl3);
     R PX[3], MX[3];
-    fvna::limited_flux(fx, dl1, dr1, dl2, dr2, dl3, dr3, dtx, PX, MX);
+    fvna::limited_flux<true>(fx, dl1, dr1, dl2, dr2, dl3, dr3, dtx, PX, MX);
     const R mr0 = shl1(MX[0]), mr1 = shl1(MX[1]), mr2 = shl1(MX[2]);
-    xn.q1 = y1q - dtxu * (mr0 + PX[0]);
-    xn.q2 = y2q - dtxu * (mr1 + PX[1]);
-    xn.q3 = y3q - dtxu * (mr2 + PX[2]);
+    xn.q1 = fvna::sub_prod(y1q, dtxu, mr0 + PX[0]);
+    xn.q2 = fvna::sub_prod(y2q, dtxu, mr1 + PX[1]);
+    xn.q3 = fvna::sub_prod(y3q, dtxu, mr2 + PX[2]);
     const R ir2 = fvna::rcp(R(1) + xn.q1);
     xn.u = xn.q2 * ir2;
     xn.v = xn.q3 * ir2;
+    if constexpr (kT == 4) {
+      seam_put(s_out, kSeamX + 0, xn.q1);
+      seam_put(s_out, kSeamX + 1, xn.q2);
+      seam_put(s_out, kSeamX + 2, xn.q3);
+      seam_put(s_out, kSeamX + 3, xn.u);
+      seam_put(s_out, kSeamX + 4, xn.v);
+    }
+    if constexpr (kT == 5) {
+      seam_put(s_out, kSeamX + 5, xn.u);
+      seam_put(s_out, kSeamX + 6, xn.v);
+    }
   };
 
-  // every window is written before it is read, except the waves of the
-  // interface before the first one (their products with the first
-  // interface's waves are formed but never used): only those are zeroed, so
-  // no unset value is read and the other windows cost no initialisation
+  // every window is written before it is read
   Row<R> B0, B1, B2;
   YI<R> F0, F1, F2;
   XY<R> X0, X1, X2;
-  F0.f.w = fvna::WavesT<R>{};
-  for (int r = y0 - kHalo; r <= y1 + 2; r += 3) {
-    body(r, B0, B2, B1, F0, F2, F1, X0, X2, X1);
-    if (r + 1 > y1 + 2) break;
-    body(r + 1, B1, B0, B2, F1, F0, F2, X1, X0, X2);
-    if (r + 2 > y1 + 2) break;
-    body(r + 2, B2, B1, B0, F2, F1, F0, X2, X1, X0);
+  body(At<0>{}, y0 - 3, B0, B2, B1, F0, F2, F1, X0, X2, X1);
+  body(At<1>{}, y0 - 2, B1, B0, B2, F1, F0, F2, X1, X0, X2);
+  body(At<2>{}, y0 - 1, B2, B1, B0, F2, F1, F0, X2, X1, X0);
+  body(At<3>{}, y0, B0, B2, B1, F0, F2, F1, X0, X2, X1);
+  body(At<4>{}, y0 + 1, B1, B0, B2, F1, F0, F2, X1, X0, X2);
+  body(At<5>{}, y0 + 2, B2, B1, B0, F2, F1, F0, X2, X1, X0);
+  seam_publish();
+  const int r_end = above ? y1 - 3 : y1 + 2;
+  for (int r = y0 + 3; r <= r_end; r += 3) {
+    body(At<6>{}, r, B0, B2, B1, F0, F2, F1, X0, X2, X1);
+    if (r + 1 > r_end) break;
+    body(At<6>{}, r + 1, B1, B0, B2, F1, F0, F2, X1, X0, X2);
+    if (r + 2 > r_end) break;
+    body(At<6>{}, r + 2, B2, B1, B0, F2, F1, F0, X2, X1, X0);
   }
-  // the last row, y1 - 1, with the window of the step r = y1 + 3 would see
-  switch ((y1 - y0) % 3) {
-    case 0: source_store(y1 - 1, X0, X1, X2); break;
-    case 1: source_store(y1 - 1, X1, X2, X0); break;
-    default: source_store(y1 - 1, X2, X0, X1); break;
+  if (above) {
+    // the host gives the items below a seam heights of 2 mod 3 (>= 5), so the
+    // loop ends with the windows in their first rotation
+    body(At<7>{}, y1 - 2, B0, B2, B1, F0, F2, F1, X0, X2, X1);
+    body(At<8>{}, y1 - 1, B1, B0, B2, F1, F0, F2, X1, X0, X2);
+    body(At<9>{}, y1, B2, B1, B0, F2, F1, F0, X2, X1, X0);
+    XY<R> a0, a1;             // the upper wave's first two rows of q_xy, y1-1 and y1
+    a0.q1 = seam_get(s_in, kSeamX + 0);
+    a0.q2 = seam_get(s_in, kSeamX + 1);
+    a0.q3 = seam_get(s_in, kSeamX + 2);
+    a0.u = seam_get(s_in, kSeamX + 3);
+    a0.v = seam_get(s_in, kSeamX + 4);
+    a1 = a0;
+    a1.u = seam_get(s_in, kSeamX + 5);
+    a1.v = seam_get(s_in, kSeamX + 6);
+    source_store(y1 - 3, X0, X1, X2);
+    source_store(y1 - 2, X1, X2, a0);
+    source_store(y1 - 1, X2, a0, a1);
+  } else {
+    // the last row, y1 - 1, with the window of the step r = y1 + 3 would see
+    switch ((y1 - y0) % 3) {
+      case 0: source_store(y1 - 1, X0, X1, X2); break;
+      case 1: source_store(y1 - 1, X1, X2, X0); break;
+      default: source_store(y1 - 1, X2, X0, X1); break;
+    }
   }
 
   // ---- CFL / error reduction ----
@@ -720,33 +859,34 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
 // directly, a kernel with one march.
 struct AnyApp {};
 
-// The step kernel: one wave per work item.
+// The step kernel: one wave per work item, kGroupWaves items per workgroup
+// (items[4 g .. 4 g + 3]; an unused slot has no rows).
 template <typename R, bool kOne, bool kExt, class BC>
-__global__ __launch_bounds__(64) void fv_step_kernel(const InstDesc* __restrict__ insts,
-                                                     const WorkItem* __restrict__ items,
-                                                     const uint64_t* __restrict__ rowmask,
-                                                     int n_items, int phase,
-                                                     const Ctl* __restrict__ ctl_in,
-                                                     const SyncSlots* __restrict__ sync_in) {
+__global__ __launch_bounds__(kLanes * kGroupWaves) void fv_step_kernel(
+    const InstDesc* __restrict__ insts, const WorkItem* __restrict__ items,
+    const uint64_t* __restrict__ rowmask, int n_groups, int phase,
+    const Ctl* __restrict__ ctl_in, const SyncSlots* __restrict__ sync_in) {
+  __shared__ R seam[kGroupWaves][kSeamFields][kLanes];
   // XCD-aware order: workgroup b runs on XCD b % 8; give each XCD a contiguous
-  // run of work items so vertically adjacent chunks of a strip (which share
+  // run of groups so vertically adjacent groups of a strip (which share
   // halo rows) hit the same L2.
-  int item;
+  int group;
   {
     const int b = blockIdx.x;
-    const int q = n_items >> 3, rem = n_items & 7, x = b & 7, k = b >> 3;
-    item = x * q + min(x, rem) + k;
+    const int q = n_groups >> 3, rem = n_groups & 7, x = b & 7, k = b >> 3;
+    group = x * q + min(x, rem) + k;
   }
-  const WorkItem it = items[item];
+  const WorkItem it = items[group * kGroupWaves + uni(threadIdx.x / kLanes)];
+  if (it.y1 <= it.y0) return;      // the barrier counts the remaining waves only
   if constexpr (!std::is_same<BC, AnyApp>::value) {
-    step_impl<R, kOne, kExt, BC>(insts, it, rowmask, phase, ctl_in, sync_in);
+    step_impl<R, kOne, kExt, BC>(insts, it, rowmask, phase, ctl_in, sync_in, seam);
     return;
   }
   switch (uni(it.bc)) {
-#define FV_APP_CASE(P)                                                        \
-  case P::kId:                                                                \
-    if constexpr (kExt || !P::kExtOnly)                                       \
-      step_impl<R, kOne, kExt, P>(insts, it, rowmask, phase, ctl_in, sync_in); \
+#define FV_APP_CASE(P)                                                              \
+  case P::kId:                                                                      \
+    if constexpr (kExt || !P::kExtOnly)                                             \
+      step_impl<R, kOne, kExt, P>(insts, it, rowmask, phase, ctl_in, sync_in, seam); \
     break;
     FIVONAGI_APPS(FV_APP_CASE)
 #undef FV_APP_CASE
@@ -885,38 +1025,40 @@ extern "C" hipError_t fv_launch_settle(const fv::InstDesc* insts, int n_inst, in
 // kernels of several instances (every app's march: the most registers), so
 // the split fits whichever kernel a context launches.
 extern "C" hipError_t fv_step_waves_per_cu(int* waves, int fp64) {
+  constexpr int kThreads = fv::kLanes * fv::kGroupWaves;
   int a = 0, b = 0;
   hipError_t e = fp64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                            &a, fv::fv_step_kernel<double, false, false, fv::AnyApp>, fv::kLanes, 0)
+                            &a, fv::fv_step_kernel<double, false, false, fv::AnyApp>, kThreads, 0)
                       : hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                            &a, fv::fv_step_kernel<float, false, false, fv::AnyApp>, fv::kLanes, 0);
+                            &a, fv::fv_step_kernel<float, false, false, fv::AnyApp>, kThreads, 0);
   if (e != hipSuccess) return e;
   e = fp64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                 &b, fv::fv_step_kernel<double, false, true, fv::AnyApp>, fv::kLanes, 0)
+                 &b, fv::fv_step_kernel<double, false, true, fv::AnyApp>, kThreads, 0)
            : hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                 &b, fv::fv_step_kernel<float, false, true, fv::AnyApp>, fv::kLanes, 0);
-  *waves = a < b ? a : b;
+                 &b, fv::fv_step_kernel<float, false, true, fv::AnyApp>, kThreads, 0);
+  *waves = fv::kGroupWaves * (a < b ? a : b);
   return e;
 }
 
 namespace {
 template <typename R, bool kOne, bool kExt, class BC>
 void launch_step_t(const fv::InstDesc* insts, const fv::WorkItem* items, const uint64_t* rowmask,
-                   int n_items, int phase, const fv::Ctl* c_in, const fv::SyncSlots* s_in,
+                   int n_groups, int phase, const fv::Ctl* c_in, const fv::SyncSlots* s_in,
                    hipStream_t stream) {
-  hipLaunchKernelGGL((fv::fv_step_kernel<R, kOne, kExt, BC>), dim3(n_items), dim3(fv::kLanes), 0,
-                     stream, insts, items, rowmask, n_items, phase, c_in, s_in);
+  hipLaunchKernelGGL((fv::fv_step_kernel<R, kOne, kExt, BC>), dim3(n_groups),
+                     dim3(fv::kLanes * fv::kGroupWaves), 0, stream, insts, items, rowmask,
+                     n_groups, phase, c_in, s_in);
 }
 // a single instance: its app's own kernel (bc), else the dispatching one
 template <typename R, bool kExt>
 void launch_one(int bc, const fv::InstDesc* insts, const fv::WorkItem* items,
-                const uint64_t* rowmask, int n_items, int phase, const fv::Ctl* c_in,
+                const uint64_t* rowmask, int n_groups, int phase, const fv::Ctl* c_in,
                 const fv::SyncSlots* s_in, hipStream_t stream) {
   switch (bc) {
 #define FV_APP_LAUNCH(P)                                                                 \
   case P::kId:                                                                           \
     if constexpr (kExt || !P::kExtOnly) {                                                \
-      launch_step_t<R, true, kExt, P>(insts, items, rowmask, n_items, phase, c_in, s_in, \
+      launch_step_t<R, true, kExt, P>(insts, items, rowmask, n_groups, phase, c_in, s_in, \
                                       stream);                                           \
       return;                                                                            \
     }                                                                                    \
@@ -926,43 +1068,43 @@ void launch_one(int bc, const fv::InstDesc* insts, const fv::WorkItem* items,
     default:
       break;
   }
-  launch_step_t<R, true, kExt, fv::AnyApp>(insts, items, rowmask, n_items, phase, c_in, s_in,
+  launch_step_t<R, true, kExt, fv::AnyApp>(insts, items, rowmask, n_groups, phase, c_in, s_in,
                                            stream);
 }
 template <typename R>
 void launch_step_r(bool one, bool ext, int bc, const fv::InstDesc* insts,
-                   const fv::WorkItem* items, const uint64_t* rowmask, int n_items, int phase,
+                   const fv::WorkItem* items, const uint64_t* rowmask, int n_groups, int phase,
                    const fv::Ctl* c_in, const fv::SyncSlots* s_in, hipStream_t stream) {
   if (one && !ext)
-    launch_one<R, false>(bc, insts, items, rowmask, n_items, phase, c_in, s_in, stream);
+    launch_one<R, false>(bc, insts, items, rowmask, n_groups, phase, c_in, s_in, stream);
   else if (one)
-    launch_one<R, true>(bc, insts, items, rowmask, n_items, phase, c_in, s_in, stream);
+    launch_one<R, true>(bc, insts, items, rowmask, n_groups, phase, c_in, s_in, stream);
   else if (!ext)
-    launch_step_t<R, false, false, fv::AnyApp>(insts, items, rowmask, n_items, phase, c_in, s_in,
+    launch_step_t<R, false, false, fv::AnyApp>(insts, items, rowmask, n_groups, phase, c_in, s_in,
                                                stream);
   else
-    launch_step_t<R, false, true, fv::AnyApp>(insts, items, rowmask, n_items, phase, c_in, s_in,
+    launch_step_t<R, false, true, fv::AnyApp>(insts, items, rowmask, n_groups, phase, c_in, s_in,
                                               stream);
 }
 }  // namespace
 
-// One step attempt of every instance.  ctl0/sync0: the control blocks and
+// One step attempt of every instance: n_groups workgroups, items[4 g ..] each.  ctl0/sync0: the control blocks and
 // slot sets of the only instance when n_inst == 1 (null otherwise), bc0 its
 // boundary kind; ext: some instance has a moving window, the HIFU boundary or
 // data collection; fp64: the instances are FP64.
 extern "C" hipError_t fv_launch_step(const fv::InstDesc* insts, const fv::WorkItem* items,
-                                     const uint64_t* rowmask, int n_items, int phase,
+                                     const uint64_t* rowmask, int n_groups, int phase,
                                      int n_inst, fv::Ctl* ctl0, fv::SyncSlots* sync0, int bc0,
                                      int ext, int fp64, hipStream_t stream) {
-  if (n_items <= 0) return hipSuccess;
+  if (n_groups <= 0) return hipSuccess;
   const bool one = n_inst == 1 && ctl0 && sync0;
   const fv::Ctl* c_in = one ? ctl0 + (phase & 1) : nullptr;
   const fv::SyncSlots* s_in = one ? sync0 + (phase + 2) % 3 : nullptr;
   if (fp64)
-    launch_step_r<double>(one, ext != 0, bc0, insts, items, rowmask, n_items, phase, c_in, s_in,
+    launch_step_r<double>(one, ext != 0, bc0, insts, items, rowmask, n_groups, phase, c_in, s_in,
                           stream);
   else
-    launch_step_r<float>(one, ext != 0, bc0, insts, items, rowmask, n_items, phase, c_in, s_in,
+    launch_step_r<float>(one, ext != 0, bc0, insts, items, rowmask, n_groups, phase, c_in, s_in,
                          stream);
   return hipGetLastError();
 }

@@ -152,20 +152,76 @@ bool cfl_counted(int cfl_mask, const std::vector<uint32_t>& fold_bits, int nx, i
   return true;
 }
 
-// Rows per work item: the smallest height (never below 12) whose total wave
-// count over all instances fits one resident round of the device
+static long strips_of(const fivonagi_params& p) {
+  return (p.nx + fv::kStripCols - 1) / fv::kStripCols;
+}
+
+// Lane mask of row j of the strip at x0: bit kHalo + n set when the CFL
+// reduction counts the output cell (x0 + n, j), columns 0 and past the grid
+// left out.
+static uint64_t lane_mask(int cfl_mask, const std::vector<uint32_t>& fold_bits, int nx, int x0,
+                          int j) {
+  const int n = std::min(fv::kStripCols, nx - x0);
+  uint64_t m = ~(uint64_t)0;
+  const size_t o = (size_t)x0 + (size_t)j * (size_t)nx;
+  if (cfl_mask == fv::kCflEven) {
+    m = (o & 1) ? 0xAAAAAAAAAAAAAAAAull : 0x5555555555555555ull;
+  } else if (cfl_mask == fv::kCflBitmap) {
+    // 64 bits from bit o of the bitmap (words past its end: no cells)
+    const size_t w = o >> 5, e = fold_bits.size();
+    const unsigned sh = o & 31;
+    const uint64_t lo = fold_bits[w] | (uint64_t)(w + 1 < e ? fold_bits[w + 1] : 0) << 32;
+    const uint64_t hi = w + 2 < e ? fold_bits[w + 2] : 0;
+    m = sh ? lo >> sh | hi << (64 - sh) : lo;
+  }
+  m &= ((uint64_t)1 << n) - 1;             // n <= 58
+  if (x0 == 0) m &= ~(uint64_t)1;
+  return m << fv::kHalo;
+}
+
+// Rows per item of the in-step cut: the smallest height (never below 12) whose
+// total wave count over all instances fits one resident round of the device
 // (CUs x resident step waves per CU): every wave then starts at once, and
 // taller work items repeat fewer halo rows.
 int auto_rows(const std::vector<fivonagi_params>& ps, long target_waves) {
   for (int H = 12; H <= 4096; ++H) {
     long waves = 0;
-    for (const auto& p : ps) {
-      const long strips = (p.nx + fv::kStripCols - 1) / fv::kStripCols;
-      waves += strips * std::max(1L, std::lround((double)p.ny / H));
-    }
+    for (const auto& p : ps)
+      waves += strips_of(p) * std::max(1L, std::lround((double)p.ny / H));
     if (waves <= target_waves) return H;
   }
   return 4096;
+}
+
+// Items of a strip of p in the in-step cut.
+static int in_step_items(const fivonagi_params& p, int auto_h) {
+  const int H = p.rows_per_wave > 0 ? p.rows_per_wave : auto_h;
+  return std::max(1, std::min(p.ny, (int)std::lround((double)p.ny / H)));
+}
+
+// March steps of the slowest of n waves that share R rows of a strip, one
+// above the other: a wave below another marches one step per row of its own,
+// at least kSeamRows (its first rows are what it hands down) and 2 mod 3 (the
+// march's unrolled rotation, fv_step.hip); the topmost marches past its end,
+// about kTail rows' worth.
+constexpr double kTail = 3.3;
+constexpr int kSeamRows = 5;
+
+std::vector<int> group_heights(int R, int max_waves) {
+  const int n = std::max(1, std::min(max_waves, (R - 1) / kSeamRows + 1));
+  std::vector<int> h(n);
+  int left = R;
+  for (int w = 0; w + 1 < n; ++w) {
+    const int rest = n - 1 - w;                        // waves above this one
+    const double even = (left + kTail) / (rest + 1);
+    const int most = left - (rest - 1) * kSeamRows - 1;
+    int H = kSeamRows + 3 * std::max(0, (int)std::floor((even - kSeamRows) / 3.0 + 0.5));
+    while (H > most) H -= 3;
+    h[w] = std::max(kSeamRows, H);
+    left -= h[w];
+  }
+  h[n - 1] = left;
+  return h;
 }
 
 // Row boundaries of one strip cut into `chunks` work items.  With skew > 0
@@ -192,92 +248,277 @@ std::vector<int> chunk_bounds(int ny, int chunks, float skew, int levels, int ro
   return b;
 }
 
-// Launch order of the work items.  Workgroup b of a launch runs on XCD b % 8
-// and takes item x*q + min(x, rem) + (b >> 3) (fv_step_kernel), so XCD x
-// works through the run of items [x*q + min(x, rem), ...) in order, and within
-// a run the hardware starts items in that order, one per SIMD, then the next
-// round of SIMD slots.  Each run is sorted by height, tallest first: the
-// waves that start first (and, as the oldest on their SIMD, issue first) get
-// the most rows, so the SIMDs' waves finish together instead of leaving one
-// wave alone at the end; on launches of several rounds the short items come
-// last.  Stable, so equal heights keep the strip order (neighbouring items,
-// which share halo rows, stay on the same XCD).
-void order_for_launch(std::vector<fv::WorkItem>& items) {
-  const int n = (int)items.size();
-  const int q = n >> 3, rem = n & 7;
-  for (int x = 0; x < 8; ++x) {
-    const int b = x * q + std::min(x, rem), e = b + q + (x < rem ? 1 : 0);
-    std::stable_sort(items.begin() + b, items.begin() + e,
-                     [](const fv::WorkItem& u, const fv::WorkItem& v) {
-                       return (u.y1 - u.y0) > (v.y1 - v.y0);
-                     });
+// Height skew where every SIMD starts its full complement of waves: evens out
+// the ends of four waves of which the oldest issues first (their speeds,
+// measured on equal items: 1.09, 0.75, 0.46, 0.32 rows per us).  Step in us at
+// skew 0 / 0.5 / 0.65: 4096x1024 38.7 / 36.9 / 37.0, 4096x2048 69.7 / 65.3 /
+// 63.1, 8192x4096 263 / 237 / 231, 6000x5001 232 / 234 / 244.
+constexpr float kAutoSkew = 0.5f;
+
+// Largest state, in and out, that is cut "running on" (cut A below).  Up to the
+// 256 MiB of the memory-side cache the step is bound by its instructions, and
+// cut A repeats fewer of them and balances better: 4096x1024 (101 MB) 37.0 us
+// against 40.5 for cut B, 4096x2048 (201 MB) 63 against 73.  Beyond it the
+// lines at the strips' edges, which two strips read and write, must meet in
+// the L2 while both march them, which needs cut B: 4096x4096 (403 MB) 147
+// against 134, 8192x4096 (805 MB) 340 against 231.
+constexpr long kRunningBytes = 256L << 20;
+
+namespace {
+
+// A row range of one strip.
+struct Piece {
+  int inst, x0, y0, rows, mrow;
+  int waves;                               // that share it
+};
+// The pieces one workgroup marches.
+struct Group {
+  int n = 0;
+  Piece p[fv::kGroupWaves];
+  long rows() const {
+    long r = 0;
+    for (int j = 0; j < n; ++j) r += p[j].rows;
+    return r;
+  }
+};
+
+// weight of height level l of L: falling linearly from 1 + skew to 1 - skew
+double level_weight(int l, int L, float skew) {
+  return L > 1 ? std::max(1.0 + (double)skew * (L - 1 - 2 * l) / (L - 1), 0.05) : 1.0;
+}
+
+// Cut A, "running on": the strips, laid end to end, are dealt to groups whose
+// waves march at most c * (the group's level weight) steps; a group that
+// reaches the end of a strip with waves to spare goes on with the next one.
+// emit: called with each group (count only: a no-op).  Returns their number.
+template <class Emit>
+long cut_running(const std::vector<Piece>& strips, double c, float skew, int levels, Emit emit) {
+  long n = 0;
+  Group cur;
+  int left = 0;                            // waves of the current group to spare
+  double cl = 0.0;
+  auto start = [&]() {
+    cl = std::max<double>(kSeamRows, c * level_weight((int)(n % levels), levels, skew));
+    left = fv::kGroupWaves;
+    cur.n = 0;
+  };
+  auto flush = [&]() {
+    if (cur.n > 0) {
+      emit(cur);
+      ++n;
+    }
+    start();
+  };
+  start();
+  for (const auto& s : strips)
+    for (int y = 0; y < s.rows;) {
+      const int rest = s.rows - y;
+      const int need = std::max(1, (int)std::ceil((rest + kTail) / cl - 1e-9));
+      Piece p{s.inst, s.x0, s.y0 + y, rest, s.mrow + y, need};
+      if (need > left) {
+        p.waves = left;
+        p.rows = std::min(rest - 1, std::max(1, (int)std::floor(left * cl - kTail + 1e-9)));
+      }
+      cur.p[cur.n++] = p;
+      left -= p.waves;
+      y += p.rows;
+      if (left == 0) flush();
+    }
+  flush();
+  return n;
+}
+
+// Groups sorted tallest first, dealt C at a time to the C CUs of an XCD: the
+// first and the last round stay in order (the last may leave the last CUs
+// without a group), and in the rounds between the tallest group goes to the CU
+// with the fewest rows.
+void balance_rounds(std::vector<Group>& run, int C) {
+  const int n = (int)run.size(), rounds = (n + C - 1) / C;
+  if (rounds < 3) return;
+  std::vector<long> load(C, 0);
+  for (int j = 0; j < C; ++j) load[j] = run[j].rows();
+  for (int g = (rounds - 1) * C; g < n; ++g) load[g % C] += run[g].rows();
+  for (int r = 1; r + 1 < rounds; ++r) {
+    std::vector<int> place(C);
+    for (int j = 0; j < C; ++j) place[j] = j;
+    std::stable_sort(place.begin(), place.end(), [&](int u, int v) { return load[u] < load[v]; });
+    const std::vector<Group> round(run.begin() + r * C, run.begin() + (r + 1) * C);
+    for (int j = 0; j < C; ++j) {
+      run[r * C + place[j]] = round[j];
+      load[place[j]] += round[j].rows();
+    }
   }
 }
 
-constexpr float kAutoSkew = 0.5f;
-
-int item_chunks(const fivonagi_params& p, int auto_h) {
-  const int H = p.rows_per_wave > 0 ? p.rows_per_wave : auto_h;
-  return std::max(1, (int)std::lround((double)p.ny / H));
-}
+}  // namespace
 
 void build_work(const std::vector<fivonagi_params>& ps, const std::vector<int>& cfl_mask,
                 const std::vector<std::vector<uint32_t>>& fold_bits, long cus, int per_cu,
-                int auto_h, float skew, bool rotate, WorkList& out) {
+                int auto_h, float skew, bool rotate, WorkList& out, int cell_bytes) {
   out.items.clear();
   out.rowmask.clear();
+  out.group_first.assign(1, 0);
   out.n_items.assign(ps.size(), 0);
+  // the strips, with their lane masks
+  std::vector<Piece> strips;
+  long bytes = 0, waves = 0;               // waves: of the in-step cut
+  double rows = 0.0, asked = 0.0;
+  for (int k = 0; k < (int)ps.size(); ++k) {
+    const auto& p = ps[k];
+    waves += strips_of(p) * in_step_items(p, auto_h);
+    rows += (double)strips_of(p) * p.ny;
+    if (p.rows_per_wave > 0) asked += (double)strips_of(p) * p.ny / p.rows_per_wave;
+    bytes += (long)cell_bytes * p.nx * p.ny;
+    for (int s = 0; s < (int)strips_of(p); ++s) {
+      const int x0 = s * fv::kStripCols;
+      strips.push_back({k, x0, 0, p.ny, (int)out.rowmask.size(), 1});
+      for (int j = 0; j < p.ny; ++j)
+        out.rowmask.push_back(lane_mask(cfl_mask[k], fold_bits[k], p.nx, x0, j));
+    }
+  }
+  // height levels = waves each SIMD starts in the launch's first round
   const long simds = 4 * cus;
   const int per_simd = std::max(1, per_cu / 4);
-  // height levels = waves each SIMD starts in the launch's first round
-  long total = 0;
-  for (const auto& p : ps)
-    total += (long)((p.nx + fv::kStripCols - 1) / fv::kStripCols) * item_chunks(p, auto_h);
-  const int levels = (int)std::max(1L, std::min<long>(per_simd, (total + simds - 1) / simds));
+  const int levels = (int)std::max(1L, std::min<long>(per_simd, (waves + simds - 1) / simds));
   // automatic: skewed only when every SIMD starts its full complement of
   // waves (there the oldest-first issue order staggers their ends; with
   // fewer waves per SIMD they progress together)
-  if (skew < 0.0f) skew = (levels >= 4 && levels == per_simd) ? kAutoSkew : 0.0f;
+  bool running = rotate;
+  if (skew < 0.0f) {
+    skew = (levels >= 4 && levels == per_simd) ? kAutoSkew : 0.0f;
+    running = bytes <= kRunningBytes;
+  }
   out.skew_used = skew;
   out.rotate_used = rotate && skew > 0.0f;
-  for (int k = 0; k < (int)ps.size(); ++k) {
-    const auto& p = ps[k];
-    const int chunks = item_chunks(p, auto_h);
-    const int strips = (p.nx + fv::kStripCols - 1) / fv::kStripCols;
-    // rotate: the level pattern shifts by one per strip (every level gets the
-    // same number of items; strips no longer share their cut rows)
-    std::vector<std::vector<int>> bounds_rot;
-    for (int r = 0; r < (rotate ? levels : 1); ++r)
-      bounds_rot.push_back(chunk_bounds(p.ny, chunks, skew, levels, r));
-    int n = 0;
-    for (int s = 0; s < strips; ++s) {
-      const std::vector<int>& bounds = bounds_rot[rotate ? s % levels : 0];
-      for (int ch = 0; ch < chunks; ++ch) {
-        fv::WorkItem w;
-        w.inst = k;
-        w.x0 = s * fv::kStripCols;
-        w.y0 = bounds[ch];
-        w.y1 = bounds[ch + 1];
-        w.mrow = (int)out.rowmask.size();
-        w.local = n;
-        w.bc = p.bc;
-        w.pad = 0;
-        for (int j = w.y0; j < w.y1; ++j) {
-          uint64_t m = 0;
-          for (int l = fv::kHalo; l < fv::kLanes - fv::kHalo; ++l) {
-            const int i = w.x0 - fv::kHalo + l;
-            if (i >= 1 && i < p.nx && cfl_counted(cfl_mask[k], fold_bits[k], p.nx, i, j))
-              m |= (uint64_t)1 << l;
-          }
-          out.rowmask.push_back(m);
-        }
-        out.items.push_back(w);
-        ++n;
+  std::vector<Group> groups;
+  if (running) {
+    // the least steps per wave whose groups are all resident at once (to 0.4%)
+    const long target = std::max(1L, cus * per_simd);
+    auto fits = [&](double c) {
+      return cut_running(strips, c, skew, levels, [](const Group&) {}) <= target;
+    };
+    double c = kSeamRows;
+    if (asked > 0.0) {
+      c = std::max<double>(kSeamRows, rows / asked);
+    } else if (!fits(c)) {
+      double lo = std::max(c, rows / (double)(target * fv::kGroupWaves)), hi = 1.05 * lo;
+      while (!fits(hi)) { lo = hi; hi *= 1.25; }
+      while (hi - lo > 0.004 * lo) {
+        const double mid = 0.5 * (lo + hi);
+        if (fits(mid)) hi = mid;
+        else lo = mid;
+      }
+      c = hi;
+    }
+    cut_running(strips, c, skew, levels, [&](const Group& g) { groups.push_back(g); });
+  } else {
+    // Cut B, "in step": each strip into the same number of one-wave items, cut
+    // at the same rows in every strip of an instance
+    std::vector<Piece> items;
+    for (const auto& s : strips) {
+      const int chunks = in_step_items(ps[s.inst], auto_h);
+      const std::vector<int> b = chunk_bounds(s.rows, chunks, skew, levels, 0);
+      for (int j = 0; j < chunks; ++j)
+        items.push_back({s.inst, s.x0, b[j], b[j + 1] - b[j], s.mrow + b[j], 1});
+    }
+    // each XCD's run tallest first (see below), four to a workgroup; equal
+    // heights by rows, so that a workgroup's waves are neighbouring strips
+    const int n = (int)items.size(), W = fv::kGroupWaves;
+    const int wgs = (n + W - 1) / W, q = wgs >> 3, rem = wgs & 7;
+    for (int x = 0; x < 8; ++x) {
+      const int b = std::min(n, W * (x * q + std::min(x, rem)));
+      const int e = std::min(n, b + W * (q + (x < rem ? 1 : 0)));
+      std::stable_sort(items.begin() + b, items.begin() + e, [](const Piece& u, const Piece& v) {
+        if (u.rows != v.rows) return u.rows > v.rows;
+        return u.inst != v.inst ? u.inst < v.inst : u.y0 < v.y0;
+      });
+      std::vector<Group> run;
+      for (int i = b; i < e; i += W) {
+        Group g;
+        while (g.n < W && i + g.n < e) { g.p[g.n] = items[i + g.n]; ++g.n; }
+        run.push_back(g);
+      }
+      balance_rounds(run, (int)std::max(1L, cus / 8));
+      groups.insert(groups.end(), run.begin(), run.end());
+    }
+  }
+  // Launch order.  Workgroup b of a launch runs on XCD b % 8 and takes group
+  // x*q + min(x, rem) + (b >> 3) (fv_step_kernel), so XCD x works through the
+  // run of groups [x*q + min(x, rem), ...) in order, and within a run the
+  // hardware starts groups in that order, one per CU, then the next round of
+  // CU slots.  A SIMD issues for its oldest wave first, so the rounds take the
+  // levels in turn, tallest first: the waves that start first get the most
+  // rows, and a SIMD's waves finish together instead of leaving one wave alone
+  // at the end.  Cut A: CU c of an XCD takes groups L c .. L c + L - 1 of the
+  // run (neighbouring rows, equal sums); cut B was sorted above.
+  std::vector<int> order(groups.size());
+  {
+    const int n = (int)groups.size(), q = n >> 3, rem = n & 7;
+    for (int x = 0; x < 8; ++x) {
+      const int b = x * q + std::min(x, rem), e = b + q + (x < rem ? 1 : 0);
+      int at = b;
+      const int L = running ? levels : 1;
+      // the level pattern starts anew every L groups of the whole list
+      for (int l = 0; l < L; ++l)
+        for (int g = b; g < e; ++g)
+          if (g % L == l) order[at++] = g;
+    }
+  }
+  for (int g : order) {
+    int used = 0;
+    for (int j = 0; j < groups[g].n; ++j) {
+      const Piece& pc = groups[g].p[j];
+      const std::vector<int> h = group_heights(pc.rows, pc.waves);
+      int y = pc.y0;
+      for (size_t w = 0; w < h.size(); ++w) {
+        fv::WorkItem it;
+        it.inst = pc.inst;
+        it.x0 = pc.x0;
+        it.y0 = y;
+        it.y1 = y + h[w];
+        it.mrow = pc.mrow + (y - pc.y0);
+        it.local = out.n_items[pc.inst]++;
+        it.bc = ps[pc.inst].bc;
+        it.role = used++ | (w + 1 < h.size() ? fv::kRoleAbove : 0);
+        out.items.push_back(it);
+        y = it.y1;
       }
     }
-    out.n_items[k] = n;
+    out.group_first.push_back((int32_t)out.items.size());
   }
-  order_for_launch(out.items);
+}
+
+std::vector<fv::WorkItem> launch_items(const WorkList& wl, long cus) {
+  fv::WorkItem none;
+  std::memset(&none, 0, sizeof(none));
+  const int n = (int)wl.group_first.size() - 1, W = fv::kGroupWaves;
+  std::vector<fv::WorkItem> v((size_t)n * W, none);
+  // the waves of a workgroup go to its CU's SIMDs in turn, and an XCD's
+  // groups to its CUs in turn: each group's tallest wave takes the place of
+  // the SIMD with the least steps so far
+  const int C = (int)std::max(1L, cus / 8), q = n >> 3, rem = n & 7;
+  for (int x = 0; x < 8; ++x) {
+    const int b = x * q + std::min(x, rem), e = b + q + (x < rem ? 1 : 0);
+    std::vector<double> load((size_t)C * W, 0.0);
+    for (int g = b; g < e; ++g) {
+      double* ld = &load[(size_t)((g - b) % C) * W];
+      std::pair<double, int> waves[fv::kGroupWaves];
+      int place[fv::kGroupWaves], m = 0;
+      for (int i = wl.group_first[g]; i < wl.group_first[g + 1]; ++i)
+        waves[m++] = {wl.items[i].y1 - wl.items[i].y0 +
+                          (wl.items[i].role & fv::kRoleAbove ? 0.0 : kTail), -i};
+      std::sort(waves, waves + m, [](const auto& u, const auto& w) { return u > w; });
+      for (int j = 0; j < W; ++j) place[j] = j;
+      std::sort(place, place + W, [&](int u, int w) {
+        return ld[u] != ld[w] ? ld[u] < ld[w] : u < w;
+      });
+      for (int j = 0; j < m; ++j) {
+        v[(size_t)g * W + place[j]] = wl.items[-waves[j].second];
+        ld[place[j]] += waves[j].first;
+      }
+    }
+  }
+  return v;
 }
 
 void build_adj_items(const std::vector<fivonagi_params>& ps, long target_waves,

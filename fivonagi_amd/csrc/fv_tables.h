@@ -46,31 +46,43 @@ void table_bytes(const std::vector<double>& v, bool f64, char* out);
 // (fv::CflMask) and bitmap?
 bool cfl_counted(int cfl_mask, const std::vector<uint32_t>& fold_bits, int nx, int i, int j);
 
-// Rows per work item: the smallest height (never below 12) whose total wave
-// count over all instances fits target_waves.
+// Rows per item of the in-step cut (see build_work): the smallest height
+// (never below 12) whose total wave count over all instances fits target_waves.
 int auto_rows(const std::vector<fivonagi_params>& ps, long target_waves);
+
+// Heights, bottom to top, of the waves (at most max_waves) that share R rows of
+// a strip in one workgroup.
+std::vector<int> group_heights(int R, int max_waves);
 
 // Row boundaries of one strip cut into `chunks` work items (skewed heights,
 // `levels` levels, pattern rotated by rot).
 std::vector<int> chunk_bounds(int ny, int chunks, float skew, int levels, int rot);
 
-// Launch order of the work items: each XCD's run sorted by height, tallest first.
-void order_for_launch(std::vector<fv::WorkItem>& items);
-
 // The work list of the step kernel.
 struct WorkList {
-  std::vector<fv::WorkItem> items;
-  std::vector<uint64_t> rowmask;     // CFL lane mask per item row (fv::WorkItem::mrow)
+  std::vector<fv::WorkItem> items;   // workgroup by workgroup in launch order, each bottom
+                                     // to top
+  std::vector<int32_t> group_first;  // workgroup g: items group_first[g] .. group_first[g+1]
+  std::vector<uint64_t> rowmask;     // CFL lane mask per row of each strip (fv::WorkItem::mrow)
   std::vector<int> n_items;          // per instance
   float skew_used = 0.0f;
   bool rotate_used = false;
 };
-// cus, per_cu: the device's CUs and resident step waves per CU; auto_h: the
-// rows per item of instances without their own rows_per_wave; skew < 0:
-// automatic.
+// The strips are cut in one of two ways (same results):
+//   running on  the strips laid end to end, dealt to workgroups of up to
+//               kGroupWaves waves of about equal march steps, one above the
+//               other, which hand their seam rows over in LDS;
+//   in step     one wave per item, every strip of an instance cut at the same
+//               rows, auto_h (or the instance's rows_per_wave) rows each.
+// cus, per_cu: the device's CUs and resident step waves per CU; skew < 0:
+// automatic, as the choice of the cut then is; else rotate picks running on.
+// cell_bytes: bytes of state, in and out, per cell.
 void build_work(const std::vector<fivonagi_params>& ps, const std::vector<int>& cfl_mask,
                 const std::vector<std::vector<uint32_t>>& fold_bits, long cus, int per_cu,
-                int auto_h, float skew, bool rotate, WorkList& out);
+                int auto_h, float skew, bool rotate, WorkList& out, int cell_bytes = 24);
+// The items as the step kernel reads them: kGroupWaves places per workgroup
+// (an unused place has no rows).
+std::vector<fv::WorkItem> launch_items(const WorkList& wl, long cus);
 
 // Work items of the adjoint's reverse march (fv_adjoint_march.hip): strips
 // of 56 output columns cut into row ranges, items in instance and strip

@@ -107,9 +107,16 @@ struct InstDesc {
   double hifu_k_d;      // FREC/4
 };
 
+// Waves of a step workgroup: items of one strip, one above the other
+// (fv_step.hip, "Seams").
+constexpr int kGroupWaves = 4;
+// WorkItem::role: the wave's place in its workgroup, counted from the bottom,
+// and whether a wave sits above it.
+constexpr int32_t kRoleIndex = 3, kRoleAbove = 4;
+
 // One wave's work: a 58-column strip of one instance, rows [y0, y1).
-// mrow: index of the item's first row in the CFL lane-mask table; entry
-// mrow + (j - y0) has bit l set when lane l's cell (x0 - 3 + l, j) is an
+// mrow: index of the item's first row in the CFL lane-mask table (a strip's
+// rows 0 .. ny-1 are contiguous there); entry mrow + (j - y0) has bit l set when lane l's cell (x0 - 3 + l, j) is an
 // output cell with i >= 1 that the CFL reduction counts.  local: the item's
 // index among its instance's items (0 publishes the instance's control block;
 // local % kGroups picks the reduction slot), independent of the launch order.
@@ -120,7 +127,7 @@ struct WorkItem {
   int32_t mrow;
   int32_t local;
   int32_t bc;           // the instance's boundary kind (picks the app's march)
-  int32_t pad;
+  int32_t role;         // kRole*
 };
 
 }  // namespace fv

@@ -39,12 +39,13 @@ _FIRST_ORDER = (
     "  {M}[0] = fvna::fma_(be1, w_.a1, be2 * w_.a2);\n"
     "  {M}[1] = fvna::fma_(be1, w_.w21, be2 * w_.w22);\n"
     "  {M}[2] = fvna::fma_(be3, w_.a3, fvna::fma_(be1, w_.w31, be2 * w_.w32)); }}")
-_Y_LIMITER = ("    fvna::limited_flux(fc.f, fc.dl[0], fn.dl[0], fc.dl[1], fn.dl[1], fc.dl[2], fn.dl[2], dty,\n"
-              "                       fc.P, M);")
-_X_LIMITER = "    fvna::limited_flux(fx, dl1, dr1, dl2, dr2, dl3, dr3, dtx, PX, MX);"
+_Y_LIMITER = ("      fvna::limited_flux<false>(fc.f, fc.dl[0], fn.dl[0], fc.dl[1], fn.dl[1], fc.dl[2], fn.dl[2],\n"
+              "                                dty, fc.P, M);")
+_X_LIMITER = "    fvna::limited_flux<true>(fx, dl1, dr1, dl2, dr2, dl3, dr3, dtx, PX, MX);"
 _X_START = "    const R ir = fvna::rcp(R(1) + y1q);\n    const R un = y2q * ir, ut = y3q * ir;"
-_Y_RIEMANN = ("    fvna::riemann(bm.q1, bm.q3, bm.q2, bm.un, bm.ut, bn.q1, bn.q3, bn.q2, bn.un, bn.ut,\n"
-              "                  hbeta, fn.f);")
+_Y_RIEMANN = ("      fvna::riemann(fvna::jump(bm.q1, bm.q3, bm.q2, bm.un, bm.ut, bn.q1, bn.q3, bn.q2, bn.un,\n"
+              "                               bn.ut),\n"
+              "                    hbeta, fn.f);")
 _SOURCE = ("    R r2 = fvna::apply_source(mid.q2, i2);\n"
            "    R r3 = fvna::apply_source(mid.q3, i3);")
 

@@ -89,7 +89,7 @@ typedef struct {
   int32_t error, cur;
   int32_t n_items, rows_per_wave; /* work items per step, mean rows per item */
   double skew;             /* height skew of the work items in use            */
-  int32_t rotate;          /* 1: skew levels rotated per strip                */
+  int32_t rotate;          /* 1: fivonagi_set_skew's rotate, with a skew > 0   */
   int32_t phase;           /* next step launch mod 6 (captured graphs replay
                               from phase 0)                                   */
   int32_t md_x, md_y;      /* moving-window offset MDX, MDY                   */
@@ -148,10 +148,12 @@ int fivonagi_autotune(fivonagi_ctx *ctx, int trial_steps, int32_t *rows_per_wave
    waves each SIMD starts (at most its resident count), from (1+s)H to
    (1-s)H, the tallest launched first, which evens out when the waves sharing
    a SIMD finish; < 0 = automatic (0.5 when every SIMD starts its full
-   complement of step waves, else 0).  rotate != 0 shifts the level pattern by
-   one per strip (same count per level; strips no longer share cut rows).
-   Which is fastest depends on the grid: fivonagi_autotune tries them.
-   Results do not depend on it. */
+   complement of step waves, else 0).  With skew >= 0, rotate != 0 cuts the
+   strips running on, one after another, into workgroups whose waves share
+   their seam rows; rotate = 0 cuts every strip of an instance at the same rows,
+   one wave per item.  Automatic: running on up to 256 MiB of state (in and
+   out), which the memory-side cache holds.  Which is fastest depends on the
+   grid: fivonagi_autotune tries them.  Results do not depend on it. */
 int fivonagi_set_skew(fivonagi_ctx *ctx, double skew, int rotate);
 
 /* dataCollect/dataExport stand-in (apps/hifu-beam/data_export.h:29-75):
