@@ -59,14 +59,16 @@ template <bool kL3Product>
 __device__ __forceinline__ void limiter_rec(const Iface& f, float dl1, float dr1, float dl2,
                                             float dr2, float dl3, float dr3, float dtd,
                                             float P[3], float M[3], LimT& t) {
-  fvna::limited_flux<kL3Product>(f, dl1, dr1, dl2, dr2, dl3, dr3, dtd, P, M);
+  const float up1 = fvna::upwind(f.L1, dl1, dr1), up2 = fvna::upwind(f.L2, dl2, dr2);
+  const float up3 = fvna::upwind(f.L3, dl3, dr3);
+  fvna::limited_flux<kL3Product>(f, up1, up2, up3, dtd, P, M);
   const Waves& w = f.w;
   const float n1 = fvna::fma_(w.a1, w.a1, fvna::fma_(w.w21, w.w21, w.w31 * w.w31));
   const float n2 = fvna::fma_(w.a2, w.a2, fvna::fma_(w.w22, w.w22, w.w32 * w.w32));
   const float n3 = w.a3 * w.a3;
-  lim_part(n1, f.L1 > 0.0f ? dl1 : dr1, t.h[0], t.qd[0], t.r[0]);
-  lim_part(n2, f.L2 > 0.0f ? dl2 : dr2, t.h[1], t.qd[1], t.r[1]);
-  lim_part(n3, f.L3 > 0.0f ? dl3 : dr3, t.h[2], t.qd[2], t.r[2]);
+  lim_part(n1, up1, t.h[0], t.qd[0], t.r[0]);
+  lim_part(n2, up2, t.h[1], t.qd[1], t.r[1]);
+  lim_part(n3, up3, t.h[2], t.qd[2], t.r[2]);
 }
 
 // Adjoint of one interface's waves (a1, w21, w31, a2, w22, w32, a3) and

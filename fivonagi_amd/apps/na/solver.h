@@ -100,7 +100,6 @@ struct IfaceT {
   WavesT<R> w;
   R L1, L2, L3;         // speeds s1, s2, s3
   R s2, rS;             // L3 = s2 * rS (limited_flux's kL3Product)
-  R smax;               // max |s_p| (|L3| <= max(|L1|,|L2|) since L3 is their mean)
   bool bad;             // tmp3 < 0: imaginary eigenvalue (simError = 2)
 };
 typedef WavesT<float> Waves;
@@ -154,7 +153,6 @@ __device__ __forceinline__ void riemann(const JumpT<R>& j, R hbeta, IfaceT<R>& f
   f.w.a1 = a1; f.w.w21 = a1 * L1; f.w.w31 = a1 * A1;
   f.w.a2 = a2; f.w.w22 = a2 * L2; f.w.w32 = a2 * A2;
   f.w.a3 = dtg - fma_(a1, A1, f.w.w32);                         // fv.h:119-125
-  f.smax = fmax2(fabs(L1), fabs(L2));
 }
 
 // MC limiter phi(r) = max(0, min((1+r)/2, 2, 2r)) (fv.h:587-605), returned
@@ -183,28 +181,34 @@ __device__ __forceinline__ R dot2(const WavesT<R>& a, const WavesT<R>& b) {
   return fma_(b.a2, a.a2, fma_(b.w22, a.w22, b.w32 * a.w32));
 }
 
+// The dot product with the upwind neighbour by the sign of the speed s:
+// dotl = W . W(k-1), dotr = W . W(k+1).
+template <typename R>
+__device__ __forceinline__ R upwind(R s, R dotl, R dotr) {
+  return s > R(0) ? dotl : dotr;
+}
+
 // Fluctuations (fv.h:141-180) and correction flux fadd (fv.h:666-711) of one
 // interface, folded into what the two adjacent cells need:
 //   P = apdq - fadd = sum_p (max(s_p,0) - c_p) W_p   (cell on the + side)
 //   M = amdq + fadd = sum_p (min(s_p,0) + c_p) W_p   (cell on the - side)
 // with c_p = |s_p| (1 - |s_p| dt/d) phi_p / 2 = |s_p| (1 - |s_p| dt/d) philim_half.  A wave with s_p = 0 enters
 // neither fluctuation, as in the reference.
-// dotl_p = W_p . W_p(k-1), dotr_p = W_p . W_p(k+1); upwind by sign(s_p).
+// up_p = W_p . W_p of the upwind neighbour (upwind()).
 // kL3Product: be_3 = L3 - al_3 from the product L3 = s2 rS with one rounding
 // (the x sweep, which has both factors at hand; the y sweep keeps L3 alone
 // in its window).
 template <bool kL3Product, typename R>
-__device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R dotl1, R dotr1, R dotl2,
-                                             R dotr2, R dotl3, R dotr3, R dtd, R P[3],
-                                             R M[3]) {
+__device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R up1, R up2, R up3, R dtd,
+                                             R P[3], R M[3]) {
 #pragma clang fp contract(off)
   const WavesT<R>& w = f.w;
   const R n1 = fma_(w.a1, w.a1, fma_(w.w21, w.w21, w.w31 * w.w31));
   const R n2 = fma_(w.a2, w.a2, fma_(w.w22, w.w22, w.w32 * w.w32));
   const R n3 = w.a3 * w.a3;
-  const R h1 = philim_half(n1, f.L1 > R(0) ? dotl1 : dotr1);
-  const R h2 = philim_half(n2, f.L2 > R(0) ? dotl2 : dotr2);
-  const R h3 = philim_half(n3, f.L3 > R(0) ? dotl3 : dotr3);
+  const R h1 = philim_half(n1, up1);
+  const R h2 = philim_half(n2, up2);
+  const R h3 = philim_half(n3, up3);
   const R s1 = fabs(f.L1), s2 = fabs(f.L2), s3 = fabs(f.L3);
   // c_p = g_p h_p
   const R g1 = s1 * fma_(-s1, dtd, R(1));

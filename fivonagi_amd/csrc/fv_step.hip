@@ -28,13 +28,16 @@
 // below ends its march on those values.  Only the topmost wave of a workgroup
 // marches the five rows past its last.
 //
-// The march is bound by VALU issue (about 270 instructions per row of a wave)
+// The march is bound by VALU issue (about 250 instructions per row of a wave)
 // and, on small grids, by the length of the longest wave's march, so both gain
 // from rows not repeated: a wave of 18 rows marched 21.3 rows' worth alone and
 // 18.8 in a group of four, and a group of 16 rows marches 6 steps where a lone
 // item needed 17.  Per step, one wave per workgroup against groups of four:
 // 4096x1024 40.7 -> 36.9 us, 2048x2048 43.2 -> 37.5, 1024x1024 20.9 -> 16.6,
 // 400x400 16.4 -> 8.7 (FP32).  Waves per group: two gave 38.4 on 4096x1024.
+// Then 13 VALU instructions fewer per row (neighbour operands by DPP, the CFL
+// maximum under the mask, dt/d carried from row to row): 37.3 -> 36.1 us on
+// 4096x1024, 64.7 -> 62.3 on 4096x2048, 237 -> 228 on 8192x4096.
 //
 // CFL and accept/reject: each wave reduces its cells' cfl to one float and
 // folds it into its group's 128-byte line (8 groups per instance) with one
@@ -129,15 +132,73 @@ __device__ __forceinline__ double unif(double v) {
   return __longlong_as_double(uni64(__double_as_longlong(v)));
 }
 
-// v on the lanes whose bit of the uniform 64-bit mask is set, 0 elsewhere
-// (one v_cndmask with the mask as the lane condition).
-__device__ __forceinline__ float lane_sel(uint64_t mask, float v) {
-  float d;
-  asm("v_cndmask_b32_e64 %0, 0, %1, %2" : "=v"(d) : "v"(v), "s"(mask));
-  return d;
+// S <- max(S, |a|, |b|) (the largest speed: |L3| <= max(|L1|, |L2|), whose mean
+// it is) on the lanes whose bit of the uniform mask is set: one
+// VALU instruction under the mask as the execution mask (the march's lanes are
+// all active around it), where a select and two maxima take three.
+__device__ __forceinline__ void masked_max(uint64_t mask, float& S, float a, float b) {
+  uint64_t keep;
+  asm("s_and_saveexec_b64 %1, %4\n\t"
+      "v_max3_f32 %0, %0, |%2|, |%3|\n\t"
+      "s_mov_b64 exec, %1"
+      : "+v"(S), "=&s"(keep)
+      : "v"(a), "v"(b), "s"(mask)
+      : "scc");
 }
-__device__ __forceinline__ double lane_sel(uint64_t mask, double v) {
-  return ((mask >> __lane_id()) & 1ull) ? v : 0.0;
+__device__ __forceinline__ void masked_max(uint64_t mask, double& S, double a, double b) {
+  const double v = ((mask >> __lane_id()) & 1ull) ? fmax(fabs(a), fabs(b)) : 0.0;
+  S = fmax(S, v);
+}
+
+// Products with the left neighbour's waves: the same sums as fvna::dot1/dot2
+// (a, shr1(a)), each multiply-add taking its neighbour operand by DPP.  The
+// compiler folds a cross-lane move only into two-operand forms it has before
+// register allocation, never into a multiply-add, so these are written out;
+// s_nop covers the two wait states between a VALU write and a DPP read.
+__device__ __forceinline__ void dots_left(const fvna::WavesT<float>& w, float& d1, float& d2,
+                                          float& d3) {
+  asm("s_nop 1\n\t"
+      "v_mul_f32_dpp %0, %5, %5 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "v_mul_f32_dpp %1, %8, %8 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "v_mul_f32_dpp %2, %9, %9 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "v_fmac_f32_dpp %0, %4, %4 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "v_fmac_f32_dpp %1, %7, %7 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "v_fmac_f32_dpp %0, %3, %3 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "v_fmac_f32_dpp %1, %6, %6 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+      : "=&v"(d1), "=&v"(d2), "=&v"(d3)
+      : "v"(w.a1), "v"(w.w21), "v"(w.w31), "v"(w.a2), "v"(w.w22), "v"(w.w32), "v"(w.a3));
+}
+__device__ __forceinline__ void dots_left(const fvna::WavesT<double>& w, double& d1, double& d2,
+                                          double& d3) {
+  fvna::WavesT<double> l;
+  l.a1 = shr1(w.a1); l.w21 = shr1(w.w21); l.w31 = shr1(w.w31);
+  l.a2 = shr1(w.a2); l.w22 = shr1(w.w22); l.w32 = shr1(w.w32);
+  l.a3 = shr1(w.a3);
+  d1 = fvna::dot1(w, l);
+  d2 = fvna::dot2(w, l);
+  d3 = w.a3 * l.a3;
+}
+
+// fvna::upwind of the x sweep: dl on the lanes with a positive speed, else the
+// right neighbour's dl, whose move folds into the select.
+__device__ __forceinline__ void upwind_x(const fvna::IfaceT<float>& f, float dl1, float dl2,
+                                         float dl3, float& up1, float& up2, float& up3) {
+  asm("s_nop 0\n\t"
+      "v_cmp_lt_f32_e32 vcc, 0, %3\n\t"
+      "v_cndmask_b32_dpp %0, %6, %6, vcc wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "v_cmp_lt_f32_e32 vcc, 0, %4\n\t"
+      "v_cndmask_b32_dpp %1, %7, %7, vcc wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "v_cmp_lt_f32_e32 vcc, 0, %5\n\t"
+      "v_cndmask_b32_dpp %2, %8, %8, vcc wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+      : "=&v"(up1), "=&v"(up2), "=&v"(up3)
+      : "v"(f.L1), "v"(f.L2), "v"(f.L3), "v"(dl1), "v"(dl2), "v"(dl3)
+      : "vcc");
+}
+__device__ __forceinline__ void upwind_x(const fvna::IfaceT<double>& f, double dl1, double dl2,
+                                         double dl3, double& up1, double& up2, double& up3) {
+  up1 = fvna::upwind(f.L1, dl1, shl1(dl1));
+  up2 = fvna::upwind(f.L2, dl2, shl1(dl2));
+  up3 = fvna::upwind(f.L3, dl3, shl1(dl3));
 }
 
 // Pins a value in a register here: its computation cannot sink into a
@@ -632,6 +693,15 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
 
   // dt/d on the lanes of interior columns, 0 on ghost columns
   const R dty_c = col_int ? dty : R(0), dtx_c = col_int ? dtx : R(0);
+  // the same on the rows of interior cells, 0 on ghost rows: ghost cells keep
+  // their value (the fluxes are finite wherever the attempt is valid, so
+  // q - 0*flux == q exactly).  In FP32 the row's two are kept from row to row,
+  // changed where the interior starts and ends; in FP64 they are selected anew
+  // each row (four registers fewer: 70.2 against 70.7 us on 4096x1024).
+  // Starts at row y0 - 1, the first one swept
+  constexpr bool kCarryRow = sizeof(R) == 4;
+  const bool first_int = y0 >= 3 && y0 <= ny - 2;
+  R dtyu = first_int ? dty_c : R(0), dtxu = first_int ? dtx_c : R(0);
   R Sx = R(0), Sy = R(0);
   uint64_t err = 0;                          // lanes that met tmp3 < 0 (or NaN)
   const uint64_t in_mask = __builtin_amdgcn_ballot_w64(col_in);
@@ -672,6 +742,13 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
     if constexpr (kT >= 6) {
       if (r >= y0 + 4) source_store(r - 4, xn, xo, xm);
     }
+    // row m = r-2 is the first interior row, or the first ghost row above
+    if constexpr (kT >= 4 && kCarryRow) {
+      if (r == 4 || r == ny) {
+        dtyu = r == 4 ? dty_c : R(0);
+        dtxu = r == 4 ? dtx_c : R(0);
+      }
+    }
     // the next row, also past the item's last row: the row index is clamped
     // to the grid, and an unconditional load needs no copy of the registers
     // it replaces
@@ -690,7 +767,7 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
       // branch-free (a branch here would split the block and stop the
       // cross-lane moves of the x sweep from folding into their users)
       err |= __builtin_amdgcn_ballot_w64(fn.f.bad) & ((r >= 1 && r < ny) ? in_mask : 0);
-      Sy = fvna::fmax2(Sy, lane_sel(mY, fn.f.smax));
+      masked_max(mY, Sy, fn.f.L1, fn.f.L2);
       if constexpr (kT == 1) {
         seam_put(s_out, kSeamW + 0, fn.f.w.a1);  seam_put(s_out, kSeamW + 1, fn.f.w.w21);
         seam_put(s_out, kSeamW + 2, fn.f.w.w31); seam_put(s_out, kSeamW + 3, fn.f.w.a2);
@@ -729,8 +806,9 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
     // ---- y limiter at interface r-1 ----
     R M[3];
     if constexpr (kT <= 8) {
-      fvna::limited_flux<false>(fc.f, fc.dl[0], fn.dl[0], fc.dl[1], fn.dl[1], fc.dl[2], fn.dl[2],
-                                dty, fc.P, M);
+      fvna::limited_flux<false>(fc.f, fvna::upwind(fc.f.L1, fc.dl[0], fn.dl[0]),
+                                fvna::upwind(fc.f.L2, fc.dl[1], fn.dl[1]),
+                                fvna::upwind(fc.f.L3, fc.dl[2], fn.dl[2]), dty, fc.P, M);
     } else {
 #pragma unroll
       for (int p = 0; p < 3; ++p) M[p] = seam_get(s_in, kSeamM + p);
@@ -743,11 +821,11 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
 
     // ---- q_y on row m = r-2 (components: density, normal=q3, tangential=q2)
     const uint64_t mX = (m >= 0 && m < ny) ? bo.cm : 0;
-    const bool row_int = (m >= 2) && (m <= ny - 3);
-    // ghost cells keep their value: dt/d is 0 there (the fluxes are finite
-    // wherever the attempt is valid, so q - 0*flux == q exactly); the column
-    // test is folded in once per item (dty_c, dtx_c), the row test here
-    const R dtyu = row_int ? dty_c : R(0), dtxu = row_int ? dtx_c : R(0);
+    if constexpr (!kCarryRow) {
+      const bool row_int = (m >= 2) && (m <= ny - 3);
+      dtyu = row_int ? dty_c : R(0);
+      dtxu = row_int ? dtx_c : R(0);
+    }
     const R y1q = fvna::sub_prod(bo.q1, dtyu, fl.P[0] + M[0]);
     const R y3q = fvna::sub_prod(bo.q3, dtyu, fl.P[1] + M[1]);
     const R y2q = fvna::sub_prod(bo.q2, dtyu, fl.P[2] + M[2]);
@@ -764,18 +842,15 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
     pin(jx.s1); pin(jx.s2); pin(jx.s3); pin(jx.drho); pin(jx.dn); pin(jx.dtg);
     fvna::riemann(jx, hbeta, fx);
     err |= __builtin_amdgcn_ballot_w64(fx.bad) & ((m >= 0 && m < ny) ? x_mask : 0);
-    Sx = fvna::fmax2(Sx, lane_sel(mX, fx.smax));
-    // waves of the interface to the left (k-1)
-    fvna::WavesT<R> wl;
-    wl.a1 = shr1(fx.w.a1); wl.w21 = shr1(fx.w.w21); wl.w31 = shr1(fx.w.w31);
-    wl.a2 = shr1(fx.w.a2); wl.w22 = shr1(fx.w.w22); wl.w32 = shr1(fx.w.w32);
-    wl.a3 = shr1(fx.w.a3);
-    const R dl1 = fvna::dot1(fx.w, wl), dl2 = fvna::dot2(fx.w, wl);
-    const R dl3 = fx.w.a3 * wl.a3;
+    masked_max(mX, Sx, fx.L1, fx.L2);
+    // W(k).W(k-1), with the waves of the interface to the left
+    R dl1, dl2, dl3;
+    dots_left(fx.w, dl1, dl2, dl3);
     // W(k).W(k+1) is the right neighbour's W(k+1).W(k)
-    const R dr1 = shl1(dl1), dr2 = shl1(dl2), dr3 = shl1(dl3);
+    R up1, up2, up3;
+    upwind_x(fx, dl1, dl2, dl3, up1, up2, up3);
     R PX[3], MX[3];
-    fvna::limited_flux<true>(fx, dl1, dr1, dl2, dr2, dl3, dr3, dtx, PX, MX);
+    fvna::limited_flux<true>(fx, up1, up2, up3, dtx, PX, MX);
     const R mr0 = shl1(MX[0]), mr1 = shl1(MX[1]), mr2 = shl1(MX[2]);
     xn.q1 = fvna::sub_prod(y1q, dtxu, mr0 + PX[0]);
     xn.q2 = fvna::sub_prod(y2q, dtxu, mr1 + PX[1]);

@@ -39,9 +39,10 @@ _FIRST_ORDER = (
     "  {M}[0] = fvna::fma_(be1, w_.a1, be2 * w_.a2);\n"
     "  {M}[1] = fvna::fma_(be1, w_.w21, be2 * w_.w22);\n"
     "  {M}[2] = fvna::fma_(be3, w_.a3, fvna::fma_(be1, w_.w31, be2 * w_.w32)); }}")
-_Y_LIMITER = ("      fvna::limited_flux<false>(fc.f, fc.dl[0], fn.dl[0], fc.dl[1], fn.dl[1], fc.dl[2], fn.dl[2],\n"
-              "                                dty, fc.P, M);")
-_X_LIMITER = "    fvna::limited_flux<true>(fx, dl1, dr1, dl2, dr2, dl3, dr3, dtx, PX, MX);"
+_Y_LIMITER = ("      fvna::limited_flux<false>(fc.f, fvna::upwind(fc.f.L1, fc.dl[0], fn.dl[0]),\n"
+              "                                fvna::upwind(fc.f.L2, fc.dl[1], fn.dl[1]),\n"
+              "                                fvna::upwind(fc.f.L3, fc.dl[2], fn.dl[2]), dty, fc.P, M);")
+_X_LIMITER = "    fvna::limited_flux<true>(fx, up1, up2, up3, dtx, PX, MX);"
 _X_START = "    const R ir = fvna::rcp(R(1) + y1q);\n    const R un = y2q * ir, ut = y3q * ir;"
 _Y_RIEMANN = ("      fvna::riemann(fvna::jump(bm.q1, bm.q3, bm.q2, bm.un, bm.ut, bn.q1, bn.q3, bn.q2, bn.un,\n"
               "                               bn.ut),\n"
@@ -59,7 +60,7 @@ VARIANTS = {
                     " xn.v = xn.q3 * ir2; }\n    return;\n" + _X_START)],
     "no y sweep": [(_Y_RIEMANN,
                     "    fn.f = fvna::IfaceT<R>{}; fn.f.L1 = R(1); fn.f.L2 = R(-1);"
-                    " fn.f.smax = R(1);\n    pin(bm.q1); pin(bn.q1);"),
+                    "\n    pin(bm.q1); pin(bn.q1);"),
                    (_Y_LIMITER, "    fc.P[0] = fc.P[1] = fc.P[2] = M[0] = M[1] = M[2] = R(0);")],
     "no source": [(_SOURCE, "    R r2 = mid.q2; R r3 = mid.q3; (void)i2; (void)i3;")],
 }
