@@ -293,13 +293,12 @@ class Context:
         p = self.problems[inst]
         dtype, ct = (np.float64, C.c_double) if self.fp64 else (np.float32, C.c_float)
         fn = load().fivonagi_collect_f64 if self.fp64 else load().fivonagi_collect
-        q = np.zeros((3, p.ny, p.nx), dtype)
+        q = np.empty((3, p.ny, p.nx), dtype)
         T, dt = C.c_double(), C.c_double()
         na, nr = C.c_int64(), C.c_int64()
-        fpp = [np.ascontiguousarray(q[k]) for k in range(3)]
-        _check(fn(self._h, inst, *[a.ctypes.data_as(C.POINTER(ct)) for a in fpp],
+        _check(fn(self._h, inst, *[q[k].ctypes.data_as(C.POINTER(ct)) for k in range(3)],
                   C.byref(T), C.byref(dt), C.byref(na), C.byref(nr)))
-        return np.stack(fpp), dict(T=T.value, dt=dt.value, n_accepted=na.value,
+        return q, dict(T=T.value, dt=dt.value, n_accepted=na.value,
                                    n_rejected=nr.value)
 
     def info(self, inst=0):
@@ -338,10 +337,10 @@ class Context:
     def adjoint_state(self, inst=0):
         """dJ/d(state at the start of the last step_adjoint call), (3, ny, nx)."""
         p = self.problems[inst]
-        ls = [np.zeros((p.ny, p.nx), np.float32) for _ in range(3)]
+        lam = np.empty((3, p.ny, p.nx), np.float32)
         _check(load().fivonagi_adjoint_state(
-            self._h, inst, *[a.ctypes.data_as(C.POINTER(C.c_float)) for a in ls]))
-        return np.stack(ls)
+            self._h, inst, *[lam[k].ctypes.data_as(C.POINTER(C.c_float)) for k in range(3)]))
+        return lam
 
     def set_collect(self, inst, jcut=2, mic=(0, 0, 0, 0), eta=1.0, on=True, cut_half=0,
                     tan_theta=0.0):
@@ -364,11 +363,11 @@ class Context:
         p = self.problems[inst]
         rows = p.ny if rows is None else int(rows)
         if self.fp64:
-            m = np.zeros((rows, p.nx), np.float64)
+            m = np.empty((rows, p.nx), np.float64)
             _check(load().fivonagi_measure_rows_f64(self._h, inst, rows,
                                                     m.ctypes.data_as(C.POINTER(C.c_double))))
         else:
-            m = np.zeros((rows, p.nx), np.float32)
+            m = np.empty((rows, p.nx), np.float32)
             _check(load().fivonagi_measure_rows(self._h, inst, rows,
                                                 m.ctypes.data_as(C.POINTER(C.c_float))))
         return m

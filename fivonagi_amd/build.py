@@ -17,7 +17,7 @@ SOURCES = [os.path.join(HERE, "csrc", n) for n in ("fv_step.hip", "fv_adjoint_ma
 ARCH = os.environ.get("FIVONAGI_ARCH", "gfx950")
 
 HIPCC_FLAGS = [
-    f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
+    f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared", "-pthread",
     # no packed FP32 (v_pk_*_f32) anywhere in device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # kernel arguments arrive preloaded in SGPRs (gfx950): a wave's first

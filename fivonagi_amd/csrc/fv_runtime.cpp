@@ -8,13 +8,16 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstdint>
 #include <cstring>
 #include <limits>
+#include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/fivonagi.h"
@@ -27,7 +30,10 @@ extern "C" hipError_t fv_launch_step(const fv::InstDesc* insts, const fv::WorkIt
                                      int n_inst, fv::Ctl* ctl0, fv::SyncSlots* sync0, int bc0,
                                      int ext, int fp64, hipStream_t stream);
 extern "C" hipError_t fv_launch_settle(const fv::InstDesc* insts, int n_inst, int phase,
-                                       hipStream_t stream);
+                                       fv::Ctl* mirror, hipStream_t stream);
+extern "C" hipError_t fv_launch_targets(const fv::InstDesc* insts, int n_inst, int phase,
+                                        const int64_t* targets, int64_t target, double T_stop,
+                                        hipStream_t stream);
 extern "C" hipError_t fv_launch_collect(const fv::InstDesc* insts, int n_inst, int max_nx,
                                         int phase, int fp64, hipStream_t stream);
 extern "C" hipError_t fv_step_waves_per_cu(int* waves, int fp64);
@@ -66,8 +72,94 @@ int hip_fail(hipError_t e, const char* what) {
 
 }  // namespace
 
+// Pinned host memory shared by the contexts of the process (allocating it takes
+// 0.2 ms and more a call): staging buffers of downloads, one per call in
+// progress, of which up to kKept idle ones are kept; and the contexts' control
+// mirrors, cut from slabs that hold kSlabBlocks of them.  All of it is freed
+// with the last context.
+namespace {
+constexpr int kStageSlots = 8;
+constexpr size_t kStageBytes = 16u << 20;
+constexpr size_t kMirrorBytes = 4096;      // a context's control mirror that fits a slab
+class PinnedPool {
+ public:
+  void enter() {
+    std::lock_guard<std::mutex> lk(mu_);
+    ++users_;
+  }
+  void leave() {
+    std::vector<void*> old;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (--users_ == 0) {
+        old.swap(idle_);
+        old.insert(old.end(), slabs_.begin(), slabs_.end());
+        slabs_.clear();
+        blocks_.clear();
+      }
+    }
+    for (void* p : old) (void)hipHostFree(p);
+  }
+  char* take_stage() {                     // null where no pinned memory is left
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (!idle_.empty()) {
+        void* p = idle_.back();
+        idle_.pop_back();
+        return (char*)p;
+      }
+    }
+    return (char*)pinned(kStageBytes);
+  }
+  void give_stage(char* p) {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (idle_.size() < kKept && users_ > 0) {
+        idle_.push_back(p);
+        return;
+      }
+    }
+    (void)hipHostFree(p);
+  }
+  void* take_mirror() {                    // kMirrorBytes, or null
+    std::lock_guard<std::mutex> lk(mu_);
+    if (blocks_.empty()) {
+      char* s = (char*)pinned(kSlabBlocks * kMirrorBytes);
+      if (!s) return nullptr;
+      slabs_.push_back(s);
+      for (size_t k = 0; k < kSlabBlocks; ++k) blocks_.push_back(s + k * kMirrorBytes);
+    }
+    void* p = blocks_.back();
+    blocks_.pop_back();
+    return p;
+  }
+  void give_mirror(void* p) {
+    std::lock_guard<std::mutex> lk(mu_);
+    blocks_.push_back(p);
+  }
+
+ private:
+  static void* pinned(size_t n) {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, n, hipHostMallocPortable) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  static constexpr size_t kKept = 2, kSlabBlocks = 64;
+  std::mutex mu_;
+  std::vector<void*> idle_, slabs_, blocks_;
+  int users_ = 0;
+};
+PinnedPool& pinned_pool() {
+  static PinnedPool* pool = new PinnedPool;   // never destroyed: contexts may outlive statics
+  return *pool;
+}
+}  // namespace
+
 struct fivonagi_ctx {
   int device = 0;
+  bool pool_user = false;                  // counted by the pinned pool
+  bool mirror_pooled = false;              // h_ctl comes from it
   hipStream_t own_stream = nullptr;
   hipStream_t stream = nullptr;
   int n_inst = 0;
@@ -124,6 +216,12 @@ struct fivonagi_ctx {
   // or host write (read_ctls, launch_attempts, write_ctls)
   std::vector<fv::Ctl> ctl_cache;
   bool ctl_cache_ok = false;
+  // pinned host memory: the control blocks as the settle kernel leaves them,
+  // then the targets the targets kernel reads
+  fv::Ctl* h_ctl = nullptr;
+  int64_t* h_targets = nullptr;
+  bool targets_pending = false;            // a launch may still have to read h_targets
+  hipEvent_t stage_ev[kStageSlots] = {};   // downloads: a slot of the staging buffer is full
 
   void* dalloc(size_t bytes, hipError_t* e) {
     void* p = nullptr;
@@ -147,6 +245,11 @@ struct fivonagi_ctx {
     if (d_items) (void)hipFree(d_items);
     if (d_rowmask) (void)hipFree(d_rowmask);
     for (void* p : allocs) (void)hipFree(p);
+    if (h_ctl && mirror_pooled) pinned_pool().give_mirror(h_ctl);
+    else if (h_ctl) (void)hipHostFree(h_ctl);
+    for (hipEvent_t e : stage_ev)
+      if (e) (void)hipEventDestroy(e);
+    if (pool_user) pinned_pool().leave();
     if (own_stream) (void)hipStreamDestroy(own_stream);
   }
 };
@@ -222,21 +325,18 @@ void set_ctl_derived(fv::Ctl& t, const fv::InstDesc& d) {
 
 // The control blocks after the last launched attempt: the settle kernel
 // folds that attempt's reduction into block (a+1)%2 (a = next attempt index),
-// which is where the next launch will store the same result.
+// which is where the next launch will store the same result, and into pinned
+// host memory.
 int read_ctls(fivonagi_ctx* c, std::vector<fv::Ctl>& out) {
   if (c->ctl_cache_ok) {
     out = c->ctl_cache;
     return 0;
   }
   const int phase = (int)(c->attempts % 6);
-  HIP_TRY(fv_launch_settle(c->d_desc, c->n_inst, phase, c->stream));
-  std::vector<fv::Ctl> both(2 * (size_t)c->n_inst);
-  HIP_TRY(hipMemcpyAsync(both.data(), c->d_ctl, sizeof(fv::Ctl) * both.size(),
-                         hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(fv_launch_settle(c->d_desc, c->n_inst, phase, c->h_ctl, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
-  out.resize(c->n_inst);
-  const int b = (phase + 1) & 1;
-  for (int k = 0; k < c->n_inst; ++k) out[k] = both[2 * (size_t)k + b];
+  c->targets_pending = false;
+  out.assign(c->h_ctl, c->h_ctl + c->n_inst);
   c->ctl_cache = out;
   c->ctl_cache_ok = true;
   return 0;
@@ -278,16 +378,19 @@ hipError_t launch_phase(fivonagi_ctx* c, int phase) {
 }
 
 // data collection overflow flags (any instance collecting): FIVONAGI_ERR_COLLECT or 0
+int collect_overflow(fivonagi_ctx* c, const std::vector<uint32_t>& flags) {
+  for (int k = 0; k < c->n_inst; ++k)
+    if (flags[k] && c->desc[k].measure)
+      return fail(FIVONAGI_ERR_COLLECT, "data collection: more than nx steps in a frame");
+  return 0;
+}
 int collect_status(fivonagi_ctx* c) {
   if (!c->d_collect_err) return 0;
   std::vector<uint32_t> v(c->n_inst);
   HIP_TRY(hipMemcpyAsync(v.data(), c->d_collect_err, sizeof(uint32_t) * c->n_inst,
                          hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
-  for (int k = 0; k < c->n_inst; ++k)
-    if (v[k] && c->desc[k].measure)
-      return fail(FIVONAGI_ERR_COLLECT, "data collection: more than nx steps in a frame");
-  return 0;
+  return collect_overflow(c, v);
 }
 
 // The captured graph of G attempts from phase 0 (phases 0..G-1 mod 6),
@@ -367,16 +470,133 @@ int check_ctx(fivonagi_ctx* c, int inst) {
 }
 
 // Stop conditions of the attempts launched from now on: an instance runs
-// while n_acc < tgt[k] and T < T_stop.
+// while n_acc < tgt[k] and T < T_stop.  One launch, no host round trip.
 int write_targets(fivonagi_ctx* c, const std::vector<int64_t>& tgt,
                   double T_stop = std::numeric_limits<double>::infinity()) {
-  std::vector<fv::Ctl> ctl;
-  if (int rc = read_ctls(c, ctl)) return rc;
-  for (int k = 0; k < c->n_inst; ++k) {
-    ctl[k].target_acc = tgt[k];
-    ctl[k].T_stop = T_stop;
+  const int64_t* list = nullptr;
+  if (c->n_inst > 1) {
+    if (c->targets_pending) HIP_TRY(hipStreamSynchronize(c->stream));
+    std::copy(tgt.begin(), tgt.end(), c->h_targets);
+    c->targets_pending = true;
+    list = c->h_targets;
   }
-  return write_ctls(c, ctl);
+  c->ctl_cache_ok = false;
+  HIP_TRY(fv_launch_targets(c->d_desc, c->n_inst, (int)(c->attempts % 6), list, tgt[0], T_stop,
+                            c->stream));
+  return 0;
+}
+
+// A device range for the host.
+struct Span {
+  const void* src;
+  void* dst;
+  size_t bytes;
+};
+
+// Copies device ranges to pageable host memory, after the work on the
+// context's stream.  They go through a pinned buffer: one synchronisation
+// where they are small, else a ring of slots filled by the device while up to kCopyThreads threads, ended before
+// the call returns, empty it -- the copy into fresh host pages is what bounds a
+// large download (8192x4096, 403 MB: 75 ms through the runtime's own staging
+// and a second host copy).
+int download(fivonagi_ctx* c, const std::vector<Span>& spans) {
+  constexpr size_t kThreadBytes = 4u << 20;      // up to this: the caller's thread alone
+  static_assert(kThreadBytes <= kStageBytes, "a small download fits the buffer");
+  constexpr int kCopyThreads = 4;
+  size_t total = 0;
+  for (const Span& s : spans) total += s.bytes;
+  struct Stage {
+    char* p = pinned_pool().take_stage();
+    ~Stage() { if (p) pinned_pool().give_stage(p); }
+  } stage;
+  if (!stage.p) {                                // no pinned memory: the runtime's own copies
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    for (const Span& s : spans)
+      if (s.bytes) HIP_TRY(hipMemcpy(s.dst, s.src, s.bytes, hipMemcpyDeviceToHost));
+    return 0;
+  }
+  if (total <= kThreadBytes) {
+    size_t off = 0;
+    for (const Span& s : spans) {
+      if (s.bytes)
+        HIP_TRY(hipMemcpyAsync(stage.p + off, s.src, s.bytes, hipMemcpyDeviceToHost, c->stream));
+      off += s.bytes;
+    }
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    c->targets_pending = false;
+    off = 0;
+    for (const Span& s : spans) {
+      std::memcpy(s.dst, stage.p + off, s.bytes);
+      off += s.bytes;
+    }
+    return 0;
+  }
+  constexpr int kSlots = kStageSlots;
+  for (hipEvent_t& e : c->stage_ev)
+    if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  constexpr size_t slot = kStageBytes / kSlots;
+  std::vector<Span> chunks;
+  for (const Span& s : spans)
+    for (size_t o = 0; o < s.bytes; o += slot)
+      chunks.push_back({(const char*)s.src + o, (char*)s.dst + o, std::min(slot, s.bytes - o)});
+  const int n = (int)chunks.size();
+  std::vector<std::atomic<int>> state(n);        // 0 waiting, 1 requested, 2 in the caller's memory
+  for (auto& v : state) v.store(0);
+  std::atomic<int> next{0};
+  std::atomic<int> err{0};
+  auto empty_one = [&](int i) {
+    const int k = i % kSlots;
+    const hipError_t e = hipEventSynchronize(c->stage_ev[k]);
+    if (e != hipSuccess) err.store((int)e);
+    else std::memcpy(chunks[i].dst, stage.p + (size_t)k * slot, chunks[i].bytes);
+    state[i].store(2);
+  };
+  auto worker = [&]() {
+    (void)hipSetDevice(c->device);
+    for (;;) {
+      const int i = next.fetch_add(1);
+      if (i >= n) return;
+      while (state[i].load() == 0) {
+        if (err.load()) { state[i].store(2); return; }
+        std::this_thread::yield();
+      }
+      empty_one(i);
+    }
+  };
+  std::vector<std::thread> threads;
+  threads.reserve(kCopyThreads);
+  try {
+    for (int t = 0; t < kCopyThreads; ++t) threads.emplace_back(worker);
+  } catch (const std::exception&) {
+    // fewer threads, or none, than asked for: the caller's helps below
+  }
+  for (int i = 0; i < n && !err.load(); ++i) {
+    if (i >= kSlots) {                           // the slot's last chunk must be out
+      while (state[i - kSlots].load() != 2 && !err.load()) {
+        if (threads.empty()) {
+          const int j = next.fetch_add(1);
+          empty_one(j);                          // j <= i - 1: requested already
+        } else {
+          std::this_thread::yield();
+        }
+      }
+      if (err.load()) break;
+    }
+    const int k = i % kSlots;
+    hipError_t e = hipMemcpyAsync(stage.p + (size_t)k * slot, chunks[i].src, chunks[i].bytes,
+                                  hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipEventRecord(c->stage_ev[k], c->stream);
+    if (e != hipSuccess) { err.store((int)e); break; }
+    state[i].store(1);
+  }
+  if (threads.empty())
+    for (int j = next.fetch_add(1); j < n && !err.load(); j = next.fetch_add(1)) empty_one(j);
+  for (auto& t : threads) t.join();
+  if (err.load()) {
+    (void)hipStreamSynchronize(c->stream);       // nothing writes the staging buffer any more
+    return hip_fail((hipError_t)err.load(), "download");
+  }
+  return 0;
 }
 
 // Parameters every entry point that sets up an instance accepts.
@@ -417,6 +637,7 @@ static int init_impl(fivonagi_ctx** out, const fivonagi_params* p, int n_inst,
   c->n_inst = n_inst;
   c->fp64 = f64;
   const size_t es = f64 ? sizeof(double) : sizeof(float);
+  constexpr size_t kFieldFromHost = 1u << 20;
   c->params.assign(p, p + n_inst);
   c->desc.resize(n_inst);
   c->dt_seq_dev.assign(n_inst, nullptr);
@@ -445,6 +666,18 @@ static int init_impl(fivonagi_ctx** out, const fivonagi_params* p, int n_inst,
   if (e != hipSuccess) { delete c; return hip_fail(e, "hipStreamCreate"); }
   c->stream = c->own_stream;
 
+  pinned_pool().enter();
+  c->pool_user = true;
+  const size_t mirror = (sizeof(fv::Ctl) + sizeof(int64_t)) * n_inst;
+  if (mirror <= kMirrorBytes) {
+    c->h_ctl = (fv::Ctl*)pinned_pool().take_mirror();
+    c->mirror_pooled = c->h_ctl != nullptr;
+  }
+  if (!c->h_ctl) {
+    e = hipHostMalloc((void**)&c->h_ctl, mirror, hipHostMallocDefault);
+    if (e != hipSuccess) { delete c; return hip_fail(e, "hipHostMalloc"); }
+  }
+  c->h_targets = (int64_t*)(c->h_ctl + n_inst);
   c->d_ctl = (fv::Ctl*)c->dalloc(sizeof(fv::Ctl) * 2 * n_inst, &e);
   if (e != hipSuccess) { delete c; return hip_fail(e, "hipMalloc ctl"); }
   c->d_sync = (fv::SyncSlots*)c->dalloc(sizeof(fv::SyncSlots) * 3 * n_inst, &e);
@@ -465,8 +698,14 @@ static int init_impl(fivonagi_ctx** out, const fivonagi_params* p, int n_inst,
       for (int f = 0; f < 3; ++f) d.q[b][f] = (float*)(buf + es * (size_t)(3 * b + f) * n);
     for (int f = 0; f < 3; ++f) {
       e = hipMemcpy(d.q[0][f], q_host[3 * k + f], es * n, hipMemcpyHostToDevice);
+      // the second buffer: a small field from the host again (the first copy
+      // between device buffers on a new stream costs more), a large one below
+      if (e == hipSuccess && es * n <= kFieldFromHost)
+        e = hipMemcpy(d.q[1][f], q_host[3 * k + f], es * n, hipMemcpyHostToDevice);
       if (e != hipSuccess) { delete c; return hip_fail(e, "hipMemcpy state"); }
-      e = hipMemcpy(d.q[1][f], q_host[3 * k + f], es * n, hipMemcpyHostToDevice);
+    }
+    if (es * n > kFieldFromHost) {
+      e = hipMemcpyAsync(d.q[1][0], d.q[0][0], 3 * es * n, hipMemcpyDeviceToDevice, c->stream);
       if (e != hipSuccess) { delete c; return hip_fail(e, "hipMemcpy state"); }
     }
     // a table in the context's precision on the device
@@ -815,9 +1054,11 @@ static int measure_impl(fivonagi_ctx* c, int inst, int rows, H* out) {
   const auto& d = c->desc[inst];
   if (!d.measure) return fail(FIVONAGI_ERR_ARG, "data collection is off for this instance");
   if (rows < 0 || rows > d.ny) return fail(FIVONAGI_ERR_ARG, "rows outside 0..ny");
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  HIP_TRY(hipMemcpy(out, d.measure, sizeof(H) * (size_t)d.nx * rows, hipMemcpyDeviceToHost));
-  return collect_status(c);
+  std::vector<uint32_t> flags(c->n_inst, 0u);
+  if (int rc = download(c, {{d.measure, out, sizeof(H) * (size_t)d.nx * rows},
+                            {c->d_collect_err, flags.data(), sizeof(uint32_t) * c->n_inst}}))
+    return rc;
+  return collect_overflow(c, flags);
 }
 
 // The relative errors of apps/taylor-angle-xy/data_export.h:96-122 in its own
@@ -858,11 +1099,15 @@ static int collect_impl(fivonagi_ctx* c, int inst, H* q1, H* q2, H* q3, double* 
   const bool same = c->fp64 == (sizeof(H) == sizeof(double));
   std::vector<double> vd;
   std::vector<float> vf;
-  for (int f = 0; f < 3; ++f) {
+  if (same) {
+    std::vector<Span> spans;
+    for (int f = 0; f < 3; ++f)
+      if (dst[f]) spans.push_back({d.q[t.cur][f], dst[f], sizeof(H) * n});
+    if (int rc = download(c, spans)) return rc;
+  }
+  for (int f = 0; f < 3 && !same; ++f) {
     if (!dst[f]) continue;
-    if (same) {
-      HIP_TRY(hipMemcpy(dst[f], d.q[t.cur][f], sizeof(H) * n, hipMemcpyDeviceToHost));
-    } else if (c->fp64) {
+    if (c->fp64) {
       vd.resize(n);
       HIP_TRY(hipMemcpy(vd.data(), d.q[t.cur][f], sizeof(double) * n, hipMemcpyDeviceToHost));
       for (size_t o = 0; o < n; ++o) dst[f][o] = (H)vd[o];
@@ -1329,11 +1574,10 @@ int fivonagi_adjoint_state(fivonagi_ctx* c, int inst, float* l1, float* l2, floa
     return fail(FIVONAGI_ERR_ARG, "no adjoint has been run on this context");
   const size_t n = (size_t)c->params[inst].nx * c->params[inst].ny;
   float* dst[3] = {l1, l2, l3};
+  std::vector<Span> spans;
   for (int f = 0; f < 3; ++f)
-    if (dst[f])
-      HIP_TRY(hipMemcpy(dst[f], c->adj_lam[inst] + (size_t)f * n, sizeof(float) * n,
-                        hipMemcpyDeviceToHost));
-  return 0;
+    if (dst[f]) spans.push_back({c->adj_lam[inst] + (size_t)f * n, dst[f], sizeof(float) * n});
+  return download(c, spans);
 }
 
 int fivonagi_step_noalloc(const fivonagi_params* p, float* const q[6], int64_t nsteps,
@@ -1445,7 +1689,7 @@ int fivonagi_step_noalloc(const fivonagi_params* p, float* const q[6], int64_t n
     }
     // the control block after the last attempt (fv_settle_kernel), read back
     const int phase = (int)(a % 6);
-    HIP_TRY(fv_launch_settle(d_desc, 1, phase, stream));
+    HIP_TRY(fv_launch_settle(d_desc, 1, phase, nullptr, stream));
     HIP_TRY(hipMemcpyAsync(&now, d.ctl + ((phase + 1) & 1), sizeof(fv::Ctl),
                            hipMemcpyDeviceToHost, stream));
     HIP_TRY(hipStreamSynchronize(stream));

@@ -971,13 +971,35 @@ __global__ __launch_bounds__(kLanes * kGroupWaves) void fv_step_kernel(
 }
 
 // Control block after the last launched attempt (phase = index of the next
-// attempt mod 6), stored where that attempt's launch will store it too; the
-// host reads it after a synchronisation.  One block per instance.
+// attempt mod 6), stored where that attempt's launch will store it too, and
+// into mirror (host memory, when given), which the host reads after a
+// synchronisation.  One block per instance.
 __global__ __launch_bounds__(64) void fv_settle_kernel(const InstDesc* __restrict__ insts,
-                                                       int phase) {
+                                                       int phase, Ctl* __restrict__ mirror) {
   const InstDesc& D = insts[blockIdx.x];
   const Ctl P = current(D, phase, true);
-  if (threadIdx.x == 0) D.ctl[(phase + 1) & 1] = P;
+  if (threadIdx.x == 0) {
+    D.ctl[(phase + 1) & 1] = P;
+    if (mirror) mirror[blockIdx.x] = P;
+  }
+}
+
+// Stop conditions of the attempts from phase on: the control block that
+// attempt would form, with the new conditions, becomes the block it starts
+// from, and the attempt before it is marked as folded in.  One block per
+// instance; targets: host memory, or null for `target` itself.
+__global__ __launch_bounds__(64) void fv_targets_kernel(const InstDesc* __restrict__ insts,
+                                                        int phase,
+                                                        const int64_t* __restrict__ targets,
+                                                        int64_t target, double T_stop) {
+  const InstDesc& D = insts[blockIdx.x];
+  Ctl P = current(D, phase, true);
+  if (threadIdx.x == 0) {
+    P.target_acc = targets ? targets[blockIdx.x] : target;
+    P.T_stop = T_stop;
+    D.ctl[phase & 1] = P;
+    D.sync[(phase + 2) % 3].ran = 0u;
+  }
 }
 
 // Data collection of attempt a, run after its step launch: if the attempt
@@ -1089,9 +1111,19 @@ extern "C" hipError_t fv_launch_collect(const fv::InstDesc* insts, int n_inst, i
 }
 
 extern "C" hipError_t fv_launch_settle(const fv::InstDesc* insts, int n_inst, int phase,
-                                       hipStream_t stream) {
+                                       fv::Ctl* mirror, hipStream_t stream) {
   if (n_inst <= 0) return hipSuccess;
-  hipLaunchKernelGGL(fv::fv_settle_kernel, dim3(n_inst), dim3(64), 0, stream, insts, phase);
+  hipLaunchKernelGGL(fv::fv_settle_kernel, dim3(n_inst), dim3(64), 0, stream, insts, phase,
+                     mirror);
+  return hipGetLastError();
+}
+
+extern "C" hipError_t fv_launch_targets(const fv::InstDesc* insts, int n_inst, int phase,
+                                        const int64_t* targets, int64_t target, double T_stop,
+                                        hipStream_t stream) {
+  if (n_inst <= 0) return hipSuccess;
+  hipLaunchKernelGGL(fv::fv_targets_kernel, dim3(n_inst), dim3(64), 0, stream, insts, phase,
+                     targets, target, T_stop);
   return hipGetLastError();
 }
 
