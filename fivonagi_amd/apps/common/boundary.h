@@ -9,12 +9,12 @@
 //
 //   kId            the instance's boundary kind (FIVONAGI_BC_*)
 //   kRowData       the policy reads per-row tables (RowData) with each row
-//   kPrepass       ghost cells written before the step by prepass() (their
+//   kPrepass       ghost cells made ahead of the step by prepass() (their
 //                  values depend on T and the cell only); the step copies them
 //   kExtOnly       the app always runs with the extended step (its instances
 //                  set it), so the plain step need not carry its march
 //   lane(ic, nx, m)                  once per lane: the source columns
-//   offset(rc, ny, m, row_bytes)     per row: byte offset of the source cell
+//   offset(rc, ny, m, row_bytes, size)   per row: byte offset of the source cell
 //   load_row(tb, rc, h)              per row: the row's table entries
 //   patch(c, rc, q, h)               per row: values that are not copies
 //
@@ -39,10 +39,13 @@ __device__ __forceinline__ int md_shift(double T, double md_t, double v, double 
 }
 
 // A lane's source columns: bA on rows 2..ny-3, bB on the ghost rows (bytes).
+// ring, ny: set before lane(): InstDesc::ring (0: none) and the grid's height.
 struct LaneMap {
   uint32_t bA, bB;
   bool left;         // the lane's column is a left ghost column (i <= 1)
   int ic;            // the lane's column, clamped to the grid
+  uint32_t ring = 0;
+  int ny = 0;
 };
 
 // The instance's per-row tables (device pointers, the context's precision):
@@ -95,7 +98,8 @@ struct ZeroGradient {
     m.bA = size * (uint32_t)colA;
     m.bB = size * (uint32_t)colB;
   }
-  __device__ static uint32_t offset(int rc, int ny, const LaneMap& m, uint32_t row_bytes) {
+  __device__ static uint32_t offset(int rc, int ny, const LaneMap& m, uint32_t row_bytes,
+                                    uint32_t size) {
     const bool grow = (rc <= 1) || (rc >= ny - 2);
     const int jm = rc >= ny - 2 ? ny - 3 : (rc <= 1 ? 2 : rc);
     const uint32_t rowL = (uint32_t)rc * row_bytes, rowM = (uint32_t)jm * row_bytes;

@@ -31,8 +31,9 @@ struct EdgeDrive {
   __device__ static void lane(int ic, int nx, LaneMap& m, uint32_t size) {
     ZeroGradient::lane(ic, nx, m, size);
   }
-  __device__ static uint32_t offset(int rc, int ny, const LaneMap& m, uint32_t row_bytes) {
-    return ZeroGradient::offset(rc, ny, m, row_bytes);
+  __device__ static uint32_t offset(int rc, int ny, const LaneMap& m, uint32_t row_bytes,
+                                    uint32_t size) {
+    return ZeroGradient::offset(rc, ny, m, row_bytes, size);
   }
   template <typename R>
   __device__ static void load_row(const Tables& tb, int rc, RowData<R>& h) {

@@ -45,7 +45,8 @@ struct Hifu {
     const int col = m.left ? 2 : (ic >= nx - 2 ? nx - 3 : ic);
     m.bA = m.bB = size * (uint32_t)col;
   }
-  __device__ static uint32_t offset(int rc, int ny, const LaneMap& m, uint32_t row_bytes) {
+  __device__ static uint32_t offset(int rc, int ny, const LaneMap& m, uint32_t row_bytes,
+                                    uint32_t size) {
     // bottom rows mirror rows 4, 3; top rows copy ny-3
     const int jm = rc <= 1 ? 4 - rc : (rc >= ny - 2 ? ny - 3 : rc);
     return (uint32_t)jm * row_bytes + m.bA;

@@ -13,13 +13,13 @@ namespace fvbc {
 
 // Data collection of the hifu app (apps/hifu-beam/data_collect.h:51-106) for
 // one accepted attempt: row jcut of its new state, staged by the step before
-// the window shift, read with the pre-shift MDX.  Thread i = column i.
+// the window shift (stage), read with the pre-shift MDX.  Thread i = column i.
 template <typename R>
-__device__ void collect_hifu(const fv::InstDesc& D, const fv::Ctl& P, double T, int64_t nf,
-                             R* __restrict__ m, int i) {
+__device__ void collect_hifu(const fv::InstDesc& D, const fv::Ctl& P, const R* __restrict__ stage,
+                             double T, int64_t nf, R* __restrict__ m, int i) {
   const int nx = D.nx, ny = D.ny;
   if (i >= nx) return;
-  const R u1 = ((const R*)D.stage)[i];
+  const R u1 = stage[i];
   const int mdx = P.mdx;
   for (int k = 0; k < 4; ++k) {                     // data_collect.h:51-76
     if (i + mdx == D.mic[k]) {

@@ -155,7 +155,7 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
   pc.any_left = __builtin_amdgcn_ballot_w64(lm.left) != 0;
   auto load_raw = [&](int r, float& a, float& b, float& c, fvbc::RowData<float>& h) {
     const int rc = min(max(r, 0), ny - 1);
-    const uint32_t o = BC::offset(rc, ny, lm, row_bytes);
+    const uint32_t o = BC::offset(rc, ny, lm, row_bytes, 4u);
     a = ldg(in1, o);
     b = ldg(in2, o);
     c = ldg(in3, o);

@@ -28,21 +28,23 @@
 extern "C" hipError_t fv_launch_step(const fv::InstDesc* insts, const fv::WorkItem* items,
                                      const uint64_t* rowmask, int n_groups, int phase,
                                      int n_inst, fv::Ctl* ctl0, fv::SyncSlots* sync0, int bc0,
-                                     int ext, int fp64, hipStream_t stream);
+                                     int ext, int fp64, int beside, int collect,
+                                     hipStream_t stream);
 extern "C" hipError_t fv_launch_settle(const fv::InstDesc* insts, int n_inst, int phase,
                                        fv::Ctl* mirror, hipStream_t stream);
 extern "C" hipError_t fv_launch_targets(const fv::InstDesc* insts, int n_inst, int phase,
                                         const int64_t* targets, int64_t target, double T_stop,
                                         hipStream_t stream);
 extern "C" hipError_t fv_launch_collect(const fv::InstDesc* insts, int n_inst, int max_nx,
-                                        int phase, int fp64, hipStream_t stream);
+                                        int phase, hipStream_t stream);
 extern "C" hipError_t fv_step_waves_per_cu(int* waves, int fp64);
 extern "C" hipError_t fv_adj_reverse(const fv::AdjDesc* ds, const fv::AdjItem* items,
                                      const int32_t* wave_first, int n_waves, int k, int slot,
                                      int par, int check, hipStream_t s);
 extern "C" hipError_t fv_adj_occupancy(int* waves_per_cu);
 extern "C" hipError_t fv_launch_taylor_ghosts(const fv::InstDesc* insts, int n_inst,
-                                              int max_ring, int phase, hipStream_t stream);
+                                              int max_ring, int phase, int settle,
+                                              hipStream_t stream);
 extern "C" hipError_t fv_scratch_get(void** ptr, size_t* bytes);
 
 using fvh::auto_rows;
@@ -196,6 +198,7 @@ struct fivonagi_ctx {
   // the rest; at most kGraphCache lengths are kept (the oldest goes first)
   static constexpr int kGraphChunk = 300, kGraphCache = 8;
   int taylor_ring = 0;                     // largest ghost ring of a Taylor instance
+  bool ring_all = true;                    // every Taylor instance's buffers have a ring
   int collect_nx = 0;                      // widest instance with data collection (0: none)
   bool keep_hist = false;                  // the step stores accepted states into the
                                            // instances' histories (adjoint forward pass)
@@ -359,21 +362,26 @@ int write_ctls(fivonagi_ctx* c, const std::vector<fv::Ctl>& in) {
   return 0;
 }
 
-// One step attempt: the Taylor ghost pre-pass (only if a Taylor instance
-// exists) and the fused step, for attempt index = phase (mod 6).
-hipError_t launch_phase(fivonagi_ctx* c, int phase) {
-  if (c->taylor_ring > 0) {
+// One step attempt, attempt index = phase (mod 6).  begin, end: the first and
+// the last of a run of launches.  What surrounds the step -- the Taylor ghost
+// ring the attempt reads, and its data collection -- is launched by itself only
+// there; between them each step launch collects the attempt before it and makes
+// the ring of the one after it (fv_step.hip, beside_step).
+hipError_t launch_phase(fivonagi_ctx* c, int phase, bool begin, bool end) {
+  if (c->taylor_ring > 0 && (begin || !c->ring_all)) {
     hipError_t e =
-        fv_launch_taylor_ghosts(c->d_desc, c->n_inst, c->taylor_ring, phase, c->stream);
+        fv_launch_taylor_ghosts(c->d_desc, c->n_inst, c->taylor_ring, phase, 0, c->stream);
     if (e != hipSuccess) return e;
   }
+  const int threads = fv::kLanes * fv::kGroupWaves;
+  const int collect = begin ? 0 : (c->collect_nx + threads - 1) / threads;
+  const int ring = end ? 0 : (c->taylor_ring + threads - 1) / threads;
   hipError_t e = fv_launch_step(c->d_desc, c->d_items, c->d_rowmask, c->n_groups(),
                                 phase, c->n_inst, c->d_ctl, c->d_sync, c->params[0].bc,
                                 c->ext_any || c->keep_hist ? 1 : 0, c->fp64 ? 1 : 0,
-                                c->stream);
-  if (e == hipSuccess && c->collect_nx > 0)
-    e = fv_launch_collect(c->d_desc, c->n_inst, c->collect_nx, phase, c->fp64 ? 1 : 0,
-                          c->stream);
+                                collect + ring, collect, c->stream);
+  if (e == hipSuccess && end && c->collect_nx > 0)
+    e = fv_launch_collect(c->d_desc, c->n_inst, c->collect_nx, phase, c->stream);
   return e;
 }
 
@@ -408,7 +416,7 @@ int graph_for(fivonagi_ctx* c, int G, hipGraphExec_t* out) {
   }
   HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   for (int a = 0; a < G; ++a) {
-    hipError_t e = launch_phase(c, a % 6);
+    hipError_t e = launch_phase(c, a % 6, a == 0, a == G - 1);
     if (e != hipSuccess) {
       hipGraph_t g = nullptr;
       (void)hipStreamEndCapture(c->stream, &g);
@@ -434,7 +442,7 @@ int graph_for(fivonagi_ctx* c, int G, hipGraphExec_t* out) {
 int launch_attempts(fivonagi_ctx* c, int64_t n) {
   c->ctl_cache_ok = false;
   while (n > 0 && c->attempts % 6 != 0) {
-    hipError_t e = launch_phase(c, (int)(c->attempts % 6));
+    hipError_t e = launch_phase(c, (int)(c->attempts % 6), true, true);
     if (e != hipSuccess) return hip_fail(e, "fv_launch_step");
     ++c->attempts;
     --n;
@@ -448,18 +456,23 @@ int launch_attempts(fivonagi_ctx* c, int64_t n) {
     n -= G;
     // a graph of a length that is not a multiple of 6 ends mid-rotation
     while (n > 0 && c->attempts % 6 != 0) {
-      hipError_t e = launch_phase(c, (int)(c->attempts % 6));
+      hipError_t e = launch_phase(c, (int)(c->attempts % 6), true, true);
       if (e != hipSuccess) return hip_fail(e, "fv_launch_step");
       ++c->attempts;
       --n;
     }
   }
   while (n > 0) {
-    hipError_t e = launch_phase(c, (int)(c->attempts % 6));
+    hipError_t e = launch_phase(c, (int)(c->attempts % 6), true, true);
     if (e != hipSuccess) return hip_fail(e, "fv_launch_step");
     ++c->attempts;
     --n;
   }
+  // a last attempt that was not accepted leaves the ghost cells it read in its
+  // input, which stays the state
+  if (c->taylor_ring > 0)
+    HIP_TRY(fv_launch_taylor_ghosts(c->d_desc, c->n_inst, c->taylor_ring,
+                                    (int)(c->attempts % 6), 1, c->stream));
   return 0;
 }
 
@@ -692,10 +705,21 @@ static int init_impl(fivonagi_ctx** out, const fivonagi_params* p, int n_inst,
     auto& d = c->desc[k];
     d = h.d;
     const size_t n = (size_t)q.nx * q.ny;
-    char* buf = (char*)c->dalloc(es * n * 6, &e);
+    // a Taylor instance's fields are followed by their ghost ring, where the
+    // kernels' 32-bit offsets reach it
+    size_t nf = n;
+    if (h.taylor_ring > 0) {
+      if (es * (n + h.taylor_ring) <= ((size_t)1 << 32) - 1) {
+        d.ring = (uint32_t)(es * n);
+        nf = n + h.taylor_ring;
+      } else {
+        c->ring_all = false;
+      }
+    }
+    char* buf = (char*)c->dalloc(es * nf * 6, &e);
     if (e != hipSuccess) { delete c; return hip_fail(e, "hipMalloc state"); }
     for (int b = 0; b < 2; ++b)
-      for (int f = 0; f < 3; ++f) d.q[b][f] = (float*)(buf + es * (size_t)(3 * b + f) * n);
+      for (int f = 0; f < 3; ++f) d.q[b][f] = (float*)(buf + es * (size_t)(3 * b + f) * nf);
     for (int f = 0; f < 3; ++f) {
       e = hipMemcpy(d.q[0][f], q_host[3 * k + f], es * n, hipMemcpyHostToDevice);
       // the second buffer: a small field from the host again (the first copy
@@ -705,7 +729,8 @@ static int init_impl(fivonagi_ctx** out, const fivonagi_params* p, int n_inst,
       if (e != hipSuccess) { delete c; return hip_fail(e, "hipMemcpy state"); }
     }
     if (es * n > kFieldFromHost) {
-      e = hipMemcpyAsync(d.q[1][0], d.q[0][0], 3 * es * n, hipMemcpyDeviceToDevice, c->stream);
+      e = hipMemcpyAsync(d.q[1][0], d.q[0][0], es * (2 * nf + n), hipMemcpyDeviceToDevice,
+                         c->stream);
       if (e != hipSuccess) { delete c; return hip_fail(e, "hipMemcpy state"); }
     }
     // a table in the context's precision on the device
@@ -1016,11 +1041,11 @@ int fivonagi_set_collect(fivonagi_ctx* c, int inst, const fivonagi_collect_opts*
     if (!b.measure) {
       hipError_t e;
       b.measure = c->dalloc(es * (size_t)nx * ny, &e);
-      if (e == hipSuccess) b.stage = c->dalloc(es * (size_t)nx, &e);
+      if (e == hipSuccess) b.stage = c->dalloc(es * 2 * (size_t)nx, &e);
       if (e != hipSuccess) return hip_fail(e, "hipMalloc (collect)");
     }
     HIP_TRY(hipMemsetAsync(b.measure, 0, es * (size_t)nx * ny, c->stream));
-    HIP_TRY(hipMemsetAsync(b.stage, 0, es * (size_t)nx, c->stream));
+    HIP_TRY(hipMemsetAsync(b.stage, 0, es * 2 * (size_t)nx, c->stream));
     HIP_TRY(hipMemsetAsync(c->d_collect_err + inst, 0, sizeof(uint32_t), c->stream));
     d.measure = b.measure;
     d.stage = taylor ? nullptr : b.stage;   // the Taylor cut reads the output state
@@ -1481,6 +1506,7 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
         d.measure = nullptr;
         d.stage = nullptr;
         d.md_on = 0;
+        d.ring = 0;                    // the segment's slots have no ghost ring
         rdh[(size_t)s * ni + k] = d;
         // the logged block as the attempt's own (an idle fold keeps it as is)
         fv::Ctl t = hlog[(size_t)k * nsteps + s0 + s];
@@ -1501,16 +1527,16 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
     for (int s = 0; s + 1 < len && !keep_all; ++s) {
       const fv::InstDesc* di = d_rdesc + (size_t)s * ni;
       if (c->taylor_ring > 0)
-        HIP_TRY(fv_launch_taylor_ghosts(di, ni, c->taylor_ring, 0, c->stream));
+        HIP_TRY(fv_launch_taylor_ghosts(di, ni, c->taylor_ring, 0, 0, c->stream));
       HIP_TRY(fv_launch_step(di, c->d_items, c->d_rowmask, c->n_groups(), 0, ni,
                              one ? d_rctl + 2 * (size_t)s : nullptr, one ? d_rsync : nullptr,
-                             c->params[0].bc, c->ext_any ? 1 : 0, 0, c->stream));
+                             c->params[0].bc, c->ext_any ? 1 : 0, 0, 0, 0, c->stream));
     }
     for (int s = len - 1; s >= 0; --s) {
       // q_n as the step read it: the Taylor ghost ring of its T (a state the
       // recompute stepped has it already; writing it again changes nothing)
       if (c->taylor_ring > 0)
-        HIP_TRY(fv_launch_taylor_ghosts(d_rdesc + (size_t)s * ni, ni, c->taylor_ring, 0,
+        HIP_TRY(fv_launch_taylor_ghosts(d_rdesc + (size_t)s * ni, ni, c->taylor_ring, 0, 0,
                                         c->stream));
       HIP_TRY(fv_adj_reverse(d_ad, d_items, d_wave_first, (int)wave_first.size() - 1,
                              (int)(s0 + s), (int)(slot0 + s), par, check ? 1 : 0, c->stream));
@@ -1683,9 +1709,9 @@ int fivonagi_step_noalloc(const fivonagi_params* p, float* const q[6], int64_t n
     for (int64_t k = 0; k < remaining; ++k, ++a) {
       const int phase = (int)(a % 6);
       if (h.taylor_ring > 0)
-        HIP_TRY(fv_launch_taylor_ghosts(d_desc, 1, h.taylor_ring, phase, stream));
+        HIP_TRY(fv_launch_taylor_ghosts(d_desc, 1, h.taylor_ring, phase, 0, stream));
       HIP_TRY(fv_launch_step(d_desc, d_items, d_mask, n_groups, phase, 1, d.ctl, d.sync, p->bc,
-                             ext, 0, stream));
+                             ext, 0, 0, 0, stream));
     }
     // the control block after the last attempt (fv_settle_kernel), read back
     const int phase = (int)(a % 6);

@@ -425,6 +425,116 @@ __device__ __forceinline__ Ctl current(const InstDesc& D, int phase, bool log) {
   return D.fp64 ? current_t<double>(D, phase, log) : current_t<float>(D, phase, log);
 }
 
+// The fold of attempt a-1 as the launch of attempt a (phase) forms it.
+template <typename R>
+__device__ __forceinline__ Fold<R> fold_prev(const InstDesc& D, int phase) {
+  return fold_decide(fold_load<R>(D.ctl + (phase & 1), D.sync + (phase + 2) % 3), D.cfl_max,
+                     D.dt_seq != nullptr);
+}
+
+// Data collection of an attempt (phase, its fold F): if it was accepted, record
+// its new T and its cfl (row 0 and row 1, entry n - 1 - n0frame) and the app's
+// measurement (collect_hifu, collect_taylor) into the instance's measurement
+// grid (data_collect.h of either app).  Thread tid = column.
+template <typename R>
+__device__ void collect_attempt(const InstDesc& D, const Fold<R>& F, int phase, int tid) {
+  typename Mem<R>::g* __restrict__ m = (typename Mem<R>::g*)D.measure;
+  if (m == nullptr || F.state != kFoldAccept) return;
+  const Ctl& P = F.p;
+  const double T = P.T + P.dt;                       // update_T
+  const int nx = D.nx;
+  // While T <= 0 the reference zeroes the whole grid every step and records
+  // nothing (data_collect.h:22-30, both apps).  Here the grid is zeroed when
+  // collection is switched on, and nothing writes it while T <= 0, so it is
+  // already zero: the pass over the grid is skipped.
+  if (T <= 0.0) return;
+  const int64_t nf = P.n_acc - D.n0frame;          // n - 1 - n0frame, n = n_acc + 1
+  if (nf >= nx) {                                   // simError 4
+    if (tid == 0) aadd_relaxed(D.collect_err, 4u);
+    return;
+  }
+  if (tid == 0) {                                   // T and cfl of the step
+    m[nf] = R(T);
+    m[nf + nx] = F.cfl;
+  }
+  if (D.bc == kBcTaylor)
+    fvbc::collect_taylor<R>(D, P, T, (R*)m, tid);
+  else
+    fvbc::collect_hifu<R>(D, P, (const R*)D.stage + (phase & 1) * nx, T, nf, (R*)m, tid);
+}
+
+// Closed-form ghost ring of a Taylor-shock instance (apps/taylor-angle-xy/
+// boundary.h:38-55) at T and window offset (mdx, mdy), into the ring of its
+// buffer b, or its grid.  The values depend on the cell and on T only, never on
+// the state.  Cells k0, k0 + dk, ... of the ring (2 cells wide).
+__device__ __forceinline__ void taylor_ring(const InstDesc& D, double T, int b, int mdx, int mdy,
+                                            bool to_ring, int k0, int dk) {
+  const int nx = D.nx, ny = D.ny;
+  const int ring = 4 * nx + 4 * (ny - 4);
+  for (int k = k0; k < ring; k += dk) {
+    int i, j;
+    if (k < 4 * nx) {            // rows 0, 1, ny-2, ny-1
+      const int rr = k / nx;
+      i = k - rr * nx;
+      j = rr < 2 ? rr : ny - 4 + rr;
+    } else {                     // columns 0, 1, nx-2, nx-1 of rows 2..ny-3
+      const int kk = k - 4 * nx;
+      const int cc = kk / (ny - 4);
+      j = 2 + (kk - cc * (ny - 4));
+      i = cc < 2 ? cc : nx - 4 + cc;
+    }
+    // the closed form is taken at the cell's position in the unmoved frame
+    // (apps/taylor-angle-xy/boundary.h:45-49: i + MDX, j + MDY)
+    const size_t size = D.fp64 ? sizeof(double) : sizeof(float);
+    const size_t o = to_ring ? D.ring + size * (size_t)k
+                             : size * ((size_t)j * (size_t)nx + (size_t)i);
+    if (D.fp64) {
+      fvbc::Cell<double> c;
+      fvbc::Taylor::prepass(D, T, i + mdx, j + mdy, c);
+      *(double*)((char*)D.q[b][0] + o) = c.q1;
+      *(double*)((char*)D.q[b][1] + o) = c.q2;
+      *(double*)((char*)D.q[b][2] + o) = c.q3;
+    } else {
+      fvbc::Cell<float> c;
+      fvbc::Taylor::prepass(D, T, i + mdx, j + mdy, c);
+      *(float*)((char*)D.q[b][0] + o) = c.q1;
+      *(float*)((char*)D.q[b][1] + o) = c.q2;
+      *(float*)((char*)D.q[b][2] + o) = c.q3;
+    }
+  }
+}
+
+// What a step launch does beside the step, in workgroups of its own: the data
+// collection of the attempt before it (collect), whose fold is known now and
+// whose new state is this attempt's input, and the ghost ring of the attempt
+// after it, for the T and window offset that follow if this one is accepted
+// (else the ring this attempt reads stays the right one).  As launches of their
+// own between the steps the two took 4.8 us each.
+// part: the workgroup's place among its instance's `beside`, the first
+// `collect` of them collect.
+template <typename R>
+__device__ __forceinline__ void beside_step(const InstDesc& D, int phase, int part, int beside,
+                                            int collect) {
+  const int threads = kLanes * kGroupWaves;
+  const Fold<R> F = fold_prev<R>(D, phase);
+  if (part < collect) {
+    collect_attempt<R>(D, F, phase + 5, part * threads + (int)threadIdx.x);   // phase - 1 (mod 6)
+    return;
+  }
+  if (D.bc != kBcTaylor || D.ring == 0) return;
+  Ctl P = advance<R>(D, F, false);
+  prescribed_exhausted(D, P);
+  if (P.err != 0 || P.n_acc >= P.target_acc || !(P.T < P.T_stop)) return;
+  const double T = P.T + P.dt;
+  int mdx = P.mdx, mdy = P.mdy;
+  if (D.md_on) {
+    mdx += md_shift(T, D.md_t, D.md_vx, D.dx, P.mdx);
+    mdy += md_shift(T, D.md_t, D.md_vy, D.dy, P.mdy);
+  }
+  taylor_ring(D, T, P.cur ^ 1, mdx, mdy, true, (part - collect) * threads + (int)threadIdx.x,
+              (beside - collect) * threads);
+}
+
 template <typename R>
 struct Row {         // one cell of a row as the y sweep sees it
   R q1, q2, q3;      // rho', rho u, rho v
@@ -541,10 +651,11 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
   const uint64_t* __restrict__ cm = rowmask + (it.mrow - y0);
 
   // the lane's ghost-cell source columns (the app's boundary policy; Taylor
-  // ghost cells were written into the input by fv_taylor_ghost_kernel and are
-  // plain copies here)
+  // ghost cells are copies of the buffer's ghost ring, or of the grid)
   constexpr uint32_t kSz = sizeof(R);
   fvbc::LaneMap lm;
+  lm.ring = D.ring;
+  lm.ny = ny;
   BC::lane(ic, nx, lm, kSz);
   const uint32_t row_bytes = kSz * (uint32_t)nx;
 
@@ -553,7 +664,7 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
   // so the load latency overlaps a full step
   auto load_raw = [&](int r, R& a, R& b, R& c, uint64_t& k, fvbc::RowData<R>& h) {
     const int rc = min(max(r, 0), ny - 1);
-    const uint32_t o = BC::offset(rc, ny, lm, row_bytes);
+    const uint32_t o = BC::offset(rc, ny, lm, row_bytes, kSz);
     a = ldg(in1, o);
     b = ldg(in2, o);
     c = ldg(in3, o);
@@ -600,8 +711,8 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
     sx = uni(md_shift(Tn, D.md_t, D.md_vx, D.dx, P.mdx));
     sy = uni(md_shift(Tn, D.md_t, D.md_vy, D.dy, P.mdy));
   }
-  typename Mem<R>::g* __restrict__ stage = (typename Mem<R>::g*)D.stage;
-  const bool stage_on = kExt && stage != nullptr;
+  const bool stage_on = kExt && D.stage != nullptr;
+  typename Mem<R>::g* __restrict__ stage = (typename Mem<R>::g*)((R*)D.stage + (phase & 1) * nx);
   // adjoint forward runs that keep every state: this attempt's output also
   // goes to history slot n_acc + 1 - log_base, the slot of the count it
   // makes if accepted.  A rejected attempt's copy is overwritten by the
@@ -935,12 +1046,22 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
 struct AnyApp {};
 
 // The step kernel: one wave per work item, kGroupWaves items per workgroup
-// (items[4 g .. 4 g + 3]; an unused slot has no rows).
+// (items[4 g .. 4 g + 3]; an unused slot has no rows); then `beside` workgroups
+// per instance for beside_step.
 template <typename R, bool kOne, bool kExt, class BC>
 __global__ __launch_bounds__(kLanes * kGroupWaves) void fv_step_kernel(
     const InstDesc* __restrict__ insts, const WorkItem* __restrict__ items,
     const uint64_t* __restrict__ rowmask, int n_groups, int phase,
-    const Ctl* __restrict__ ctl_in, const SyncSlots* __restrict__ sync_in) {
+    const Ctl* __restrict__ ctl_in, const SyncSlots* __restrict__ sync_in, int beside,
+    int collect) {
+  // (the plain kernels of the other apps have nothing beside the step)
+  constexpr bool kBeside = kExt || std::is_same<BC, AnyApp>::value ||
+                           std::is_same<BC, fvbc::Taylor>::value;
+  if (kBeside && (int)blockIdx.x >= n_groups) {
+    const int e = blockIdx.x - n_groups, inst = uni(e / beside);
+    beside_step<R>(insts[inst], phase, e - inst * beside, beside, collect);
+    return;
+  }
   __shared__ R seam[kGroupWaves][kSeamFields][kLanes];
   // XCD-aware order: workgroup b runs on XCD b % 8; give each XCD a contiguous
   // run of groups so vertically adjacent groups of a strip (which share
@@ -1002,111 +1123,69 @@ __global__ __launch_bounds__(64) void fv_targets_kernel(const InstDesc* __restri
   }
 }
 
-// Data collection of attempt a, run after its step launch: if the attempt
-// was accepted, record its new T and its cfl (row 0 and row 1, entry
-// n - 1 - n0frame) and the app's measurement (collect_hifu, collect_taylor)
-// into the instance's measurement grid (data_collect.h of either app).
-// blockIdx.y = instance; threads cover the columns.
-template <typename R>
+// Data collection of the attempt of phase `phase` alone, run after its launch
+// (the last attempt of a run of launches; the others' comes with the launch
+// after them, ahead_of_step).  blockIdx.y = instance; threads cover the columns.
 __global__ __launch_bounds__(256) void fv_collect_kernel(const InstDesc* __restrict__ insts,
                                                          int phase) {
   const InstDesc& D = insts[blockIdx.y];
-  typename Mem<R>::g* __restrict__ m = (typename Mem<R>::g*)D.measure;
-  if (m == nullptr) return;
-  // attempt a's control block (its step launch published it) and slots
-  const Fold<R> F = fold_decide(fold_load<R>(D.ctl + ((phase + 1) & 1), D.sync + phase % 3),
-                                D.cfl_max, D.dt_seq != nullptr);
-  if (F.state != kFoldAccept) return;
-  const Ctl& P = F.p;
-  const double T = P.T + P.dt;                       // update_T
-  const int nx = D.nx;
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  // While T <= 0 the reference zeroes the whole grid every step and records
-  // nothing (data_collect.h:22-30, both apps).  Here the grid is zeroed when
-  // collection is switched on, and nothing writes it while T <= 0, so it is
-  // already zero: the pass over the grid is skipped.
-  if (T <= 0.0) return;
-  const int64_t nf = P.n_acc - D.n0frame;          // n - 1 - n0frame, n = n_acc + 1
-  if (nf >= nx) {                                   // simError 4
-    if (tid == 0) aadd_relaxed(D.collect_err, 4u);
-    return;
-  }
-  if (tid == 0) {                                   // T and cfl of the step
-    m[nf] = R(T);
-    m[nf + nx] = F.cfl;
-  }
-  if (D.bc == kBcTaylor)
-    fvbc::collect_taylor<R>(D, P, T, (R*)m, tid);
+  if (D.fp64)
+    collect_attempt<double>(D, fold_prev<double>(D, phase + 1), phase, tid);
   else
-    fvbc::collect_hifu<R>(D, P, T, nf, (R*)m, tid);
+    collect_attempt<float>(D, fold_prev<float>(D, phase + 1), phase, tid);
 }
 
-// Closed-form ghost ring of the Taylor-shock instances (apps/taylor-angle-xy/
-// boundary.h:38-55), written into the current input buffer before the step
-// reads it.  The values depend on the cell and on T only, never on the state,
-// so writing them in place is the reference's boundary kernel.  blockIdx.y =
-// instance; the ring (2 cells wide) is enumerated by a flat index.
+// Ghost ring of the Taylor-shock instances for the attempt of phase `phase`
+// (the first attempt of a run of launches, or every one where a buffer has no
+// ring: then into the grid).  settle: instead, after that phase's last attempt:
+// where it was not accepted, the grid's ghost cells take the values it read, as
+// if they had been written there.  blockIdx.y = instance; the ring is
+// enumerated by a flat index.
 __global__ __launch_bounds__(256) void fv_taylor_ghost_kernel(const InstDesc* __restrict__ insts,
-                                                             int phase) {
+                                                             int phase, int settle) {
   const InstDesc& D = insts[blockIdx.y];
   if (D.bc != kBcTaylor) return;
+  const int k0 = blockIdx.x * blockDim.x + threadIdx.x, dk = gridDim.x * blockDim.x;
+  if (settle) {
+    if (D.ring == 0) return;
+    int state;
+    Ctl P;
+    if (D.fp64) {
+      const Fold<double> F = fold_prev<double>(D, phase);
+      state = F.state;
+      P = F.p;
+    } else {
+      const Fold<float> F = fold_prev<float>(D, phase);
+      state = F.state;
+      P = F.p;
+    }
+    if (state == kFoldReject || state == kFoldError)
+      taylor_ring(D, P.T, P.cur, P.mdx, P.mdy, false, k0, dk);
+    return;
+  }
   const Ctl P = current(D, phase, false);
   if (P.err != 0 || P.n_acc >= P.target_acc || !(P.T < P.T_stop)) return;
-  const int nx = D.nx, ny = D.ny;
-  const int ring = 4 * nx + 4 * (ny - 4);
-  const double T = P.T;
-  const int cur = P.cur;
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < ring; k += gridDim.x * blockDim.x) {
-    int i, j;
-    if (k < 4 * nx) {            // rows 0, 1, ny-2, ny-1
-      const int rr = k / nx;
-      i = k - rr * nx;
-      j = rr < 2 ? rr : ny - 4 + rr;
-    } else {                     // columns 0, 1, nx-2, nx-1 of rows 2..ny-3
-      const int kk = k - 4 * nx;
-      const int cc = kk / (ny - 4);
-      j = 2 + (kk - cc * (ny - 4));
-      i = cc < 2 ? cc : nx - 4 + cc;
-    }
-    // the closed form is taken at the cell's position in the unmoved frame
-    // (apps/taylor-angle-xy/boundary.h:45-49: i + MDX, j + MDY)
-    const size_t o = (size_t)j * (size_t)nx + (size_t)i;
-    if (D.fp64) {
-      fvbc::Cell<double> c;
-      fvbc::Taylor::prepass(D, T, i + P.mdx, j + P.mdy, c);
-      ((double*)D.q[cur][0])[o] = c.q1;
-      ((double*)D.q[cur][1])[o] = c.q2;
-      ((double*)D.q[cur][2])[o] = c.q3;
-    } else {
-      fvbc::Cell<float> c;
-      fvbc::Taylor::prepass(D, T, i + P.mdx, j + P.mdy, c);
-      D.q[cur][0][o] = c.q1;
-      D.q[cur][1][o] = c.q2;
-      D.q[cur][2][o] = c.q3;
-    }
-  }
+  taylor_ring(D, P.T, P.cur, P.mdx, P.mdy, D.ring != 0, k0, dk);
 }
 
 }  // namespace fv
 
 extern "C" hipError_t fv_launch_taylor_ghosts(const fv::InstDesc* insts, int n_inst,
-                                              int max_ring, int phase, hipStream_t stream) {
+                                              int max_ring, int phase, int settle,
+                                              hipStream_t stream) {
   if (n_inst <= 0) return hipSuccess;
   const int blocks = (max_ring + 255) / 256;
   hipLaunchKernelGGL(fv::fv_taylor_ghost_kernel, dim3(blocks, n_inst), dim3(256), 0, stream,
-                     insts, phase);
+                     insts, phase, settle);
   return hipGetLastError();
 }
 
 extern "C" hipError_t fv_launch_collect(const fv::InstDesc* insts, int n_inst, int max_nx,
-                                        int phase, int fp64, hipStream_t stream) {
+                                        int phase, hipStream_t stream) {
   if (n_inst <= 0) return hipSuccess;
-  if (fp64)
-    hipLaunchKernelGGL(fv::fv_collect_kernel<double>, dim3((max_nx + 255) / 256, n_inst),
-                       dim3(256), 0, stream, insts, phase);
-  else
-    hipLaunchKernelGGL(fv::fv_collect_kernel<float>, dim3((max_nx + 255) / 256, n_inst),
-                       dim3(256), 0, stream, insts, phase);
+  hipLaunchKernelGGL(fv::fv_collect_kernel, dim3((max_nx + 255) / 256, n_inst), dim3(256), 0,
+                     stream, insts, phase);
   return hipGetLastError();
 }
 
@@ -1148,25 +1227,30 @@ extern "C" hipError_t fv_step_waves_per_cu(int* waves, int fp64) {
 }
 
 namespace {
+// the workgroups for beside_step: parts per instance
+struct Beside {
+  int n_inst, parts, collect;
+};
 template <typename R, bool kOne, bool kExt, class BC>
 void launch_step_t(const fv::InstDesc* insts, const fv::WorkItem* items, const uint64_t* rowmask,
                    int n_groups, int phase, const fv::Ctl* c_in, const fv::SyncSlots* s_in,
-                   hipStream_t stream) {
-  hipLaunchKernelGGL((fv::fv_step_kernel<R, kOne, kExt, BC>), dim3(n_groups),
-                     dim3(fv::kLanes * fv::kGroupWaves), 0, stream, insts, items, rowmask,
-                     n_groups, phase, c_in, s_in);
+                   const Beside& bs, hipStream_t stream) {
+  hipLaunchKernelGGL((fv::fv_step_kernel<R, kOne, kExt, BC>),
+                     dim3(n_groups + bs.n_inst * bs.parts), dim3(fv::kLanes * fv::kGroupWaves), 0,
+                     stream, insts, items, rowmask, n_groups, phase, c_in, s_in, bs.parts,
+                     bs.collect);
 }
 // a single instance: its app's own kernel (bc), else the dispatching one
 template <typename R, bool kExt>
 void launch_one(int bc, const fv::InstDesc* insts, const fv::WorkItem* items,
                 const uint64_t* rowmask, int n_groups, int phase, const fv::Ctl* c_in,
-                const fv::SyncSlots* s_in, hipStream_t stream) {
+                const fv::SyncSlots* s_in, const Beside& bs, hipStream_t stream) {
   switch (bc) {
 #define FV_APP_LAUNCH(P)                                                                 \
   case P::kId:                                                                           \
     if constexpr (kExt || !P::kExtOnly) {                                                \
       launch_step_t<R, true, kExt, P>(insts, items, rowmask, n_groups, phase, c_in, s_in, \
-                                      stream);                                           \
+                                      bs, stream);                                           \
       return;                                                                            \
     }                                                                                    \
     break;
@@ -1176,42 +1260,46 @@ void launch_one(int bc, const fv::InstDesc* insts, const fv::WorkItem* items,
       break;
   }
   launch_step_t<R, true, kExt, fv::AnyApp>(insts, items, rowmask, n_groups, phase, c_in, s_in,
-                                           stream);
+                                           bs, stream);
 }
 template <typename R>
 void launch_step_r(bool one, bool ext, int bc, const fv::InstDesc* insts,
                    const fv::WorkItem* items, const uint64_t* rowmask, int n_groups, int phase,
-                   const fv::Ctl* c_in, const fv::SyncSlots* s_in, hipStream_t stream) {
+                   const fv::Ctl* c_in, const fv::SyncSlots* s_in, const Beside& bs,
+                   hipStream_t stream) {
   if (one && !ext)
-    launch_one<R, false>(bc, insts, items, rowmask, n_groups, phase, c_in, s_in, stream);
+    launch_one<R, false>(bc, insts, items, rowmask, n_groups, phase, c_in, s_in, bs, stream);
   else if (one)
-    launch_one<R, true>(bc, insts, items, rowmask, n_groups, phase, c_in, s_in, stream);
+    launch_one<R, true>(bc, insts, items, rowmask, n_groups, phase, c_in, s_in, bs, stream);
   else if (!ext)
     launch_step_t<R, false, false, fv::AnyApp>(insts, items, rowmask, n_groups, phase, c_in, s_in,
-                                               stream);
+                                               bs, stream);
   else
     launch_step_t<R, false, true, fv::AnyApp>(insts, items, rowmask, n_groups, phase, c_in, s_in,
-                                              stream);
+                                              bs, stream);
 }
 }  // namespace
 
 // One step attempt of every instance: n_groups workgroups, items[4 g ..] each.  ctl0/sync0: the control blocks and
 // slot sets of the only instance when n_inst == 1 (null otherwise), bc0 its
 // boundary kind; ext: some instance has a moving window, the HIFU boundary or
-// data collection; fp64: the instances are FP64.
+// data collection; fp64: the instances are FP64; beside, collect: workgroups per
+// instance for beside_step, and how many of them collect the attempt before.
 extern "C" hipError_t fv_launch_step(const fv::InstDesc* insts, const fv::WorkItem* items,
                                      const uint64_t* rowmask, int n_groups, int phase,
                                      int n_inst, fv::Ctl* ctl0, fv::SyncSlots* sync0, int bc0,
-                                     int ext, int fp64, hipStream_t stream) {
+                                     int ext, int fp64, int beside, int collect,
+                                     hipStream_t stream) {
   if (n_groups <= 0) return hipSuccess;
   const bool one = n_inst == 1 && ctl0 && sync0;
   const fv::Ctl* c_in = one ? ctl0 + (phase & 1) : nullptr;
   const fv::SyncSlots* s_in = one ? sync0 + (phase + 2) % 3 : nullptr;
+  const Beside bs{n_inst, beside, collect};
   if (fp64)
     launch_step_r<double>(one, ext != 0, bc0, insts, items, rowmask, n_groups, phase, c_in, s_in,
-                          stream);
+                          bs, stream);
   else
     launch_step_r<float>(one, ext != 0, bc0, insts, items, rowmask, n_groups, phase, c_in, s_in,
-                         stream);
+                         bs, stream);
   return hipGetLastError();
 }

@@ -81,7 +81,12 @@ struct InstDesc {
   int32_t tay_jc;
   int32_t md_on;        // moving window (common/main.cu:109-177)
   float beta2m2;        // 2*(BETA - 1)
-  float pad;
+  // Taylor instances: byte offset, from the start of each field of a state
+  // buffer, of that buffer's ghost ring (rows 0, 1, ny-2, ny-1, then columns 0,
+  // 1, nx-2, nx-1 of the rows between): the closed form at the state's T, which
+  // the step reads in place of the grid's ghost cells.  0: none, the ghost
+  // cells are written into the grid before each attempt
+  uint32_t ring;
   double md_vx, md_vy, md_t;   // MDVX, MDVY, MDT
   // kBcHifu: edge_c/edge_s hold AMPL cos/sin(ISPW phi_j); per row j,
   // hifu_tab[4j..4j+3] = phi_j, nu_x, nu_y, 1 on aperture rows (0 elsewhere)
@@ -89,8 +94,9 @@ struct InstDesc {
   float hifu_k;         // FREC/4: envelope argument per unit of T + phi
   int32_t jcut;         // data collection: row (JCUT)
   // data collection (apps/hifu-beam/data_collect.h, apps/taylor-angle-xy/
-  // data_collect.h): measure = nx*ny grid (null: off), stage = row jcut of
-  // the last attempt before the window shift (hifu); float or double (fp64)
+  // data_collect.h): measure = nx*ny grid (null: off), stage = row jcut of an
+  // attempt's state before the window shift (hifu; two rows of nx, by the
+  // attempt's parity); float or double (fp64)
   void* measure;
   void* stage;
   uint32_t* collect_err;  // 4 once a frame holds more than nx steps
