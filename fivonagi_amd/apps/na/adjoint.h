@@ -20,6 +20,8 @@
 //   r_p = W_p . W_p(upwind) / |W_p|^2, h_p = clamp(min((1 + r_p)/4, r_p), 0, 1)
 //   c_p = |L_p| (1 - |L_p| dt/d) h_p, al_p = max(L_p, 0) - c_p, be_p = L_p - al_p
 //   P = sum_p al_p W_p, M = sum_p be_p W_p
+// Every multiply-add is written out and contraction is off in these bodies:
+// the kernel holds several copies of its row, and they must round alike.
 // The derivatives are those of that branch path with dt frozen; a limiter
 // ratio at a clamp (h = 0 or 1) or of a zero wave has derivative 0.
 #ifndef FIVONAGI_APPS_NA_ADJOINT_H
@@ -34,23 +36,17 @@ namespace fvad {
 using fvna::Iface;
 using fvna::Waves;
 
-// What the limiter's transpose needs of one interface, per wave family:
-// h = phi/2, qd = (dh/dr) / |W|^2 and r (both 0 where h is clamped or the
-// wave is zero, so no infinity or NaN of the forward enters a product).
+// What the limiter's transpose needs of one interface, per wave family, formed
+// with the forward values rather than from them a second time: with g2 the
+// adjoint of al - be,
+//   adjoint of the dot product with the upwind neighbour  g2 kd
+//   adjoint of the speed, beside be's                     g2 ks
+//   twice the adjoint of |W|^2                            g2 kn
+// kd and kn are 0 where h is clamped or the wave is zero, so no infinity or
+// NaN of the forward enters a product.
 struct LimT {
-  float h[3], qd[3], r[3];
+  float al[3], kd[3], ks[3], kn[3];
 };
-
-__device__ __forceinline__ void lim_part(float n, float dot, float& h, float& qd, float& r) {
-  const float rn = fvna::rcp(n);
-  const float rr = dot * rn;
-  const float t = fvna::fma_(0.25f, rr, 0.25f);
-  const float mn = fvna::min_(t, rr);
-  h = fvna::clamp01(mn);
-  const bool live = mn > 0.0f && mn < 1.0f;
-  qd = live ? (rr < t ? rn : 0.25f * rn) : 0.0f;
-  r = live ? rr : 0.0f;
-}
 
 // The limited fluxes of interface f as the step kernel forms them (same
 // call), and the transpose's quantities.  dl_p = W_p . W_p(k-1),
@@ -59,16 +55,24 @@ template <bool kL3Product>
 __device__ __forceinline__ void limiter_rec(const Iface& f, float dl1, float dr1, float dl2,
                                             float dr2, float dl3, float dr3, float dtd,
                                             float P[3], float M[3], LimT& t) {
+#pragma clang fp contract(off)
   const float up1 = fvna::upwind(f.L1, dl1, dr1), up2 = fvna::upwind(f.L2, dl2, dr2);
   const float up3 = fvna::upwind(f.L3, dl3, dr3);
-  fvna::limited_flux<kL3Product>(f, up1, up2, up3, dtd, P, M);
-  const Waves& w = f.w;
-  const float n1 = fvna::fma_(w.a1, w.a1, fvna::fma_(w.w21, w.w21, w.w31 * w.w31));
-  const float n2 = fvna::fma_(w.a2, w.a2, fvna::fma_(w.w22, w.w22, w.w32 * w.w32));
-  const float n3 = w.a3 * w.a3;
-  lim_part(n1, up1, t.h[0], t.qd[0], t.r[0]);
-  lim_part(n2, up2, t.h[1], t.qd[1], t.r[1]);
-  lim_part(n3, up3, t.h[2], t.qd[2], t.r[2]);
+  fvna::LimitT<float> v;
+  fvna::limited_flux<kL3Product>(f, up1, up2, up3, dtd, P, M, v);
+  const float L[3] = {f.L1, f.L2, f.L3};
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    // al = max(L, 0) - c, be = L - al, c = g h, g = s om, om = 1 - s dt/d,
+    // s = |L|, h = min(t, r) where it is not clamped, r = dot / |W|^2
+    t.al[p] = v.al[p];
+    const bool live = v.mn[p] > 0.0f && v.mn[p] < 1.0f;
+    const float qd = v.r[p] < v.t[p] ? v.rn[p] : 0.25f * v.rn[p];   // dh/ddot
+    t.kd[p] = live ? -v.g[p] * qd : 0.0f;
+    t.kn[p] = -2.0f * t.kd[p] * (live ? v.r[p] : 0.0f);
+    const float e = v.h[p] * fvna::fma_(2.0f, v.om[p], -1.0f);      // dc/ds
+    t.ks[p] = L[p] > 0.0f ? 1.0f - e : (L[p] < 0.0f ? e : 0.0f);
+  }
 }
 
 // Adjoint of one interface's waves (a1, w21, w31, a2, w22, w32, a3) and
@@ -90,45 +94,37 @@ __device__ __forceinline__ void zero(WaveAdj& a) {
 // Transpose of limiter_rec: from the adjoints gP, gM of the interface's P
 // and M (component order of the sweep), accumulate the adjoint of its own
 // waves and speeds into ga and return the adjoint of each family's dot
-// product with its upwind neighbour (gd).
-__device__ __forceinline__ void limiter_bw(const Iface& f, const LimT& t, float dtd,
-                                           const float gP[3], const float gM[3], WaveAdj& ga,
-                                           float gd[3]) {
+// product with its upwind neighbour (gd).  With be = L - al only
+// D = gP - gM meets al: sum_p (al_p gP + be_p gM) . W_p =
+// sum_p (al_p D + L_p gM) . W_p.
+__device__ __forceinline__ void limiter_bw(const Iface& f, const LimT& t, const float gP[3],
+                                           const float gM[3], WaveAdj& ga, float gd[3]) {
+#pragma clang fp contract(off)
   const Waves& w = f.w;
-  const float L[3] = {f.L1, f.L2, f.L3};
-  float gal[3], gbe[3];
-  gal[0] = fvna::fma_(gP[0], w.a1, fvna::fma_(gP[1], w.w21, gP[2] * w.w31));
-  gbe[0] = fvna::fma_(gM[0], w.a1, fvna::fma_(gM[1], w.w21, gM[2] * w.w31));
-  gal[1] = fvna::fma_(gP[0], w.a2, fvna::fma_(gP[1], w.w22, gP[2] * w.w32));
-  gbe[1] = fvna::fma_(gM[0], w.a2, fvna::fma_(gM[1], w.w22, gM[2] * w.w32));
-  gal[2] = gP[2] * w.a3;
-  gbe[2] = gM[2] * w.a3;
-  float al[3], be[3], gn2[3];
+  const float D[3] = {gP[0] - gM[0], gP[1] - gM[1], gP[2] - gM[2]};
+  const float g2[3] = {fvna::fma_(D[0], w.a1, fvna::fma_(D[1], w.w21, D[2] * w.w31)),
+                       fvna::fma_(D[0], w.a2, fvna::fma_(D[1], w.w22, D[2] * w.w32)),
+                       D[2] * w.a3};
+  ga.gs[0] = fvna::fma_(gM[0], w.a1, fvna::fma_(gM[1], w.w21, fvna::fma_(gM[2], w.w31, ga.gs[0])));
+  ga.gs[1] = fvna::fma_(gM[0], w.a2, fvna::fma_(gM[1], w.w22, fvna::fma_(gM[2], w.w32, ga.gs[1])));
+  ga.gs[2] = fvna::fma_(gM[2], w.a3, ga.gs[2]);
+  float gn[3];
 #pragma unroll
   for (int p = 0; p < 3; ++p) {
-    const float s = fabsf(L[p]);
-    const float om = fvna::fma_(-s, dtd, 1.0f);        // 1 - |L| dt/d
-    const float c = s * om * t.h[p];
-    al[p] = fvna::fmax2(L[p], 0.0f) - c;
-    be[p] = L[p] - al[p];
-    // be = L - al; al = max(L, 0) - c; c = s (1 - s dt/d) h
-    const float g2 = gal[p] - gbe[p];                  // adjoint of al, be's share folded
-    const float gc = -g2;
-    const float gh = gc * s * om;
-    const float gsa = gc * t.h[p] * fvna::fma_(-2.0f * s, dtd, 1.0f);
-    float gl = gbe[p] + (L[p] > 0.0f ? g2 : 0.0f);
-    gl += L[p] > 0.0f ? gsa : (L[p] < 0.0f ? -gsa : 0.0f);
-    ga.gs[p] += gl;
-    gd[p] = gh * t.qd[p];                              // h(r), r = dot / |W|^2
-    gn2[p] = -2.0f * gd[p] * t.r[p];                   // 2 x adjoint of |W|^2
+    ga.gs[p] = fvna::fma_(g2[p], t.ks[p], ga.gs[p]);
+    gd[p] = g2[p] * t.kd[p];
+    gn[p] = g2[p] * t.kn[p];
   }
-  ga.g[0] += fvna::fma_(al[0], gP[0], fvna::fma_(be[0], gM[0], gn2[0] * w.a1));
-  ga.g[1] += fvna::fma_(al[0], gP[1], fvna::fma_(be[0], gM[1], gn2[0] * w.w21));
-  ga.g[2] += fvna::fma_(al[0], gP[2], fvna::fma_(be[0], gM[2], gn2[0] * w.w31));
-  ga.g[3] += fvna::fma_(al[1], gP[0], fvna::fma_(be[1], gM[0], gn2[1] * w.a2));
-  ga.g[4] += fvna::fma_(al[1], gP[1], fvna::fma_(be[1], gM[1], gn2[1] * w.w22));
-  ga.g[5] += fvna::fma_(al[1], gP[2], fvna::fma_(be[1], gM[2], gn2[1] * w.w32));
-  ga.g[6] += fvna::fma_(al[2], gP[2], fvna::fma_(be[2], gM[2], gn2[2] * w.a3));
+  auto add = [&](int c, float al, float L, float gn2, int k, float wk) {
+    ga.g[c] = fvna::fma_(al, D[k], fvna::fma_(L, gM[k], fvna::fma_(gn2, wk, ga.g[c])));
+  };
+  add(0, t.al[0], f.L1, gn[0], 0, w.a1);
+  add(1, t.al[0], f.L1, gn[0], 1, w.w21);
+  add(2, t.al[0], f.L1, gn[0], 2, w.w31);
+  add(3, t.al[1], f.L2, gn[1], 0, w.a2);
+  add(4, t.al[1], f.L2, gn[1], 1, w.w22);
+  add(5, t.al[1], f.L2, gn[1], 2, w.w32);
+  add(6, t.al[2], f.L3, gn[2], 2, w.a3);
 }
 
 // ga += the dot-product adjoints of the families of a neighbouring
@@ -151,20 +147,37 @@ struct SumAdj {
   float s1, s2, s3, dr, dn, dt;
 };
 
+// The values riemann_bw needs of an interface whose solve is rows back (only
+// its waves and speeds are kept): formed again, with the square root from
+// L1 - L2 = 2 sq.
+__device__ __forceinline__ fvna::SolveT<float> solve_again(float s1, float s2, float s3,
+                                                           const Iface& f) {
+#pragma clang fp contract(off)
+  fvna::SolveT<float> v;
+  const float S1 = s1 + 2.0f;
+  v.rS = fvna::rcp(S1);
+  v.rs = 2.0f * fvna::rcp(f.L1 - f.L2);
+  v.d1 = fvna::fma_(f.L1, S1, -s3);
+  v.d2 = fvna::fma_(f.L2, S1, -s3);
+  v.rdd = fvna::rcp(v.d1 * v.d2);
+  const float srd = s3 * v.rdd;
+  v.A1 = (f.L1 - s2) * (v.d2 * srd);
+  v.A2 = (f.L2 - s2) * (v.d1 * srd);
+  return v;
+}
+
 // Transpose of solver.h riemann at one interface, from the adjoint of its
-// waves and speeds (ga).  s1..dn as the forward forms them; f its result.
+// waves and speeds (ga).  s1..dn as the forward forms them; f, v its result.
 __device__ __forceinline__ SumAdj riemann_bw(float s1, float s2, float s3, float drho, float dn,
-                                             float hbeta, const Iface& f, const WaveAdj& ga) {
+                                             float hbeta, const Iface& f,
+                                             const fvna::SolveT<float>& v, const WaveAdj& ga) {
+#pragma clang fp contract(off)
   const float L1 = f.L1, L2 = f.L2, tmp1 = f.L3;
   const float a1 = f.w.a1, a2 = f.w.a2;
   const float S1 = s1 + 2.0f;
-  const float rS = fvna::rcp(S1);
-  const float tmp3 = fvna::fma_(tmp1, tmp1 - s2, fvna::fma_(hbeta, s1, 1.0f));
-  const float hrs = 0.5f * fvna::rsq(tmp3);             // 1 / (2 sq) = 1 / (L1 - L2)
-  const float d1 = fvna::fma_(L1, S1, -s3), d2 = fvna::fma_(L2, S1, -s3);
-  const float rdd = fvna::rcp(d1 * d2);
-  const float id1 = d2 * rdd, id2 = d1 * rdd;           // 1/d1, 1/d2
-  const float A1 = s3 * (L1 - s2) * id1, A2 = s3 * (L2 - s2) * id2;
+  const float rS = v.rS, hrs = 0.5f * v.rs;             // hrs = 1 / (2 sq)
+  const float id1 = v.d2 * v.rdd, id2 = v.d1 * v.rdd;   // 1/d1, 1/d2
+  const float A1 = v.A1, A2 = v.A2;
   SumAdj o;
   // a3 = dtg - (a1 A1 + a2 A2), w21 = a1 L1, w31 = a1 A1, w22 = a2 L2, w32 = a2 A2
   const float ga3 = ga.g[6];
@@ -183,7 +196,6 @@ __device__ __forceinline__ SumAdj riemann_bw(float s1, float s2, float s3, float
   o.dn = t1;
   gdr = fvna::fma_(-t1, L2, gdr);
   gL2 = fvna::fma_(-t1, drho, gL2);
-  float gsq = -2.0f * t1 * a1;
   // A_p = s3 (L_p - s2) / d_p, d_p = L_p S1 - s3
   const float e1 = gA1 * id1, e2 = gA2 * id2;
   gL1 = fvna::fma_(e1, fvna::fma_(-A1, S1, s3), gL1);
@@ -193,16 +205,16 @@ __device__ __forceinline__ SumAdj riemann_bw(float s1, float s2, float s3, float
   float gS1 = -fvna::fma_(e1 * A1, L1, e2 * A2 * L2);
   // L1,2 = tmp1 +- sq, L3 = tmp1; sq = sqrt(tmp3)
   float gt1 = gL1 + gL2 + ga.gs[2];
-  gsq += gL1 - gL2;
+  const float gsq = fvna::fma_(-2.0f * t1, a1, gL1 - gL2);
   const float gt3 = gsq * hrs;
   // tmp3 = tmp1 (tmp1 - s2) + hbeta s1 + 1
-  gt1 = fvna::fma_(gt3, 2.0f * tmp1 - s2, gt1);
+  gt1 = fvna::fma_(gt3, fvna::fma_(2.0f, tmp1, -s2), gt1);
   gs2 = fvna::fma_(-gt3, tmp1, gs2);
-  float gs1 = gt3 * hbeta;
   // tmp1 = s2 / S1, S1 = s1 + 2
-  gs2 = fvna::fma_(gt1, rS, gs2);
-  gS1 = fvna::fma_(-gt1 * tmp1, rS, gS1);
-  gs1 += gS1;
+  const float gtS = gt1 * rS;
+  gs2 += gtS;
+  gS1 = fvna::fma_(-gtS, tmp1, gS1);
+  const float gs1 = fvna::fma_(gt3, hbeta, gS1);
   o.s1 = gs1;
   o.s2 = gs2;
   o.dr = gdr;

@@ -124,11 +124,19 @@ __device__ __forceinline__ JumpT<R> jump(R r1L, R nL, R tL, R unL, R utL, R r1R,
   return JumpT<R>{r1L + r1R, unL + unR, utL + utR, r1R - r1L, nR - nL, tR - tL};
 }
 
+// Intermediate values of a Riemann solve that its transpose needs again.
+template <typename R>
+struct SolveT {
+  R rS, rs;             // 1 / (2 Z1), 1 / sqrt(tmp3)
+  R d1, d2, rdd;        // L_p S1 - s3, 1 / (d1 d2)
+  R A1, A2;
+};
+
 // Riemann solve at an interface.  hbeta = BETA - 1.  The fluctuations
 // amdq/apdq (fv.h:141-180) are not formed here: limited_flux() folds them with
 // the correction flux.
 template <typename R>
-__device__ __forceinline__ void riemann(const JumpT<R>& j, R hbeta, IfaceT<R>& f) {
+__device__ __forceinline__ void riemann(const JumpT<R>& j, R hbeta, IfaceT<R>& f, SolveT<R>& v) {
 #pragma clang fp contract(off)
   const R s1 = j.s1, s2 = j.s2, s3 = j.s3, drho = j.drho, dn = j.dn, dtg = j.dtg;
   const R S1 = s1 + R(2);                           // 2 Z1
@@ -144,7 +152,8 @@ __device__ __forceinline__ void riemann(const JumpT<R>& j, R hbeta, IfaceT<R>& f
   // fv.h:110-113: A_p = (L_p Z3 - 2 Z2 Z3)/(L_p Z1 - Z3) = s3 (L_p - s2)/(L_p S1 - s3),
   // with one reciprocal for both denominators (each is ~ +-2)
   const R d1 = fma_(L1, S1, -s3), d2 = fma_(L2, S1, -s3);
-  const R srd = s3 * rcp(d1 * d2);
+  const R rdd = rcp(d1 * d2);
+  const R srd = s3 * rdd;
   const R A1 = (L1 - s2) * (d2 * srd);
   const R A2 = (L2 - s2) * (d1 * srd);
   const R hrs = R(0.5) * rs, dnl = fma_(-drho, L2, dn);
@@ -153,19 +162,12 @@ __device__ __forceinline__ void riemann(const JumpT<R>& j, R hbeta, IfaceT<R>& f
   f.w.a1 = a1; f.w.w21 = a1 * L1; f.w.w31 = a1 * A1;
   f.w.a2 = a2; f.w.w22 = a2 * L2; f.w.w32 = a2 * A2;
   f.w.a3 = dtg - fma_(a1, A1, f.w.w32);                         // fv.h:119-125
+  v = SolveT<R>{rS, rs, d1, d2, rdd, A1, A2};
 }
-
-// MC limiter phi(r) = max(0, min((1+r)/2, 2, 2r)) (fv.h:587-605), returned
-// halved: phi/2 = clamp(min((1+r)/4, r), 0, 1), where the clamp is the VOP3
-// output modifier of the min.  The reference sets phi = 1 where wnorm2 == 0;
-// such a wave is the zero vector, so its correction phi*W is 0 for any
-// finite phi.  Here wnorm2 == 0 gives r = NaN (0 * inf), which the clamp
-// turns into 0 (finite), and the select is skipped.
 template <typename R>
-__device__ __forceinline__ R philim_half(R wnorm2, R dot) {
-#pragma clang fp contract(off)
-  const R r = dot * rcp(wnorm2);
-  return clamp01(min_(fma_(R(0.25), r, R(0.25)), r));
+__device__ __forceinline__ void riemann(const JumpT<R>& j, R hbeta, IfaceT<R>& f) {
+  SolveT<R> v;
+  riemann(j, hbeta, f, v);
 }
 
 // W_p(a) . W_p(b); b is the operand that may come from a neighbouring lane
@@ -192,32 +194,49 @@ __device__ __forceinline__ R upwind(R s, R dotl, R dotr) {
 // interface, folded into what the two adjacent cells need:
 //   P = apdq - fadd = sum_p (max(s_p,0) - c_p) W_p   (cell on the + side)
 //   M = amdq + fadd = sum_p (min(s_p,0) + c_p) W_p   (cell on the - side)
-// with c_p = |s_p| (1 - |s_p| dt/d) phi_p / 2 = |s_p| (1 - |s_p| dt/d) philim_half.  A wave with s_p = 0 enters
+// with c_p = g_p phi_p / 2 and g_p = |s_p| (1 - |s_p| dt/d).  A wave with s_p = 0 enters
 // neither fluctuation, as in the reference.
 // up_p = W_p . W_p of the upwind neighbour (upwind()).
 // kL3Product: be_3 = L3 - al_3 from the product L3 = s2 rS with one rounding
 // (the x sweep, which has both factors at hand; the y sweep keeps L3 alone
 // in its window).
+//
+// MC limiter phi(r) = max(0, min((1+r)/2, 2, 2r)) (fv.h:587-605), taken
+// halved: h = phi/2 = clamp(min((1+r)/4, r), 0, 1), where the clamp is the VOP3
+// output modifier of the min.  The reference sets phi = 1 where wnorm2 == 0;
+// such a wave is the zero vector, so its correction phi*W is 0 for any
+// finite phi.  Here wnorm2 == 0 gives r = NaN (0 * inf), which the clamp
+// turns into 0 (finite), and the select is skipped.
+template <typename R>
+struct LimitT {         // per wave family
+  R rn[3], r[3];        // 1/|W|^2, W . W(upwind) / |W|^2
+  R t[3], mn[3], h[3];  // (1+r)/4, min(t, r), clamp(mn)
+  R om[3], g[3];        // 1 - |s| dt/d, |s| (1 - |s| dt/d)
+  R al[3];              // max(s, 0) - g h
+};
 template <bool kL3Product, typename R>
 __device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R up1, R up2, R up3, R dtd,
-                                             R P[3], R M[3]) {
+                                             R P[3], R M[3], LimitT<R>& v) {
 #pragma clang fp contract(off)
   const WavesT<R>& w = f.w;
-  const R n1 = fma_(w.a1, w.a1, fma_(w.w21, w.w21, w.w31 * w.w31));
-  const R n2 = fma_(w.a2, w.a2, fma_(w.w22, w.w22, w.w32 * w.w32));
-  const R n3 = w.a3 * w.a3;
-  const R h1 = philim_half(n1, up1);
-  const R h2 = philim_half(n2, up2);
-  const R h3 = philim_half(n3, up3);
-  const R s1 = fabs(f.L1), s2 = fabs(f.L2), s3 = fabs(f.L3);
-  // c_p = g_p h_p
-  const R g1 = s1 * fma_(-s1, dtd, R(1));
-  const R g2 = s2 * fma_(-s2, dtd, R(1));
-  const R g3 = s3 * fma_(-s3, dtd, R(1));
+  const R n[3] = {fma_(w.a1, w.a1, fma_(w.w21, w.w21, w.w31 * w.w31)),
+                  fma_(w.a2, w.a2, fma_(w.w22, w.w22, w.w32 * w.w32)), w.a3 * w.a3};
+  const R up[3] = {up1, up2, up3}, L[3] = {f.L1, f.L2, f.L3};
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    v.rn[p] = rcp(n[p]);
+    v.r[p] = up[p] * v.rn[p];
+    v.t[p] = fma_(R(0.25), v.r[p], R(0.25));
+    v.mn[p] = min_(v.t[p], v.r[p]);
+    v.h[p] = clamp01(v.mn[p]);
+    const R s = fabs(L[p]);
+    v.om[p] = fma_(-s, dtd, R(1));
+    v.g[p] = s * v.om[p];
+    v.al[p] = fma_(-v.g[p], v.h[p], fmax2(L[p], R(0)));
+  }
   // al_p = max(s_p, 0) - c_p; be_p = min(s_p, 0) + c_p = s_p - al_p
-  const R al1 = fma_(-g1, h1, fmax2(f.L1, R(0))), be1 = f.L1 - al1;
-  const R al2 = fma_(-g2, h2, fmax2(f.L2, R(0))), be2 = f.L2 - al2;
-  const R al3 = fma_(-g3, h3, fmax2(f.L3, R(0)));
+  const R al1 = v.al[0], al2 = v.al[1], al3 = v.al[2];
+  const R be1 = f.L1 - al1, be2 = f.L2 - al2;
   const R be3 = kL3Product ? fma_(f.s2, f.rS, -al3) : f.L3 - al3;
   P[0] = fma_(al1, w.a1, al2 * w.a2);
   P[1] = fma_(al1, w.w21, al2 * w.w22);
@@ -225,6 +244,12 @@ __device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R up1, R up2, R
   M[0] = fma_(be1, w.a1, be2 * w.a2);
   M[1] = fma_(be1, w.w21, be2 * w.w22);
   M[2] = fma_(be3, w.a3, fma_(be1, w.w31, be2 * w.w32));
+}
+template <bool kL3Product, typename R>
+__device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R up1, R up2, R up3, R dtd,
+                                             R P[3], R M[3]) {
+  LimitT<R> v;
+  limited_flux<kL3Product>(f, up1, up2, up3, dtd, P, M, v);
 }
 
 }  // namespace fvna

@@ -25,6 +25,14 @@
 // x neighbours come from DPP lane shifts, y neighbours from register windows.
 // A wave runs one or more work items (row ranges of a strip) in turn; the
 // host groups them into waves of about equal cost.
+//
+// Bound by VALU issue: two waves per SIMD (255 registers each) keep it busy,
+// and HBM is a third used.  So the row is kept short: the limiter's transpose
+// takes factors formed with the forward values, neighbours' waves enter the
+// multiply-adds by DPP, rules of single rows and columns stand in branches,
+// and four rows per round leave no window moves: 872 -> about 680 VALU
+// instructions per row, a reverse step of 2048x1024 75 -> 63 us, of eight
+// 512x512 instances 81 -> 69 us (3 rows per round: 18 more moves a row).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -32,7 +40,12 @@
 #include "../apps/na/adjoint.h"
 #include "../apps/na/source.h"
 #include "fv_adjoint.h"
+#include "fv_lanes.h"
 #include "fv_types.h"
+
+// no contraction but the written-out fma_: the copies of the unrolled row
+// must round alike
+#pragma clang fp contract(off)
 
 namespace fv {
 namespace adjm {
@@ -48,21 +61,16 @@ typedef __attribute__((address_space(1))) char gchar;
 typedef __attribute__((address_space(1))) const char cgchar;
 typedef __attribute__((address_space(4))) const float kfloat;   // read-only: scalar loads
 
+__device__ __forceinline__ void add_f64(double* p, double v) {
+  __builtin_amdgcn_global_atomic_fadd_f64((__attribute__((address_space(1))) double*)p, v);
+}
+
 // loads and stores at a 32-bit byte offset from a uniform base
 __device__ __forceinline__ float ldg(cgfloat* base, uint32_t off) {
   return *(cgfloat*)((cgchar*)base + off);
 }
 __device__ __forceinline__ void stg(gfloat* base, uint32_t off, float v) {
   *(gfloat*)((gchar*)base + off) = v;
-}
-
-// shr1: lane l receives lane l-1's value (lane 0 receives 0);
-// shl1: lane l receives lane l+1's value (lane 63 receives 0).
-__device__ __forceinline__ float shr1(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float shl1(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130, 0xf, 0xf, true));
 }
 
 struct Vec3 {
@@ -75,6 +83,8 @@ __device__ __forceinline__ Vec3 operator+(const Vec3& x, const Vec3& y) {
 __device__ __forceinline__ Vec3 sel(bool p, const Vec3& x) {
   return Vec3{p ? x.a : 0.0f, p ? x.b : 0.0f, p ? x.c : 0.0f};
 }
+using fv::shl1;
+using fv::shr1;
 __device__ __forceinline__ Vec3 shr1(const Vec3& x) { return Vec3{shr1(x.a), shr1(x.b), shr1(x.c)}; }
 __device__ __forceinline__ Vec3 shl1(const Vec3& x) { return Vec3{shl1(x.a), shl1(x.b), shl1(x.c)}; }
 
@@ -87,13 +97,40 @@ struct XRow {          // one cell of q_xy (the recomputed-state check)
   float q1, q2, q3, u, v;
 };
 
-__device__ __forceinline__ fvad::SumAdj zero_sum() { return fvad::SumAdj{0.f, 0.f, 0.f, 0.f, 0.f, 0.f}; }
-// a where keep holds, else 0: one select per field (no branch, so no merge
-// of two versions of every field)
-__device__ __forceinline__ fvad::SumAdj keep_if(bool keep, const fvad::SumAdj& a) {
-  return fvad::SumAdj{keep ? a.s1 : 0.f, keep ? a.s2 : 0.f, keep ? a.s3 : 0.f,
-                      keep ? a.dr : 0.f, keep ? a.dn : 0.f, keep ? a.dt : 0.f};
+struct Vec2 {          // momentum parts
+  float b, c;
+};
+
+// ga += kp[p] times family p of the waves of the interface to the left (kR
+// false) or right: the lane move is the operand of the multiply-add (which
+// the compiler forms only where a moved value has a single use).  The s_nop
+// covers the two wait states between a write of W and its read across lanes.
+#define FV_FMAC7(dir)                                                                  \
+  asm("s_nop 1\n\t"                                                                    \
+      "v_fmac_f32_dpp %0, %7, %14 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"  \
+      "v_fmac_f32_dpp %1, %8, %14 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"  \
+      "v_fmac_f32_dpp %2, %9, %14 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"  \
+      "v_fmac_f32_dpp %3, %10, %15 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %4, %11, %15 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %5, %12, %15 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %6, %13, %16 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1"      \
+      : "+&v"(ga.g[0]), "+&v"(ga.g[1]), "+&v"(ga.g[2]), "+&v"(ga.g[3]), "+&v"(ga.g[4]),     \
+        "+&v"(ga.g[5]), "+&v"(ga.g[6])                                                   \
+      : "v"(W.a1), "v"(W.w21), "v"(W.w31), "v"(W.a2), "v"(W.w22), "v"(W.w32), "v"(W.a3), \
+        "v"(kp[0]), "v"(kp[1]), "v"(kp[2]))
+template <bool kR>
+__device__ __forceinline__ void add_scaled_lane(fvad::WaveAdj& ga, const float kp[3],
+                                                const fvna::Waves& W) {
+  if (kR)
+    FV_FMAC7("wave_shl:1");
+  else
+    FV_FMAC7("wave_shr:1");
 }
+#undef FV_FMAC7
+
+// Keeps the block it stands in a branch: a uniform condition that seldom
+// holds is then skipped, not turned into a select per register.
+__device__ __forceinline__ void stay_branch() { asm volatile(""); }
 
 // The reverse step of one work item of an instance whose ghost cells follow
 // the boundary policy BC.  kCheck: also recompute q_{n+1} on the item's
@@ -127,7 +164,6 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
   const bool col_in = i >= 0 && i < nx;
   const int ic = min(max(i, 0), nx - 1);
   const bool col_int = i >= 2 && i <= nx - 3;
-  const bool col_x = col_in && i >= 1;           // lane holds an x interface of the grid
   const bool out_lane = i >= it.xo0 && i < it.xo1;
   // dt/d on the lanes of interior columns, 0 on ghost columns
   const float dty_c = col_int ? dty : 0.0f, dtx_c = col_int ? dtx : 0.0f;
@@ -177,24 +213,33 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
   // item's own rows
   double jacc = 0.0;
   const bool in_box_col = col_in && box_col;
-  auto box_row = [&](int l) { return l >= 0 && l < ny && l >= D.by0 && l < D.by0 + D.bny; };
+  const int box0 = max(D.by0, 0), box1 = min(D.by0 + D.bny, ny);
+  auto box_row = [&](int l) { return l >= box0 && l < box1; };
+  // rows off the grid read a copy of the nearest row: what follows gives
+  // weight 0 to all but the interior rows and columns of g, which also
+  // covers the lanes off the grid
   auto load_g = [&](int l, Vec3& g, float& rn) {
-    g = v3(0.f, 0.f, 0.f);
-    rn = 0.0f;
-    if (l < 0 || l >= ny) return;
-    const uint32_t o = (uint32_t)l * row_bytes + cb;
+    const uint32_t o = (uint32_t)min(max(l, 0), ny - 1) * row_bytes + cb;
     g.a = ldg(g1p, o);
     g.b = ldg(g2p, o);
     g.c = ldg(g3p, o);
-    if (box_row(l)) rn = ldg(nq1, o);
-  };
-  auto finish_g = [&](int l, Vec3& g, float rn) {
-    g = sel(col_in, g);
     if (box_row(l)) {
-      g.a = in_box_col ? fvna::fma_(two_dt, rn, g.a) : g.a;
-      if (l >= y0 && l < y1 && in_box_col && out_lane) jacc += (double)rn * (double)rn;
+      stay_branch();
+      rn = ldg(nq1, o);
     }
   };
+  auto finish_g = [&](int l, Vec3& g, Vec2& G, float rn) {
+    if (box_row(l)) {
+      stay_branch();
+      g.a = in_box_col ? fvna::fma_(two_dt, rn, g.a) : g.a;
+      if (l >= y0 && l < y1 && in_box_col && out_lane) jacc = fma((double)rn, (double)rn, jacc);
+    }
+    const bool in = col_int && l >= 2 && l <= ny - 3;
+    G.b = in ? g.b : 0.0f;
+    G.c = in ? g.c : 0.0f;
+  };
+  const bool strip_l = it.xo0 <= 2 && 2 < it.xo1;             // holds column 2
+  const bool strip_r = it.xo0 <= nx - 3 && nx - 3 < it.xo1;   // holds column nx-3
 
   // ---- windows (every one zeroed: the first rows of the march only warm
   // them up, and nothing they hold reaches an emitted row) ----
@@ -207,11 +252,13 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
   fvad::zero(acc3);
   fvad::zero(acc2);
   Vec3 ly1{}, ly2{};                        // lam_y rows r-3, r-4
-  fvad::SumAdj gRp = zero_sum();            // transpose of interface r-4 (its cell r-4 part)
-  Vec3 gd{}, g0{}, gu{}, gnx{};             // g rows m-1, m, m+1 and the prefetched row
+  float gR1 = 0.f, gRn = 0.f, gRt = 0.f, gRun = 0.f, gRut = 0.f;   // what the transpose of
+                                            // interface r-4 gives cell r-4
+  Vec3 g0{}, gu{}, gnx{};                   // g rows m, m+1 and the prefetched row
+  Vec2 Gd{}, G0{}, Gu{};                    // g's momenta on the interior cells of rows m-1, m, m+1
   float rnx = 0.0f;                         // rho' of q_{n+1} on the prefetched row (box rows)
-  Vec3 hbot{}, htop{}, hold{};              // lam_b(0) + lam_b(1); lam_b(ny-2) + lam_b(ny-1);
-                                            // lam_n(ny-3) waiting for the top rule
+  Vec3 held{};                              // lam_b(0) + lam_b(1), later lam_n(ny-3) waiting for
+                                            // lam_b(ny-2) + lam_b(ny-1)
   XRow xc1{}, xc2{};                        // check: q_xy rows m-1, m-2
   uint32_t bad = 0;
 
@@ -224,267 +271,289 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
   load_raw(r0, n1, n2, n3, nh);
   load_g(r0 - 1, gnx, rnx);
 
-  for (int r = r0; r <= r_end; ++r) {
-    Row bn;
+  // q_b of row r, g of row r-1, the y interface r (rows r-1 | r; normal = q3,
+  // tangential = q2) and the y limiter at interface r-1
+  auto forward = [&](int r, Row& bn, fvna::Iface& fn, float* dln, float* P1, float* M,
+                     fvad::LimT& lim1) {
     bn.q1 = n1; bn.q2 = n2; bn.q3 = n3;
     patch(bn, nh, r);
     load_raw(r + 1, n1, n2, n3, nh);     // row index clamped (past r_end: unused)
-    gd = g0; g0 = gu; gu = gnx;
-    finish_g(r - 1, gu, rnx);
+    g0 = gu; gu = gnx;
+    Gd = G0; G0 = Gu;
+    finish_g(r - 1, gu, Gu, rnx);
     load_g(r, gnx, rnx);
-
-    // ---- y interface r (rows r-1 | r): normal = q3, tangential = q2 ----
-    fvna::Iface fn;
     fvna::riemann(fvna::jump(b1.q1, b1.q3, b1.q2, b1.un, b1.ut, bn.q1, bn.q3, bn.q2, bn.un,
                              bn.ut),
                   hbeta, fn);
-    float dln[3];
     dln[0] = fvna::dot1(fn.w, f1.w);
     dln[1] = fvna::dot2(fn.w, f1.w);
     dln[2] = fn.w.a3 * f1.w.a3;
-    // ---- y limiter at interface r-1 ----
-    float P1[3], M[3];
-    fvad::LimT lim1;
     fvad::limiter_rec<false>(f1, dl1[0], dln[0], dl1[1], dln[1], dl1[2], dln[2], dty, P1, M, lim1);
-
-    // The rows before y0 only warm up the windows of the forward recompute
-    // (the y interfaces and limiters the first emitted rows need); everything
-    // from q_y on is skipped there, and its window entries stay at zero (no
-    // emitted row reads them).  One guard: finer ones split the row into
-    // blocks the scheduler cannot interleave, which costs tall items more
-    // than the rows they skip.
-    Vec3 lyc{};                               // lam_y of row m = r-2
-    fvad::WaveAdj acc1;                       // wave adjoint of interface r-1
-    fvad::zero(acc1);
-    if (r >= y0) {
-      // ---- q_y on row m = r-2 (components: density, normal=q3, tangential=q2) ----
-      const int m = r - 2;
-      const bool row_int = m >= 2 && m <= ny - 3;
-      const bool upd = col_int && row_int;
-      const float dtyu = row_int ? dty_c : 0.0f, dtxu = row_int ? dtx_c : 0.0f;
-      const float y1q = fvna::sub_prod(b2.q1, dtyu, Pp[0] + M[0]);
-      const float y3q = fvna::sub_prod(b2.q3, dtyu, Pp[1] + M[1]);
-      const float y2q = fvna::sub_prod(b2.q2, dtyu, Pp[2] + M[2]);
-
-      // ---- x sweep on row m: normal = q2, tangential = q3 ----
-      const float ir = fvna::rcp(1.0f + y1q);
-      const float un = y2q * ir, ut = y3q * ir;
-      const float l1 = shr1(y1q), l2 = shr1(y2q), l3 = shr1(y3q);
-      const float lun = shr1(un), lut = shr1(ut);
-      fvna::Iface fx;
-      const fvna::Jump jx = fvna::jump(l1, l2, l3, lun, lut, y1q, y2q, y3q, un, ut);
-      fvna::riemann(jx, hbeta, fx);
-      fvna::Waves wl;
-      wl.a1 = shr1(fx.w.a1); wl.w21 = shr1(fx.w.w21); wl.w31 = shr1(fx.w.w31);
-      wl.a2 = shr1(fx.w.a2); wl.w22 = shr1(fx.w.w22); wl.w32 = shr1(fx.w.w32);
-      wl.a3 = shr1(fx.w.a3);
-      const float dlx1 = fvna::dot1(fx.w, wl), dlx2 = fvna::dot2(fx.w, wl);
-      const float dlx3 = fx.w.a3 * wl.a3;
-      const float drx1 = shl1(dlx1), drx2 = shl1(dlx2), drx3 = shl1(dlx3);
-      float PX[3], MX[3];
-      fvad::LimT limx;
-      fvad::limiter_rec<true>(fx, dlx1, drx1, dlx2, drx2, dlx3, drx3, dtx, PX, MX, limx);
-      const float mr0 = shl1(MX[0]), mr1 = shl1(MX[1]), mr2 = shl1(MX[2]);
-      XRow xc;
-      xc.q1 = fvna::sub_prod(y1q, dtxu, mr0 + PX[0]);
-      xc.q2 = fvna::sub_prod(y2q, dtxu, mr1 + PX[1]);
-      xc.q3 = fvna::sub_prod(y3q, dtxu, mr2 + PX[2]);
-      const float ir2 = fvna::rcp(1.0f + xc.q1);
-      xc.u = xc.q2 * ir2;
-      xc.v = xc.q3 * ir2;
-
-      if (kCheck) {
-        // the source of row m-1 from q_xy rows m-2, m-1, m, against q_{n+1}
-        const int s = m - 1;
-        const float uwe = shr1(xc1.u) + shl1(xc1.u);
-        const float vwe = shr1(xc1.v) + shl1(xc1.v);
-        const float i2 = fvna::source_increment(ddx2, ddy2, xc1.u, uwe, xc2.u, xc.u);
-        const float i3 = fvna::source_increment(ddx2, ddy2, xc1.v, vwe, xc2.v, xc.v);
-        const bool s_int = col_int && s >= 2 && s <= ny - 3;
-        const float r2 = s_int ? fvna::apply_source(xc1.q2, i2) : xc1.q2;
-        const float r3 = s_int ? fvna::apply_source(xc1.q3, i3) : xc1.q3;
-        // a Taylor state's ghost ring is rewritten in place by the next step's
-        // prepass (its closed form at the next T): only the cells the step
-        // computes are compared there
-        const bool cmp = BC::kId != kBcTaylor || s_int;
-        if (s >= y0 && s < y1 && out_lane && cmp) {
-          const uint32_t o = (uint32_t)s * row_bytes + cb;
-          const bool same = __float_as_uint(ldg(nq1, o)) == __float_as_uint(xc1.q1) &&
-                            __float_as_uint(ldg(nq2, o)) == __float_as_uint(r2) &&
-                            __float_as_uint(ldg(nq3, o)) == __float_as_uint(r3);
-          bad += same ? 0u : 1u;
-        }
-        xc2 = xc1;
-        xc1 = xc;
-      }
-
-      // ---- S^T on row m: the source adds ddx2 (u_W - 2u + u_E) +
-      // ddy2 (u_S - 2u + u_N) to rho u, the same with v to rho v, on interior cells ----
-      const bool int_d = col_int && m - 1 >= 2 && m - 1 <= ny - 3;
-      const bool int_u = col_int && m + 1 >= 2 && m + 1 <= ny - 3;
-      const float G2c = upd ? g0.b : 0.0f, G3c = upd ? g0.c : 0.0f;
-      const float G2y = (int_d ? gd.b : 0.0f) + (int_u ? gu.b : 0.0f);
-      const float G3y = (int_d ? gd.c : 0.0f) + (int_u ? gu.c : 0.0f);
-      const float sU = fvna::fma_(ddx2, fvna::fma_(-2.0f, G2c, shr1(G2c) + shl1(G2c)),
-                                  ddy2 * fvna::fma_(-2.0f, G2c, G2y));
-      const float sV = fvna::fma_(ddx2, fvna::fma_(-2.0f, G3c, shr1(G3c) + shl1(G3c)),
-                                  ddy2 * fvna::fma_(-2.0f, G3c, G3y));
-      Vec3 lxy;
-      lxy.a = g0.a - fvna::fma_(sU, xc.u, sV * xc.v) * ir2;
-      lxy.b = fvna::fma_(sU, ir2, g0.b);
-      lxy.c = fvna::fma_(sV, ir2, g0.c);
-
-      // ---- X^T on row m ----
-      // q_xy(k) = q_y(k) - dtxu(k) (PX(k) + MX(k+1))
-      float gPX[3] = {-dtxu * lxy.a, -dtxu * lxy.b, -dtxu * lxy.c};
-      float gMX[3] = {shr1(gPX[0]), shr1(gPX[1]), shr1(gPX[2])};
-      fvad::WaveAdj gx;
-      fvad::zero(gx);
-      float gdx[3];
-      fvad::limiter_bw(fx, limx, dtx, gPX, gMX, gx, gdx);
-      {
-        // family p of interface k dotted with k-1 (L_p > 0) or with k+1
-        fvna::Waves wr;
-        wr.a1 = shl1(fx.w.a1); wr.w21 = shl1(fx.w.w21); wr.w31 = shl1(fx.w.w31);
-        wr.a2 = shl1(fx.w.a2); wr.w22 = shl1(fx.w.w22); wr.w32 = shl1(fx.w.w32);
-        wr.a3 = shl1(fx.w.a3);
-        const float Ls[3] = {fx.L1, fx.L2, fx.L3};
-        float kl[3], kr[3];
-  #pragma unroll
-        for (int p = 0; p < 3; ++p) {
-          const float gdl = Ls[p] > 0.0f ? gdx[p] : 0.0f;
-          const float gdr = gdx[p] - gdl;
-          kl[p] = gdl + shr1(gdr);      // times W(k-1): own left dot, and k-1's right dot
-          kr[p] = gdr + shl1(gdl);      // times W(k+1): own right dot, and k+1's left dot
-        }
-        fvad::add_scaled(gx, kl, wl);
-        fvad::add_scaled(gx, kr, wr);
-      }
-      fvad::SumAdj sx = fvad::riemann_bw(jx.s1, jx.s2, jx.s3, jx.drho, jx.dn, hbeta, fx, gx);
-      sx = keep_if(col_x, sx);
-      {
-        // cell k: interface k's R part and interface k+1's L part (lane k+1)
-        const float ar1 = (sx.s1 + sx.dr) + shl1(sx.s1 - sx.dr);
-        const float an = sx.dn - shl1(sx.dn);
-        const float at = sx.dt - shl1(sx.dt);
-        const float aun = sx.s2 + shl1(sx.s2);
-        const float aut = sx.s3 + shl1(sx.s3);
-        lyc.a = lxy.a + ar1 - fvna::fma_(aun, un, aut * ut) * ir;
-        lyc.b = lxy.b + fvna::fma_(aun, ir, an);
-        lyc.c = lxy.c + fvna::fma_(aut, ir, at);
-      }
-
-      // ---- Y^T: limiter of interface m (P -> cell m, M -> cell m-1) ----
-      {
-        const float dtyu1 = (m - 1 >= 2 && m - 1 <= ny - 3) ? dty_c : 0.0f;
-        // y component order (rho', normal = rho v, tangential = rho u)
-        float gPy[3] = {-dtyu * lyc.a, -dtyu * lyc.c, -dtyu * lyc.b};
-        float gMy[3] = {-dtyu1 * ly1.a, -dtyu1 * ly1.c, -dtyu1 * ly1.b};
-        float gdy[3];
-        fvad::limiter_bw(f2, lim2, dty, gPy, gMy, acc2, gdy);
-        const float Ls[3] = {f2.L1, f2.L2, f2.L3};
-        float kdn[3], kup[3];
-  #pragma unroll
-        for (int p = 0; p < 3; ++p) {
-          kdn[p] = Ls[p] > 0.0f ? gdy[p] : 0.0f;   // dotted with interface m-1
-          kup[p] = gdy[p] - kdn[p];                // ... with m+1
-        }
-        fvad::add_scaled(acc2, kdn, f3.w);
-        fvad::add_scaled(acc2, kup, f1.w);
-        fvad::add_scaled(acc3, kdn, f2.w);
-        fvad::add_scaled(acc1, kup, f2.w);
-      }
-      // ---- Riemann transpose of interface m-1 = r-3 (rows r-4 | r-3) ----
-      fvad::SumAdj sy = fvad::riemann_bw(fvna::add_nc(b4.q1, b3.q1), fvna::add_nc(b4.un, b3.un),
-                                         fvna::add_nc(b4.ut, b3.ut), b3.q1 - b4.q1, b3.q3 - b4.q3,
-                                         hbeta, f3, acc3);
-      sy = keep_if(col_in && r - 3 >= 1 && r - 3 <= ny - 1, sy);
-      // ---- lam_b of row r-4: lam_y, interface r-4's R part, interface r-3's L part ----
-      Vec3 lb;
-      {
-        const float br1 = (gRp.s1 + gRp.dr) + (sy.s1 - sy.dr);
-        const float bn_ = gRp.dn - sy.dn;
-        const float bt = gRp.dt - sy.dt;
-        const float bun = gRp.s2 + sy.s2;
-        const float but = gRp.s3 + sy.s3;
-        const float ir4 = fvna::rcp(1.0f + b4.q1);
-        lb.a = ly2.a + br1 - fvna::fma_(bun, b4.un, but * b4.ut) * ir4;
-        lb.c = ly2.c + fvna::fma_(bun, ir4, bn_);     // normal = rho v
-        lb.b = ly2.b + fvna::fma_(but, ir4, bt);      // tangential = rho u
-      }
-      gRp = sy;
-
-      // ---- B^T and the drive gradient of row j = r-4 ----
-      const int j = r - 4;
-      if (j >= y0 && j < y1) {
-        const bool interior = col_int && j >= 2 && j <= ny - 3;
-        Vec3 a = sel(interior, lb);
-        bool defer = false;
-        if (BC::kId != kBcTaylor) {
-          // zero-gradient copies (apps/common/boundary.h): left columns <- 2
-          // (zero-gradient app only; the edge drive sets them), right columns
-          // <- nx-3 on rows 2..ny-3, rows 0, 1 <- 2 and ny-2, ny-1 <- ny-3 off
-          // the left columns
-          if (BC::kId == kBcZeroGrad) {
-            const Vec3 w1 = shr1(lb), w2 = shr1(w1);
-            if (i == 2) a = a + w1 + w2;
-          }
-          {
-            const Vec3 e1 = shl1(lb), e2 = shl1(e1);
-            if (i == nx - 3 && j >= 2 && j <= ny - 3) a = a + e1 + e2;
-          }
-          if (j == 0) hbot = lb;
-          if (j == 1) hbot = hbot + lb;
-          if (j == 2 && i >= 2) a = a + hbot;
-          if (j >= ny - 2) htop = htop + lb;
-          if (j == ny - 3) {
-            hold = a;
-            defer = true;
-          }
-        }
-        const uint32_t o = (uint32_t)j * row_bytes + cb;
-        if (out_lane && !defer) {
-          stg(o1, o, a.a);
-          stg(o2, o, a.b);
-          stg(o3, o, a.c);
-        }
-        if (BC::kId != kBcTaylor && j == ny - 1) {
-          const Vec3 t = i >= 2 ? hold + htop : hold;
-          const uint32_t ot = (uint32_t)(ny - 3) * row_bytes + cb;
-          if (out_lane) {
-            stg(o1, ot, t.a);
-            stg(o2, ot, t.b);
-            stg(o3, ot, t.c);
-          }
-        }
-        if (BC::kId == kBcEdgeDrive && it.xo0 == 0) {
-          // left columns hold p = ampc sin(theta) + amps cos(theta), rho u = p (p + 1)
-          const float ec = ((kfloat*)D.edge_c)[j], es = ((kfloat*)D.edge_s)[j];
-          fvbc::Cell<float> dc;
-          fvbc::drive(ec, es, sin_t, cos_t, dc);
-          const float p = dc.q1;
-          const float tp = (i == 0 || i == 1) ? fvna::fma_(lb.b, 2.0f * p + 1.0f, lb.a) : 0.0f;
-          // columns 0 and 1 are lanes kHalo and kHalo + 1 of the first strip
-          const int tb0 = __builtin_amdgcn_readlane(__float_as_int(tp), kHalo);
-          const int tb1 = __builtin_amdgcn_readlane(__float_as_int(tp), kHalo + 1);
-          const double g = (double)__int_as_float(tb0) + (double)__int_as_float(tb1);
-          if (lane == 0) {
-            D.grad_ec[j] += g * (double)sin_t;
-            D.grad_es[j] += g * (double)cos_t;
-          }
-        }
-      }
-
-    }
-
-    // ---- rotate the windows ----
+  };
+  auto rotate = [&](const Row& bn, const fvna::Iface& fn, const float* dln, const float* P1,
+                    const fvad::LimT& lim1) {
     b4 = b3; b3 = b2; b2 = b1; b1 = bn;
     f3 = f2; f2 = f1; f1 = fn;
     lim2 = lim1;
     dl1[0] = dln[0]; dl1[1] = dln[1]; dl1[2] = dln[2];
     Pp[0] = P1[0]; Pp[1] = P1[1]; Pp[2] = P1[2];
+  };
+
+  // The rows before y0 only warm up the windows of the forward recompute (the
+  // y interfaces and limiters the first emitted rows need); everything from
+  // q_y on is skipped there, and its windows stay at zero (no emitted row
+  // reads them).
+#pragma unroll 1
+  for (int r = r0; r < y0; ++r) {
+    Row bn;
+    fvna::Iface fn;
+    fvad::LimT lim1;
+    float dln[3], P1[3], M[3];
+    forward(r, bn, fn, dln, P1, M, lim1);
+    rotate(bn, fn, dln, P1, lim1);
+  }
+  auto row = [&](int r) {
+    Row bn;
+    fvna::Iface fn;
+    fvad::LimT lim1;
+    float dln[3], P1[3], M[3];
+    forward(r, bn, fn, dln, P1, M, lim1);
+
+    // ---- q_y on row m = r-2 (components: density, normal=q3, tangential=q2) ----
+    const int m = r - 2;
+    const bool row_int = m >= 2 && m <= ny - 3;
+    const float dtyu = row_int ? dty_c : 0.0f, dtxu = row_int ? dtx_c : 0.0f;
+    const float y1q = fvna::sub_prod(b2.q1, dtyu, Pp[0] + M[0]);
+    const float y3q = fvna::sub_prod(b2.q3, dtyu, Pp[1] + M[1]);
+    const float y2q = fvna::sub_prod(b2.q2, dtyu, Pp[2] + M[2]);
+
+    // ---- x sweep on row m: normal = q2, tangential = q3 ----
+    const float ir = fvna::rcp(1.0f + y1q);
+    const float un = y2q * ir, ut = y3q * ir;
+    fvna::Iface fx;
+    fvna::SolveT<float> vx;
+    const fvna::Jump jx = fvna::jump(shr1(y1q), shr1(y2q), shr1(y3q), shr1(un), shr1(ut), y1q,
+                                     y2q, y3q, un, ut);
+    fvna::riemann(jx, hbeta, fx, vx);
+    float dlx1, dlx2, dlx3;
+    dots_left(fx.w, dlx1, dlx2, dlx3);
+    const float drx1 = shl1(dlx1), drx2 = shl1(dlx2), drx3 = shl1(dlx3);
+    float PX[3], MX[3];
+    fvad::LimT limx;
+    fvad::limiter_rec<true>(fx, dlx1, drx1, dlx2, drx2, dlx3, drx3, dtx, PX, MX, limx);
+    const float mr0 = shl1(MX[0]), mr1 = shl1(MX[1]), mr2 = shl1(MX[2]);
+    XRow xc;
+    xc.q1 = fvna::sub_prod(y1q, dtxu, mr0 + PX[0]);
+    xc.q2 = fvna::sub_prod(y2q, dtxu, mr1 + PX[1]);
+    xc.q3 = fvna::sub_prod(y3q, dtxu, mr2 + PX[2]);
+    const float ir2 = fvna::rcp(1.0f + xc.q1);
+    xc.u = xc.q2 * ir2;
+    xc.v = xc.q3 * ir2;
+
+    if (kCheck) {
+      // the source of row m-1 from q_xy rows m-2, m-1, m, against q_{n+1}
+      const int s = m - 1;
+      const float uwe = shr1(xc1.u) + shl1(xc1.u);
+      const float vwe = shr1(xc1.v) + shl1(xc1.v);
+      const float i2 = fvna::source_increment(ddx2, ddy2, xc1.u, uwe, xc2.u, xc.u);
+      const float i3 = fvna::source_increment(ddx2, ddy2, xc1.v, vwe, xc2.v, xc.v);
+      const bool s_int = col_int && s >= 2 && s <= ny - 3;
+      const float r2 = s_int ? fvna::apply_source(xc1.q2, i2) : xc1.q2;
+      const float r3 = s_int ? fvna::apply_source(xc1.q3, i3) : xc1.q3;
+      // a Taylor state's ghost ring is rewritten in place by the next step's
+      // prepass (its closed form at the next T): only the cells the step
+      // computes are compared there
+      const bool cmp = BC::kId != kBcTaylor || s_int;
+      if (s >= y0 && s < y1 && out_lane && cmp) {
+        const uint32_t o = (uint32_t)s * row_bytes + cb;
+        const bool same = __float_as_uint(ldg(nq1, o)) == __float_as_uint(xc1.q1) &&
+                          __float_as_uint(ldg(nq2, o)) == __float_as_uint(r2) &&
+                          __float_as_uint(ldg(nq3, o)) == __float_as_uint(r3);
+        bad += same ? 0u : 1u;
+      }
+      xc2 = xc1;
+      xc1 = xc;
+    }
+
+    // ---- S^T on row m: the source adds ddx2 (u_W - 2u + u_E) +
+    // ddy2 (u_S - 2u + u_N) to rho u, the same with v to rho v, on interior cells ----
+    const float sU = fvna::fma_(ddx2, fvna::fma_(-2.0f, G0.b, shr1(G0.b) + shl1(G0.b)),
+                                ddy2 * fvna::fma_(-2.0f, G0.b, Gd.b + Gu.b));
+    const float sV = fvna::fma_(ddx2, fvna::fma_(-2.0f, G0.c, shr1(G0.c) + shl1(G0.c)),
+                                ddy2 * fvna::fma_(-2.0f, G0.c, Gd.c + Gu.c));
+    Vec3 lxy;
+    lxy.a = fvna::fma_(-fvna::fma_(sU, xc.u, sV * xc.v), ir2, g0.a);
+    lxy.b = fvna::fma_(sU, ir2, g0.b);
+    lxy.c = fvna::fma_(sV, ir2, g0.c);
+
+    // ---- X^T on row m ----
+    // q_xy(k) = q_y(k) - dtxu(k) (PX(k) + MX(k+1)).  The adjoints gPX, gMX are
+    // 0 but for the interfaces 2 .. nx-2 (dtxu is 0 on ghost columns), so the
+    // waves' adjoints are 0 off the interfaces 1 .. nx-1 of the grid, and so is
+    // what their Riemann transposes give; the same holds for y.
+    Vec3 lyc;                                 // lam_y of row m
+    {
+      const float gPX[3] = {-dtxu * lxy.a, -dtxu * lxy.b, -dtxu * lxy.c};
+      const float gMX[3] = {shr1(gPX[0]), shr1(gPX[1]), shr1(gPX[2])};
+      fvad::WaveAdj gx;
+      fvad::zero(gx);
+      float gdx[3];
+      fvad::limiter_bw(fx, limx, gPX, gMX, gx, gdx);
+      // family p of interface k dotted with k-1 (L_p > 0) or with k+1
+      const float Ls[3] = {fx.L1, fx.L2, fx.L3};
+      float kl[3], kr[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        const float gdl = Ls[p] > 0.0f ? gdx[p] : 0.0f;
+        const float gdr = gdx[p] - gdl;
+        kl[p] = gdl + shr1(gdr);      // times W(k-1): own left dot, and k-1's right dot
+        kr[p] = gdr + shl1(gdl);      // times W(k+1): own right dot, and k+1's left dot
+      }
+      add_scaled_lane<false>(gx, kl, fx.w);
+      add_scaled_lane<true>(gx, kr, fx.w);
+      const fvad::SumAdj sx =
+          fvad::riemann_bw(jx.s1, jx.s2, jx.s3, jx.drho, jx.dn, hbeta, fx, vx, gx);
+      // cell k: interface k's R part and interface k+1's L part (lane k+1)
+      const float ar1 = (sx.s1 + sx.dr) + shl1(sx.s1 - sx.dr);
+      const float an = sx.dn - shl1(sx.dn);
+      const float at = sx.dt - shl1(sx.dt);
+      const float aun = sx.s2 + shl1(sx.s2);
+      const float aut = sx.s3 + shl1(sx.s3);
+      lyc.a = fvna::fma_(-fvna::fma_(aun, un, aut * ut), ir, lxy.a + ar1);
+      lyc.b = lxy.b + fvna::fma_(aun, ir, an);
+      lyc.c = lxy.c + fvna::fma_(aut, ir, at);
+    }
+
+    // ---- Y^T: limiter of interface m (P -> cell m, M -> cell m-1) ----
+    fvad::WaveAdj acc1;                       // wave adjoint of interface r-1
+    fvad::zero(acc1);
+    {
+      // y component order (rho', normal = rho v, tangential = rho u)
+      const float dtyu1 = (m - 1 >= 2 && m - 1 <= ny - 3) ? dty_c : 0.0f;
+      const float gPy[3] = {-dtyu * lyc.a, -dtyu * lyc.c, -dtyu * lyc.b};
+      const float gMy[3] = {-dtyu1 * ly1.a, -dtyu1 * ly1.c, -dtyu1 * ly1.b};
+      float gdy[3];
+      fvad::limiter_bw(f2, lim2, gPy, gMy, acc2, gdy);
+      const float Ls[3] = {f2.L1, f2.L2, f2.L3};
+      float kdn[3], kup[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        kdn[p] = Ls[p] > 0.0f ? gdy[p] : 0.0f;   // dotted with interface m-1
+        kup[p] = gdy[p] - kdn[p];                // ... with m+1
+      }
+      fvad::add_scaled(acc2, kdn, f3.w);
+      fvad::add_scaled(acc2, kup, f1.w);
+      fvad::add_scaled(acc3, kdn, f2.w);
+      fvad::add_scaled(acc1, kup, f2.w);
+    }
+    // ---- Riemann transpose of interface m-1 = r-3 (rows r-4 | r-3) ----
+    const float ys1 = fvna::add_nc(b4.q1, b3.q1), ys2 = fvna::add_nc(b4.un, b3.un);
+    const float ys3 = fvna::add_nc(b4.ut, b3.ut);
+    const fvad::SumAdj sy =
+        fvad::riemann_bw(ys1, ys2, ys3, b3.q1 - b4.q1, b3.q3 - b4.q3, hbeta, f3,
+                         fvad::solve_again(ys1, ys2, ys3, f3), acc3);
+    // ---- lam_b of row r-4: lam_y, interface r-4's R part, interface r-3's L part ----
+    Vec3 lb;
+    {
+      const float br1 = gR1 + (sy.s1 - sy.dr);
+      const float bn_ = gRn - sy.dn;
+      const float bt = gRt - sy.dt;
+      const float bun = gRun + sy.s2;
+      const float but = gRut + sy.s3;
+      const float ir4 = fvna::rcp(1.0f + b4.q1);
+      lb.a = fvna::fma_(-fvna::fma_(bun, b4.un, but * b4.ut), ir4, ly2.a + br1);
+      lb.c = ly2.c + fvna::fma_(bun, ir4, bn_);     // normal = rho v
+      lb.b = ly2.b + fvna::fma_(but, ir4, bt);      // tangential = rho u
+    }
+    gR1 = sy.s1 + sy.dr;
+    gRn = sy.dn;
+    gRt = sy.dt;
+    gRun = sy.s2;
+    gRut = sy.s3;
+
+    // ---- B^T and the drive gradient of row j = r-4 (< y1) ----
+    const int j = r - 4;
+    if (j >= y0) {
+      stay_branch();
+      const bool interior = col_int && j >= 2 && j <= ny - 3;
+      Vec3 a = sel(interior, lb);
+      uint32_t o = (uint32_t)j * row_bytes + cb;
+      bool defer = false;
+      if (BC::kId != kBcTaylor) {
+        // zero-gradient copies (apps/common/boundary.h): left columns <- 2
+        // (zero-gradient app only; the edge drive sets them), right columns
+        // <- nx-3 on rows 2..ny-3, rows 0, 1 <- 2 and ny-2, ny-1 <- ny-3 off
+        // the left columns
+        if (BC::kId == kBcZeroGrad && strip_l) {
+          stay_branch();
+          const Vec3 w1 = shr1(lb), w2 = shr1(w1);
+          if (i == 2) a = a + w1 + w2;
+        }
+        if (strip_r && j >= 2 && j <= ny - 3) {
+          stay_branch();
+          const Vec3 e1 = shl1(lb), e2 = shl1(e1);
+          if (i == nx - 3) a = a + e1 + e2;
+        }
+        if (j <= 2 || j >= ny - 3) {
+          stay_branch();
+          if (j == 0) held = lb;
+          if (j == 1) held = held + lb;
+          if (j == 2) a = a + sel(i >= 2, held);
+          if (j == ny - 3) {
+            held = a;
+            defer = true;
+          }
+          if (j >= ny - 2) held = held + sel(i >= 2, lb);
+          if (j == ny - 1 && out_lane) {
+            const uint32_t ot = (uint32_t)(ny - 3) * row_bytes + cb;
+            stg(o1, ot, held.a);
+            stg(o2, ot, held.b);
+            stg(o3, ot, held.c);
+          }
+        }
+      }
+      if (out_lane && !defer) {
+        stg(o1, o, a.a);
+        stg(o2, o, a.b);
+        stg(o3, o, a.c);
+      }
+      if (BC::kId == kBcEdgeDrive && it.xo0 == 0) {
+        stay_branch();
+        // left columns hold p = ampc sin(theta) + amps cos(theta), rho u = p (p + 1)
+        const float ec = ((kfloat*)D.edge_c)[j], es = ((kfloat*)D.edge_s)[j];
+        fvbc::Cell<float> dc;
+        fvbc::drive(ec, es, sin_t, cos_t, dc);
+        const float p = dc.q1;
+        const float tp = (i == 0 || i == 1) ? fvna::fma_(lb.b, fvna::fma_(2.0f, p, 1.0f), lb.a) : 0.0f;
+        // columns 0 and 1 are lanes kHalo and kHalo + 1 of the first strip
+        const int tb0 = __builtin_amdgcn_readlane(__float_as_int(tp), kHalo);
+        const int tb1 = __builtin_amdgcn_readlane(__float_as_int(tp), kHalo + 1);
+        const double g = (double)__int_as_float(tb0) + (double)__int_as_float(tb1);
+        // one adder per row and launch (the sum's order is the steps'): the
+        // atomic is sent off without waiting for the old value
+        if (lane == 0) {
+          add_f64(D.grad_ec + j, g * (double)sin_t);
+          add_f64(D.grad_es + j, g * (double)cos_t);
+        }
+      }
+    }
+
+    rotate(bn, fn, dln, P1, lim1);
     acc3 = acc2; acc2 = acc1;
     ly2 = ly1; ly1 = lyc;
+  };
+  // Four rows per round: the windows are four rows deep, so all but a few of
+  // the 94 register moves a row would take to shift them vanish (the compiler
+  // cannot unroll a loop with cross-lane moves by itself).
+  for (int r = y0; r <= r_end; ++r) {
+    row(r);
+    if (kCheck) continue;
+    if (++r > r_end) break;
+    row(r);
+    if (++r > r_end) break;
+    row(r);
+    if (++r > r_end) break;
+    row(r);
   }
 
   // J of this step over the item's box cells, one double per item
@@ -512,7 +581,7 @@ using namespace adjm;
 // wave_first[w] .. wave_first[w+1] in turn (the end of one strip and the
 // start of the next, when the host balances the waves' rows).
 template <bool kCheck>
-__global__ __launch_bounds__(64) void adj_reverse_kernel(const AdjDesc* __restrict__ ds,
+__global__ __launch_bounds__(64, 2) void adj_reverse_kernel(const AdjDesc* __restrict__ ds,
                                                          const AdjItem* __restrict__ items,
                                                          const int32_t* __restrict__ wave_first,
                                                          int n_waves, int k, int slot, int par) {

@@ -320,3 +320,36 @@ def test_waves_of_several_items_match_one_item_per_wave():
     assert np.abs(res[0][1]).max() > 0
     assert np.array_equal(res[0][1], res[1][1]) and np.array_equal(res[0][2], res[1][2])
     assert np.array_equal(res[0][3], res[1][3])
+
+
+@pytest.mark.parametrize("kind", ["edge_drive", "zero_gradient", "taylor"])
+def test_item_heights_do_not_change_the_gradient(kind):
+    """The reverse march takes four rows per round and leaves the round at any
+    of them: heights of 8 to 12 rows per item and the whole column in one item
+    (every remainder, cuts next to the ghost rows) give the same gradients and
+    dJ/dq0 bit for bit, and so does the checking form of the kernel (one row per
+    round)."""
+    rng = np.random.default_rng(33)
+    n = 14
+    if kind == "taylor":
+        prob, box = mk_taylor(), (20, 40, 16, 12)
+    elif kind == "zero_gradient":
+        prob, box = mk_zero_gradient(setup_case(rng)[2]), (1, 30, 12, 9)
+    else:
+        amp, ph, q0 = setup_case(rng)
+        prob, box = mk(amp, ph), BOX
+        prob.q0 = q0
+    prob.q0 = np.ascontiguousarray(prob.q0, np.float32)
+    res = []
+    for rows, check in ((1000, True), (1000, False), (8, False), (9, False), (10, False),
+                        (11, False), (12, False), (0, False)):
+        with fa.Context(prob) as ctx:
+            ctx.set_dt_sequence(0, np.full(n + 3, 0.05 if kind == "taylor" else 0.04))
+            J, ga, gp = ctx.step_adjoint(n, box, check_recompute=check, rows_per_wave=rows)
+            res.append((J[0], ga[0], gp[0], ctx.adjoint_state(0)))
+    assert res[0][0] > 0 and np.abs(np.asarray(res[0][3])).max() > 0
+    for J, ga, gp, lam in res[1:]:
+        # J is summed per item: its rounding follows the split
+        assert abs(J - res[0][0]) <= 1e-13 * res[0][0]
+        assert np.array_equal(ga, res[0][1]) and np.array_equal(gp, res[0][2])
+        assert np.array_equal(lam, res[0][3])
