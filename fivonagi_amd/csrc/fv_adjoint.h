@@ -15,14 +15,21 @@ struct AdjDesc {
   int32_t bx0, by0, bnx, bny;          // objective box
   const void* edge_c;                  // the step's drive tables (float, ny each)
   const void* edge_s;
-  float* seg;                          // states of the current segment: slot s = 3 grids
+  float* kept;                         // states kept by the forward run: slot = 3 grids
+  float* seg;                          // recomputed states 1, 2, .. of the current segment
   float* lam[2];                       // adjoint of the state (3 grids), ping-pong by step
-  const Ctl* ctl_log;                  // control block accepted step n of the run ran with
+  Ctl* ctl_log;                        // control block accepted step n of the run ran with
   double* grad_ec;                     // dJ/d(amp_j cos phase_j), ny, accumulated
   double* grad_es;                     // dJ/d(amp_j sin phase_j)
   double* jpart;                       // per work item: sum over steps of dt sum_box rho'^2
-  uint32_t* mismatch;                  // cells whose recomputed state differs (checking)
+  uint32_t* mismatch;                  // cells whose recomputed state differs (checking), and
+                                       // steps missing from the log
+  const float* start[3];               // the state the forward run starts from
+  float* lam_out;                      // where dJ/dq0 is left
 };
+
+// The place of a state: a slot of `kept` (>= 0) or, as ~slot, of `seg`.
+typedef int32_t StateSlot;
 
 // One wave's work in the reverse march: the strip whose lane kHalo holds
 // column x0, output columns [xo0, xo1), output rows [y0, y1).  Strip and row

@@ -61,6 +61,10 @@ typedef __attribute__((address_space(1))) char gchar;
 typedef __attribute__((address_space(1))) const char cgchar;
 typedef __attribute__((address_space(4))) const float kfloat;   // read-only: scalar loads
 
+__device__ __forceinline__ float* state_at(const AdjDesc& D, StateSlot s, size_t cells3) {
+  return s >= 0 ? D.kept + (size_t)s * cells3 : D.seg + (size_t)~s * cells3;
+}
+
 __device__ __forceinline__ void add_f64(double* p, double v) {
   __builtin_amdgcn_global_atomic_fadd_f64((__attribute__((address_space(1))) double*)p, v);
 }
@@ -137,7 +141,7 @@ __device__ __forceinline__ void stay_branch() { asm volatile(""); }
 // cells and count those that differ from the stored one (D.mismatch).
 template <class BC, bool kCheck>
 __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it, int item,
-                                             int k, int slot, int par) {
+                                             int k, StateSlot from, StateSlot to, int par) {
   const int nx = D.nx, ny = D.ny;
   const uint32_t n = (uint32_t)nx * (uint32_t)ny;
   const Ctl* __restrict__ C = D.ctl_log + k;
@@ -145,13 +149,14 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
   const float dtx = C->dtx, dty = C->dty, ddx2 = C->ddx2, ddy2 = C->ddy2;
   const float sin_t = (float)C->drive_s, cos_t = (float)C->drive_c;
   const float hbeta = D.hbeta;
-  const float* qs = D.seg + (size_t)slot * 3 * n;
+  const float* qs = state_at(D, from, 3 * (size_t)n);
+  const float* qn = state_at(D, to, 3 * (size_t)n);            // q_{n+1}
   cgfloat* __restrict__ in1 = (cgfloat*)qs;
   cgfloat* __restrict__ in2 = (cgfloat*)(qs + n);
   cgfloat* __restrict__ in3 = (cgfloat*)(qs + 2 * (size_t)n);
-  cgfloat* __restrict__ nq1 = (cgfloat*)(qs + 3 * (size_t)n);   // q_{n+1}
-  cgfloat* __restrict__ nq2 = (cgfloat*)(qs + 4 * (size_t)n);
-  cgfloat* __restrict__ nq3 = (cgfloat*)(qs + 5 * (size_t)n);
+  cgfloat* __restrict__ nq1 = (cgfloat*)qn;
+  cgfloat* __restrict__ nq2 = (cgfloat*)(qn + n);
+  cgfloat* __restrict__ nq3 = (cgfloat*)(qn + 2 * (size_t)n);
   cgfloat* __restrict__ g1p = (cgfloat*)D.lam[par];
   cgfloat* __restrict__ g2p = (cgfloat*)(D.lam[par] + n);
   cgfloat* __restrict__ g3p = (cgfloat*)(D.lam[par] + 2 * (size_t)n);
@@ -576,15 +581,16 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
 using namespace adjm;
 
 // One reverse step of every instance: step index k of the run (its logged
-// control block), segment slot `slot` (q_n; slot+1 holds q_{n+1}), adjoint
-// ping-pong index par (lam[par] -> lam[par^1]).  Wave w runs the items
+// control block), the places of q_n and q_{n+1}, adjoint ping-pong index par
+// (lam[par] -> lam[par^1]).  Wave w runs the items
 // wave_first[w] .. wave_first[w+1] in turn (the end of one strip and the
 // start of the next, when the host balances the waves' rows).
 template <bool kCheck>
 __global__ __launch_bounds__(64, 2) void adj_reverse_kernel(const AdjDesc* __restrict__ ds,
                                                          const AdjItem* __restrict__ items,
                                                          const int32_t* __restrict__ wave_first,
-                                                         int n_waves, int k, int slot, int par) {
+                                                         int n_waves, int k, StateSlot from,
+                                                         StateSlot to, int par) {
   // XCD-aware order, as the step kernel: consecutive waves of a strip on one XCD
   int w;
   {
@@ -598,17 +604,91 @@ __global__ __launch_bounds__(64, 2) void adj_reverse_kernel(const AdjDesc* __res
     const AdjDesc& D = ds[it.inst];
     switch (__builtin_amdgcn_readfirstlane(D.bc)) {
       case kBcZeroGrad:
-        reverse_item<fvbc::ZeroGradient, kCheck>(D, it, item, k, slot, par);
+        reverse_item<fvbc::ZeroGradient, kCheck>(D, it, item, k, from, to, par);
         break;
       case kBcEdgeDrive:
-        reverse_item<fvbc::EdgeDrive, kCheck>(D, it, item, k, slot, par);
+        reverse_item<fvbc::EdgeDrive, kCheck>(D, it, item, k, from, to, par);
         break;
       case kBcTaylor:
-        reverse_item<fvbc::Taylor, kCheck>(D, it, item, k, slot, par);
+        reverse_item<fvbc::Taylor, kCheck>(D, it, item, k, from, to, par);
         break;
       default:
         break;
     }
+  }
+}
+
+// The call's buffers before the forward run: state 0 kept, everything that is
+// accumulated or checked cleared, in one launch (seven copies and fills per
+// instance took 0.3 ms for 8).  blockIdx.y strides over the instances.
+__global__ __launch_bounds__(256) void adj_begin_kernel(const AdjDesc* __restrict__ ds,
+                                                        int n_inst, int n_items, int nsteps,
+                                                        uint32_t* __restrict__ sync,
+                                                        int sync_words) {
+  const size_t t0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t step = (size_t)gridDim.x * blockDim.x;
+  for (int k = blockIdx.y; k < n_inst; k += gridDim.y) {
+    const AdjDesc& D = ds[k];
+    const size_t n = (size_t)D.nx * (size_t)D.ny;
+    for (int f = 0; f < 3; ++f)
+      for (size_t e = t0; e < n; e += step) {
+        D.kept[f * n + e] = D.start[f][e];
+        D.lam[0][f * n + e] = 0.0f;
+      }
+    for (size_t e = t0; e < (size_t)D.ny; e += step) D.grad_ec[e] = D.grad_es[e] = 0.0;
+    for (size_t e = t0; e < (size_t)nsteps; e += step) D.ctl_log[e].dt = 0.0;
+  }
+  if (blockIdx.y == 0) {
+    const AdjDesc& D = ds[0];
+    for (size_t e = t0; e < (size_t)n_items; e += step) D.jpart[e] = 0.0;
+    for (size_t e = t0; e < (size_t)sync_words; e += step) sync[e] = 0u;
+    if (t0 < 2) D.mismatch[t0] = 0u;
+  }
+}
+
+// A segment's tables, one thread per (local step, instance): the step kernel's
+// control blocks from the log -- the logged block as the attempt's own, which
+// an idle fold keeps as it is -- and the state each step reads.  Formed here,
+// a segment needs no upload and no wait for the one before it.
+__global__ __launch_bounds__(64) void adj_segment_kernel(const AdjDesc* __restrict__ ds, int n_inst,
+                                                         int s0, int len, int keep_all,
+                                                         StateSlot first,
+                                                         InstDesc* __restrict__ rdesc,
+                                                         Ctl* __restrict__ rctl) {
+  const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (e >= len * n_inst) return;
+  const int s = e / n_inst;
+  const AdjDesc& D = ds[e - s * n_inst];
+  Ctl t = D.ctl_log[s0 + s];
+  t.cur = 0;
+  t.err = 0;
+  t.target_acc = INT64_MAX;
+  t.T_stop = __builtin_inf();
+  rctl[2 * e] = t;
+  rctl[2 * e + 1] = t;
+  const size_t n = (size_t)D.nx * (size_t)D.ny;
+  float* q = state_at(D, s == 0 ? first : keep_all ? first + s : ~(StateSlot)(s - 1), 3 * n);
+  for (int f = 0; f < 3; ++f) rdesc[e].q[0][f] = q + f * n;
+}
+
+// After the forward run: steps the log does not hold (none, by then).
+__global__ __launch_bounds__(256) void adj_log_kernel(const AdjDesc* __restrict__ ds, int n_inst,
+                                                      int nsteps) {
+  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  for (int k = blockIdx.y; k < n_inst; k += gridDim.y)
+    if (e < (size_t)nsteps && !(ds[k].ctl_log[e].dt > 0.0)) atomicAdd(ds[k].mismatch + 1, 1u);
+}
+
+// dJ/dq0 into the grids the context keeps, unless a check failed.
+__global__ __launch_bounds__(256) void adj_end_kernel(const AdjDesc* __restrict__ ds, int n_inst,
+                                                      int par) {
+  if (ds[0].mismatch[0] != 0u || ds[0].mismatch[1] != 0u) return;
+  for (int k = blockIdx.y; k < n_inst; k += gridDim.y) {
+    const AdjDesc& D = ds[k];
+    const size_t n3 = 3 * (size_t)D.nx * (size_t)D.ny;
+    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n3;
+         e += (size_t)gridDim.x * blockDim.x)
+      D.lam_out[e] = D.lam[par][e];
   }
 }
 
@@ -617,15 +697,51 @@ __global__ __launch_bounds__(64, 2) void adj_reverse_kernel(const AdjDesc* __res
 // ---------------------------------------------------------------- launches --
 
 extern "C" hipError_t fv_adj_reverse(const fv::AdjDesc* ds, const fv::AdjItem* items,
-                                     const int32_t* wave_first, int n_waves, int k, int slot,
-                                     int par, int check, hipStream_t s) {
+                                     const int32_t* wave_first, int n_waves, int k,
+                                     fv::StateSlot from, fv::StateSlot to, int par, int check,
+                                     hipStream_t s) {
   if (n_waves <= 0) return hipSuccess;
   if (check)
     hipLaunchKernelGGL(fv::adj_reverse_kernel<true>, dim3(n_waves), dim3(64), 0, s, ds, items,
-                       wave_first, n_waves, k, slot, par);
+                       wave_first, n_waves, k, from, to, par);
   else
     hipLaunchKernelGGL(fv::adj_reverse_kernel<false>, dim3(n_waves), dim3(64), 0, s, ds, items,
-                       wave_first, n_waves, k, slot, par);
+                       wave_first, n_waves, k, from, to, par);
+  return hipGetLastError();
+}
+
+// Grid of the copying kernels: 4 cells per thread, up to a few blocks per CU.
+static dim3 adj_grid(size_t max_cells, int n_inst) {
+  const size_t b = (max_cells + 1023) / 1024;
+  return dim3((unsigned)(b > 2048 ? 2048 : b), (unsigned)(n_inst > 65535 ? 65535 : n_inst));
+}
+
+extern "C" hipError_t fv_adj_begin(const fv::AdjDesc* ds, int n_inst, size_t max_cells,
+                                   int n_items, int nsteps, fv::SyncSlots* sync, int n_sync,
+                                   hipStream_t s) {
+  hipLaunchKernelGGL(fv::adj_begin_kernel, adj_grid(max_cells, n_inst), dim3(256), 0, s, ds,
+                     n_inst, n_items, nsteps, (uint32_t*)sync,
+                     (int)(sizeof(fv::SyncSlots) / 4) * n_sync);
+  return hipGetLastError();
+}
+
+extern "C" hipError_t fv_adj_segment(const fv::AdjDesc* ds, int n_inst, int s0, int len,
+                                     int keep_all, fv::StateSlot first, fv::InstDesc* rdesc,
+                                     fv::Ctl* rctl, hipStream_t s) {
+  hipLaunchKernelGGL(fv::adj_segment_kernel, dim3((len * n_inst + 63) / 64), dim3(64), 0, s, ds,
+                     n_inst, s0, len, keep_all, first, rdesc, rctl);
+  return hipGetLastError();
+}
+
+extern "C" hipError_t fv_adj_log(const fv::AdjDesc* ds, int n_inst, int nsteps, hipStream_t s) {
+  hipLaunchKernelGGL(fv::adj_log_kernel, dim3((nsteps + 255) / 256, adj_grid(1, n_inst).y), dim3(256),
+                     0, s, ds, n_inst, nsteps);
+  return hipGetLastError();
+}
+
+extern "C" hipError_t fv_adj_end(const fv::AdjDesc* ds, int n_inst, size_t max_cells, int par,
+                                 hipStream_t s) {
+  hipLaunchKernelGGL(fv::adj_end_kernel, adj_grid(max_cells, n_inst), dim3(256), 0, s, ds, n_inst, par);
   return hipGetLastError();
 }
 

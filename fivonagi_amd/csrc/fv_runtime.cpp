@@ -39,8 +39,18 @@ extern "C" hipError_t fv_launch_collect(const fv::InstDesc* insts, int n_inst, i
                                         int phase, hipStream_t stream);
 extern "C" hipError_t fv_step_waves_per_cu(int* waves, int fp64);
 extern "C" hipError_t fv_adj_reverse(const fv::AdjDesc* ds, const fv::AdjItem* items,
-                                     const int32_t* wave_first, int n_waves, int k, int slot,
-                                     int par, int check, hipStream_t s);
+                                     const int32_t* wave_first, int n_waves, int k,
+                                     fv::StateSlot from, fv::StateSlot to, int par, int check,
+                                     hipStream_t s);
+extern "C" hipError_t fv_adj_begin(const fv::AdjDesc* ds, int n_inst, size_t max_cells,
+                                   int n_items, int nsteps, fv::SyncSlots* sync, int n_sync,
+                                   hipStream_t s);
+extern "C" hipError_t fv_adj_segment(const fv::AdjDesc* ds, int n_inst, int s0, int len,
+                                     int keep_all, fv::StateSlot kept0, fv::InstDesc* rdesc,
+                                     fv::Ctl* rctl, hipStream_t s);
+extern "C" hipError_t fv_adj_log(const fv::AdjDesc* ds, int n_inst, int nsteps, hipStream_t s);
+extern "C" hipError_t fv_adj_end(const fv::AdjDesc* ds, int n_inst, size_t max_cells, int par,
+                                 hipStream_t s);
 extern "C" hipError_t fv_adj_occupancy(int* waves_per_cu);
 extern "C" hipError_t fv_launch_taylor_ghosts(const fv::InstDesc* insts, int n_inst,
                                               int max_ring, int phase, int settle,
@@ -439,8 +449,17 @@ int graph_for(fivonagi_ctx* c, int G, hipGraphExec_t* out) {
 // n attempts: single launches up to a phase-0 boundary, then graph replays
 // (graph_for: the exact length of a request up to kGraphChunk, else chunks
 // and the rest); fewer than 6 attempts run as single launches.
+// An adjoint's forward run, whose step kernel stores what the captured ones do
+// not, is launched singly: a graph made and dropped in each call costs 0.5 ms,
+// and the launches run ahead of the device.
 int launch_attempts(fivonagi_ctx* c, int64_t n) {
   c->ctl_cache_ok = false;
+  for (int64_t a = 0; a < n && c->keep_hist; ++a) {
+    hipError_t e = launch_phase(c, (int)(c->attempts % 6), a == 0, a == n - 1);
+    if (e != hipSuccess) return hip_fail(e, "fv_launch_step");
+    ++c->attempts;
+  }
+  if (c->keep_hist) n = 0;
   while (n > 0 && c->attempts % 6 != 0) {
     hipError_t e = launch_phase(c, (int)(c->attempts % 6), true, true);
     if (e != hipSuccess) return hip_fail(e, "fv_launch_step");
@@ -1283,7 +1302,13 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
   const bool keep_all = req == 1 || (req <= 0 && hist_bytes <= free_b / 2);
   int K = keep_all ? 64 : (req > 1 ? req : (int)std::ceil(std::sqrt((double)nsteps)));
   K = (int)std::min<int64_t>(K, nsteps);
-  const int64_t ncp = (nsteps + K - 1) / K;   // segments (descriptor batches when keep_all)
+  const int64_t ncp = (nsteps + K - 1) / K;   // segments (table batches when keep_all)
+  // where the reverse pass finds state n: kept, or recomputed in its segment
+  auto place = [&](int64_t n) -> fv::StateSlot {
+    if (keep_all) return (fv::StateSlot)n;
+    if (n % K == 0 || n == nsteps) return (fv::StateSlot)((n + K - 1) / K);
+    return ~(fv::StateSlot)(n % K - 1);
+  };
   const bool plain = opts && opts->plain_forward;
   const bool check = opts && opts->check_recompute;
 
@@ -1310,43 +1335,52 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
 
   // ---- device buffers of the call ----
   std::vector<fv::AdjDesc> ad(ni);
-  std::vector<float*> cps(ni);
-  std::vector<fv::Ctl*> logd(ni);
-  std::vector<float*> hist(ni, nullptr);
-  double* jpart = nullptr;
-  uint32_t* d_mis = nullptr;
+  size_t max_cells = 0;
+  // read back together: J parts, check counters, drive gradients
+  char* results = nullptr;
+  size_t results_end = 0;
+  // sent together: items, waves, descriptors, the step kernel's descriptors
+  char* tables = nullptr;
+  size_t tables_off = 0, tables_end = 0;
   fv::AdjItem* d_items = nullptr;
   int32_t* d_wave_first = nullptr;
   fv::AdjDesc* d_ad = nullptr;
   fv::InstDesc* d_rdesc = nullptr;    // the step kernel's descriptors and control
-  fv::Ctl* d_rctl = nullptr;          // blocks for the segment recompute: slot s of
-  fv::SyncSlots* d_rsync = nullptr;   // every instance, and its logged control block
+  fv::Ctl* d_rctl = nullptr;          // blocks for a segment: local step s of every
+  fv::SyncSlots* d_rsync = nullptr;   // instance, and its logged control block
+  double* jpart = nullptr;
+  uint32_t* d_mis = nullptr;
+  const bool tabled = !keep_all || c->taylor_ring > 0;   // the reverse pass launches the step
+                                                         // or the ghost kernel
   auto carve = [&](AdjArena& A) {
     jpart = A.get<double>(items.size());
-    d_mis = A.get<uint32_t>(1);
+    results = (char*)jpart;
+    d_mis = A.get<uint32_t>(2);
+    for (int k = 0; k < ni; ++k) {
+      ad[k].grad_ec = A.get<double>(c->params[k].ny);
+      ad[k].grad_es = A.get<double>(c->params[k].ny);
+    }
+    results_end = tables_off = A.off;
+    d_items = A.get<fv::AdjItem>(items.size());
+    tables = (char*)d_items;
+    d_wave_first = A.get<int32_t>(wave_first.size());
+    d_ad = A.get<fv::AdjDesc>(ni);
+    d_rdesc = A.get<fv::InstDesc>(tabled ? (size_t)K * ni : 0);
+    tables_end = A.off;
+    d_rctl = A.get<fv::Ctl>(tabled ? (size_t)K * ni * 2 : 0);
+    d_rsync = A.get<fv::SyncSlots>((size_t)3 * ni);
     for (int k = 0; k < ni; ++k) {
       const size_t n = (size_t)c->params[k].nx * c->params[k].ny;
       auto& a = ad[k];
-      if (keep_all)
-        hist[k] = a.seg = A.get<float>((size_t)(nsteps + 1) * 3 * n);
-      else
-        a.seg = A.get<float>((size_t)(K + 1) * 3 * n);
+      a.kept = A.get<float>((size_t)(keep_all ? nsteps + 1 : ncp + 1) * 3 * n);
+      // states 1 .. K-1 of a segment, and for Taylor its state 0
+      a.seg = A.get<float>(keep_all ? 0 : (size_t)(c->taylor_ring > 0 ? K : K - 1) * 3 * n);
       a.lam[0] = A.get<float>(3 * n);
       a.lam[1] = A.get<float>(3 * n);
-      logd[k] = A.get<fv::Ctl>(nsteps);
-      a.ctl_log = logd[k];
-      a.grad_ec = A.get<double>(c->params[k].ny);
-      a.grad_es = A.get<double>(c->params[k].ny);
+      a.ctl_log = A.get<fv::Ctl>(nsteps);
       a.jpart = jpart;
       a.mismatch = d_mis;
-      cps[k] = keep_all ? nullptr : A.get<float>((size_t)ncp * 3 * n);
     }
-    d_items = A.get<fv::AdjItem>(items.size());
-    d_wave_first = A.get<int32_t>(wave_first.size());
-    d_ad = A.get<fv::AdjDesc>(ni);
-    d_rdesc = A.get<fv::InstDesc>((size_t)K * ni);
-    d_rctl = A.get<fv::Ctl>((size_t)K * ni * 2);
-    d_rsync = A.get<fv::SyncSlots>((size_t)3 * ni);
   };
   for (int k = 0; k < ni; ++k) {
     const auto& p = c->params[k];
@@ -1357,6 +1391,7 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
     a.bx0 = obj[k].box_x0; a.by0 = obj[k].box_y0; a.bnx = obj[k].box_nx; a.bny = obj[k].box_ny;
     a.edge_c = c->desc[k].edge_c;
     a.edge_s = c->desc[k].edge_s;
+    max_cells = std::max(max_cells, (size_t)p.nx * p.ny);
   }
   {
     AdjArena size_only;
@@ -1377,75 +1412,80 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
     A.base = (char*)c->adj_pool;
     carve(A);
   }
+  // the grids that will hold dJ/dq0 for fivonagi_adjoint_state: those of an
+  // earlier call, or new ones that become the context's with this call's success
+  struct NewGrids {
+    std::vector<float*> v;
+    ~NewGrids() { for (float* q : v) (void)hipFree(q); }
+  } lam_new;
+  lam_new.v.assign(ni, nullptr);
   for (int k = 0; k < ni; ++k) {
-    const auto& p = c->params[k];
-    const size_t n = (size_t)p.nx * p.ny;
-    HIP_TRY(hipMemsetAsync(ad[k].lam[0], 0, sizeof(float) * 3 * n, c->stream));
-    HIP_TRY(hipMemsetAsync(ad[k].grad_ec, 0, sizeof(double) * p.ny, c->stream));
-    HIP_TRY(hipMemsetAsync(ad[k].grad_es, 0, sizeof(double) * p.ny, c->stream));
-    HIP_TRY(hipMemsetAsync(logd[k], 0, sizeof(fv::Ctl) * nsteps, c->stream));
+    float* have = k < (int)c->adj_lam.size() ? c->adj_lam[k] : nullptr;
+    if (!have) {
+      const hipError_t e = hipMalloc(&lam_new.v[k], sizeof(float) * 3 * (size_t)c->params[k].nx *
+                                                        c->params[k].ny);
+      if (e != hipSuccess) {
+        lam_new.v[k] = nullptr;
+        return hip_fail(e, "hipMalloc (adjoint state)");
+      }
+    }
+    ad[k].lam_out = have ? have : lam_new.v[k];
+    for (int f = 0; f < 3; ++f) ad[k].start[f] = c->desc[k].q[ctl[k].cur][f];
   }
-  HIP_TRY(hipMemsetAsync(jpart, 0, sizeof(double) * items.size(), c->stream));
-  HIP_TRY(hipMemsetAsync(d_mis, 0, sizeof(uint32_t), c->stream));
-  HIP_TRY(hipMemsetAsync(d_rsync, 0, sizeof(fv::SyncSlots) * 3 * ni, c->stream));
-  HIP_TRY(hipMemcpyAsync(d_items, items.data(), sizeof(fv::AdjItem) * items.size(),
-                         hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipMemcpyAsync(d_wave_first, wave_first.data(), sizeof(int32_t) * wave_first.size(),
-                         hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipMemcpyAsync(d_ad, ad.data(), sizeof(fv::AdjDesc) * ni, hipMemcpyHostToDevice,
+  std::vector<char> h;                 // read by the copy until the stream is waited for
+  {
+    // The step kernel's descriptors of a segment's local steps.  The state a
+    // step reads is set per segment on the device (fv_adj_segment); its output
+    // goes to the segment's next slot (the last local step is not recomputed)
+    h.assign(tables_end - tables_off, 0);
+    auto at = [&](const void* d) { return h.data() + ((const char*)d - tables); };
+    std::memcpy(at(d_items), items.data(), sizeof(fv::AdjItem) * items.size());
+    std::memcpy(at(d_wave_first), wave_first.data(), sizeof(int32_t) * wave_first.size());
+    std::memcpy(at(d_ad), ad.data(), sizeof(fv::AdjDesc) * ni);
+    for (int s = 0; s < K && tabled; ++s)
+      for (int k = 0; k < ni; ++k) {
+        const size_t n = (size_t)c->params[k].nx * c->params[k].ny;
+        fv::InstDesc d = c->desc[k];
+        for (int f = 0; f < 3; ++f) {
+          d.q[0][f] = nullptr;
+          d.q[1][f] = keep_all || s + 1 >= K ? nullptr : ad[k].seg + ((size_t)s * 3 + f) * n;
+        }
+        d.ctl = d_rctl + 2 * ((size_t)s * ni + k);
+        d.sync = d_rsync + 3 * (size_t)k;
+        d.dt_seq = nullptr;
+        d.dt_seq_len = 0;
+        d.ctl_log = nullptr;
+        d.hist = nullptr;
+        d.measure = nullptr;
+        d.stage = nullptr;
+        d.md_on = 0;
+        d.ring = 0;                    // these states have no ghost ring
+        std::memcpy(at(d_rdesc + (size_t)s * ni + k), &d, sizeof(d));
+      }
+    HIP_TRY(hipMemcpyAsync(tables, h.data(), h.size(), hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(fv_adj_begin(d_ad, ni, max_cells, (int)items.size(), (int)nsteps, d_rsync, 3 * ni,
                          c->stream));
+  }
 
-  // ---- forward: log the control block of every accepted step; keep every
-  // state (the extended step kernel also stores its output into the history
-  // slot of its step) or a checkpoint every K steps ----
+  // ---- forward: log the control block of every accepted step and keep every
+  // state, or one every K steps and the last (the extended step kernel also
+  // stores its output into the history slot of its step) ----
   for (int k = 0; k < ni; ++k) {
-    c->desc[k].ctl_log = logd[k];
+    c->desc[k].ctl_log = ad[k].ctl_log;
     c->desc[k].log_base = ctl[k].n_acc;
     c->desc[k].log_len = nsteps;
-    c->desc[k].hist = hist[k];
+    c->desc[k].hist = ad[k].kept;
+    c->desc[k].hist_every = keep_all ? 1 : K;
   }
   int rc = upload_tables(c);
-  if (keep_all && rc == 0) {
-    for (int k = 0; k < ni && rc == 0; ++k) {
-      const size_t n = (size_t)c->params[k].nx * c->params[k].ny;
-      for (int f = 0; f < 3 && rc == 0; ++f) {
-        hipError_t e = hipMemcpyAsync(hist[k] + (size_t)f * n, c->desc[k].q[ctl[k].cur][f],
-                                      sizeof(float) * n, hipMemcpyDeviceToDevice, c->stream);
-        if (e != hipSuccess) rc = hip_fail(e, "state history copy");
-      }
-    }
-    c->keep_hist = true;
-    c->drop_graph();            // the captured launches become the extended kernel's
-    if (rc == 0) {
-      if (plain) {
-        for (int64_t s = 0; s < nsteps && rc == 0; ++s) rc = fivonagi_step(c, 1);
-      } else {
-        rc = fivonagi_step(c, nsteps);
-      }
-    }
-    c->keep_hist = false;
-    c->drop_graph();
+  c->keep_hist = true;
+  if (plain) {
+    // the reference's pattern: one launch per step, dt read back every step
+    for (int64_t s = 0; s < nsteps && rc == 0; ++s) rc = fivonagi_step(c, 1);
+  } else if (rc == 0) {
+    rc = fivonagi_step(c, nsteps);
   }
-  for (int64_t cp = 0; cp < ncp && rc == 0 && !keep_all; ++cp) {
-    if ((rc = read_ctls(c, ctl))) break;
-    for (int k = 0; k < ni; ++k) {
-      const size_t n = (size_t)c->params[k].nx * c->params[k].ny;
-      for (int f = 0; f < 3; ++f) {
-        hipError_t e = hipMemcpyAsync(cps[k] + ((size_t)cp * 3 + f) * n,
-                                      c->desc[k].q[ctl[k].cur][f], sizeof(float) * n,
-                                      hipMemcpyDeviceToDevice, c->stream);
-        if (e != hipSuccess) { rc = hip_fail(e, "checkpoint copy"); break; }
-      }
-    }
-    if (rc) break;
-    const int64_t len = std::min<int64_t>(K, nsteps - cp * K);
-    if (plain) {
-      // the reference's pattern: one launch per step, dt read back every step
-      for (int64_t s = 0; s < len && rc == 0; ++s) rc = fivonagi_step(c, 1);
-    } else {
-      rc = fivonagi_step(c, len);
-    }
-  }
+  c->keep_hist = false;
   for (int k = 0; k < ni; ++k) {
     c->desc[k].ctl_log = nullptr;
     c->desc[k].hist = nullptr;
@@ -1453,75 +1493,31 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
   int rc2 = upload_tables(c);
   if (rc) return rc;
   if (rc2) return rc2;
-  if (int r = read_ctls(c, ctl)) return r;      // the final state's buffer (cur)
-  std::vector<fv::Ctl> hlog((size_t)ni * nsteps);
-  for (int k = 0; k < ni; ++k)
-    HIP_TRY(hipMemcpyAsync(hlog.data() + (size_t)k * nsteps, logd[k], sizeof(fv::Ctl) * nsteps,
-                           hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  for (size_t e = 0; e < hlog.size(); ++e)
-    if (!(hlog[e].dt > 0.0)) return fail(FIVONAGI_ERR_ARG, "adjoint: step log incomplete");
+  HIP_TRY(fv_adj_log(d_ad, ni, (int)nsteps, c->stream));
 
   // ---- reverse, segment by segment: recompute the segment's states with
   // the step kernel (each step from its logged control block) unless every
   // state was kept, then march the adjoint back over them ----
-  std::vector<fv::InstDesc> rdh((size_t)K * ni);
-  std::vector<fv::Ctl> rch((size_t)K * ni * 2);
   const bool one = ni == 1;
   int par = 0;
   for (int64_t seg = ncp - 1; seg >= 0; --seg) {
     const int64_t s0 = seg * K;
     const int len = (int)std::min<int64_t>(K, nsteps - s0);
-    // the previous segment's kernels read the descriptors rewritten below
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    // the reverse kernel's slot of local step s: its own slot of the
-    // segment buffer, or step s0 + s of the kept states
-    const int64_t slot0 = keep_all ? s0 : 0;
-    for (int k = 0; k < ni; ++k) {
-      const size_t n = (size_t)c->params[k].nx * c->params[k].ny;
-      float* sg = ad[k].seg + (size_t)slot0 * 3 * n;
-      if (!keep_all) {
-        HIP_TRY(hipMemcpyAsync(sg, cps[k] + (size_t)seg * 3 * n, sizeof(float) * 3 * n,
+    fv::StateSlot first = place(s0);
+    if (c->taylor_ring > 0 && !keep_all) {
+      // the ghost launch below writes into the state it is given; the kept one
+      // stays as the step before it left it
+      first = ~(fv::StateSlot)(K - 1);
+      for (int k = 0; k < ni; ++k) {
+        const size_t n = (size_t)c->params[k].nx * c->params[k].ny;
+        HIP_TRY(hipMemcpyAsync(ad[k].seg + (size_t)(K - 1) * 3 * n,
+                               ad[k].kept + (size_t)place(s0) * 3 * n, sizeof(float) * 3 * n,
                                hipMemcpyDeviceToDevice, c->stream));
-        // the state after the segment into slot len (rho' for the objective;
-        // every field when checking the recompute against it)
-        for (int f = 0; f < (check ? 3 : 1); ++f) {
-          const float* src = seg + 1 < ncp ? cps[k] + ((size_t)(seg + 1) * 3 + f) * n
-                                           : c->desc[k].q[ctl[k].cur][f];
-          HIP_TRY(hipMemcpyAsync(sg + ((size_t)len * 3 + f) * n, src, sizeof(float) * n,
-                                 hipMemcpyDeviceToDevice, c->stream));
-        }
-      }
-      for (int s = 0; s < len; ++s) {
-        fv::InstDesc d = c->desc[k];
-        for (int f = 0; f < 3; ++f) {
-          d.q[0][f] = sg + ((size_t)s * 3 + f) * n;
-          d.q[1][f] = sg + ((size_t)(s + 1) * 3 + f) * n;
-        }
-        d.ctl = d_rctl + 2 * ((size_t)s * ni + k);
-        d.sync = d_rsync + 3 * (size_t)k;
-        d.dt_seq = nullptr;
-        d.dt_seq_len = 0;
-        d.ctl_log = nullptr;
-        d.measure = nullptr;
-        d.stage = nullptr;
-        d.md_on = 0;
-        d.ring = 0;                    // the segment's slots have no ghost ring
-        rdh[(size_t)s * ni + k] = d;
-        // the logged block as the attempt's own (an idle fold keeps it as is)
-        fv::Ctl t = hlog[(size_t)k * nsteps + s0 + s];
-        t.cur = 0;
-        t.err = 0;
-        t.target_acc = INT64_MAX;
-        t.T_stop = INFINITY;
-        rch[2 * ((size_t)s * ni + k)] = t;
-        rch[2 * ((size_t)s * ni + k) + 1] = t;
       }
     }
-    HIP_TRY(hipMemcpyAsync(d_rdesc, rdh.data(), sizeof(fv::InstDesc) * len * ni,
-                           hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipMemcpyAsync(d_rctl, rch.data(), sizeof(fv::Ctl) * 2 * len * ni,
-                           hipMemcpyHostToDevice, c->stream));
+    if (tabled)
+      HIP_TRY(fv_adj_segment(d_ad, ni, (int)s0, len, keep_all ? 1 : 0, first, d_rdesc, d_rctl,
+                             c->stream));
     // recompute states 1 .. len-1 of the segment (phase 0: every launch
     // reads control block 0 and the never-written slot set 2, an idle fold)
     for (int s = 0; s + 1 < len && !keep_all; ++s) {
@@ -1539,26 +1535,25 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
         HIP_TRY(fv_launch_taylor_ghosts(d_rdesc + (size_t)s * ni, ni, c->taylor_ring, 0, 0,
                                         c->stream));
       HIP_TRY(fv_adj_reverse(d_ad, d_items, d_wave_first, (int)wave_first.size() - 1,
-                             (int)(s0 + s), (int)(slot0 + s), par, check ? 1 : 0, c->stream));
+                             (int)(s0 + s), s == 0 ? first : place(s0 + s), place(s0 + s + 1),
+                             par, check ? 1 : 0, c->stream));
       par ^= 1;
     }
   }
+  HIP_TRY(fv_adj_end(d_ad, ni, max_cells, par, c->stream));
 
   // ---- results ----
-  std::vector<double> jp(items.size());
-  HIP_TRY(hipMemcpyAsync(jp.data(), jpart, sizeof(double) * items.size(), hipMemcpyDeviceToHost,
-                         c->stream));
-  uint32_t mism = 0;
-  HIP_TRY(hipMemcpyAsync(&mism, d_mis, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+  std::vector<char> res(results_end);
+  if (int r = download(c, {Span{results, res.data(), res.size()}})) return r;
+  auto host = [&](const void* d) { return res.data() + ((const char*)d - results); };
+  const double* jp = (const double*)host(jpart);
+  const uint32_t* mis = (const uint32_t*)host(d_mis);
+  if (mis[1] != 0) return fail(FIVONAGI_ERR_ARG, "adjoint: step log incomplete");
   size_t goff = 0;
   for (int k = 0; k < ni; ++k) {
     const auto& p = c->params[k];
-    std::vector<double> gc(p.ny), gs(p.ny);
-    HIP_TRY(hipMemcpyAsync(gc.data(), ad[k].grad_ec, sizeof(double) * p.ny,
-                           hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(gs.data(), ad[k].grad_es, sizeof(double) * p.ny,
-                           hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    const double* gc = (const double*)host(ad[k].grad_ec);
+    const double* gs = (const double*)host(ad[k].grad_es);
     double acc = 0.0;                       // item order: the same sum every call
     for (size_t it = first_item[k]; it < first_item[k + 1]; ++it) acc += jp[it];
     J[k] = acc;
@@ -1572,25 +1567,12 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
     }
     goff += p.ny;
   }
-  if (check && mism != 0)
-    return fail(FIVONAGI_ERR_CHECK, "adjoint: " + std::to_string(mism) +
+  if (check && mis[0] != 0)
+    return fail(FIVONAGI_ERR_CHECK, "adjoint: " + std::to_string(mis[0]) +
                                          " recomputed cells differ from the forward's");
-  // keep dJ/dq0 for fivonagi_adjoint_state (the grids of the first call are
-  // reused: an instance's size does not change)
   if (c->adj_lam.size() != (size_t)ni) c->adj_lam.assign(ni, nullptr);
-  for (int k = 0; k < ni; ++k) {
-    const size_t n = (size_t)c->params[k].nx * c->params[k].ny;
-    if (!c->adj_lam[k]) {
-      hipError_t e = hipMalloc(&c->adj_lam[k], sizeof(float) * 3 * n);
-      if (e != hipSuccess) {
-        c->adj_lam[k] = nullptr;
-        return hip_fail(e, "hipMalloc (adjoint state)");
-      }
-    }
-    HIP_TRY(hipMemcpyAsync(c->adj_lam[k], ad[k].lam[par], sizeof(float) * 3 * n,
-                           hipMemcpyDeviceToDevice, c->stream));
-  }
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  for (int k = 0; k < ni; ++k)
+    if (lam_new.v[k]) std::swap(c->adj_lam[k], lam_new.v[k]);
   return 0;
 }
 

@@ -662,9 +662,8 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
   }
   const bool stage_on = kExt && D.stage != nullptr;
   typename Mem<R>::g* __restrict__ stage = (typename Mem<R>::g*)((R*)D.stage + (phase & 1) * nx);
-  // adjoint forward runs that keep every state: this attempt's output also
-  // goes to history slot n_acc + 1 - log_base, the slot of the count it
-  // makes if accepted.  A rejected attempt's copy is overwritten by the
+  // adjoint forward runs: this attempt's output also goes to its history slot
+  // where the count it makes if accepted is one of those kept.  A rejected attempt's copy is overwritten by the
   // retry, which has the same count, so the slot ends with the accepted
   // state (FP32 instances, extended instantiation only).
   gfloat* __restrict__ hs1 = nullptr;
@@ -673,10 +672,14 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
   if constexpr (kExt && sizeof(R) == 4) {
     const int64_t t = P.n_acc + 1 - D.log_base;
     if (D.hist != nullptr && t >= 1 && t <= D.log_len) {
-      const size_t n = (size_t)nx * (size_t)ny;
-      hs1 = (gfloat*)(D.hist + (size_t)t * 3 * n);
-      hs2 = hs1 + n;
-      hs3 = hs2 + n;
+      const uint32_t every = (uint32_t)D.hist_every;
+      const uint32_t slot = ((uint32_t)t + every - 1) / every;
+      if (slot * every == (uint32_t)t || t == D.log_len) {
+        const size_t n = (size_t)nx * (size_t)ny;
+        hs1 = (gfloat*)(D.hist + (size_t)slot * 3 * n);
+        hs2 = hs1 + n;
+        hs3 = hs2 + n;
+      }
     }
   }
   const bool hist_on = kExt && sizeof(R) == 4 && hs1 != nullptr;

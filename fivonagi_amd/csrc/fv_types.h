@@ -66,8 +66,9 @@ struct InstDesc {
   int64_t dt_seq_len;
   Ctl* ctl_log;         // when set: the control block accepted step n_acc - log_base ran with
   int64_t log_base, log_len;
-  float* hist;          // when set (FP32): state n_acc - log_base after each accepted
-                        // step, slot t = 3 grids, t in [1, log_len] (the extended step kernel)
+  float* hist;          // when set (FP32): the state after accepted step t = n_acc - log_base,
+                        // t in [1, log_len], every hist_every steps and after the last, slot
+                        // ceil(t / hist_every) = 3 grids (the extended step kernel)
   double dx, dy, delta, cfl_max, cfl_wish, omega;
   double inv_dx, inv_dy;     // 1/dx, 1/dy
   double dif_x, dif_y;       // delta/dx^2, delta/dy^2
@@ -77,7 +78,7 @@ struct InstDesc {
   int32_t bc, cfl_mask;  // cfl_mask: host-side record of the fold subset kind
   SyncSlots* sync;      // 3 reduction slot sets (attempt index mod 3)
   int32_t n_items;      // work items (waves) of this instance per step
-  int32_t pad2;
+  int32_t hist_every;
   int32_t tay_jc;
   int32_t md_on;        // moving window (common/main.cu:109-177)
   float beta2m2;        // 2*(BETA - 1)

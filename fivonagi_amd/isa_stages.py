@@ -99,7 +99,7 @@ def compile_asm(text, tmp, tag):
     src = os.path.join(tmp, f"{tag}.hip")
     # the copy includes the kernel's headers by their paths from csrc/
     text = text.replace('#include "../apps/', f'#include "{os.path.join(HERE, "apps")}/')
-    text = text.replace('#include "fv_types.h"', f'#include "{os.path.join(HERE, "csrc", "fv_types.h")}"')
+    text = text.replace('#include "fv_', f'#include "{os.path.join(HERE, "csrc")}/fv_')
     with open(src, "w") as f:
         f.write(text)
     out = os.path.join(tmp, f"{tag}.s")
