@@ -59,7 +59,9 @@ __device__ __forceinline__ void limiter_rec(const Iface& f, float dl1, float dr1
   const float up1 = fvna::upwind(f.L1, dl1, dr1), up2 = fvna::upwind(f.L2, dl2, dr2);
   const float up3 = fvna::upwind(f.L3, dl3, dr3);
   fvna::LimitT<float> v;
-  fvna::limited_flux<kL3Product>(f, up1, up2, up3, dtd, P, M, v);
+  float n1, n2;
+  fvna::norms(f.w, n1, n2);
+  fvna::limited_flux<kL3Product>(f, n1, n2, up1, up2, up3, dtd, P, M, v);
   const float L[3] = {f.L1, f.L2, f.L3};
 #pragma unroll
   for (int p = 0; p < 3; ++p) {

@@ -183,6 +183,14 @@ __device__ __forceinline__ R dot2(const WavesT<R>& a, const WavesT<R>& b) {
   return fma_(b.a2, a.a2, fma_(b.w22, a.w22, b.w32 * a.w32));
 }
 
+// |W_1|^2, |W_2|^2
+template <typename R>
+__device__ __forceinline__ void norms(const WavesT<R>& w, R& n1, R& n2) {
+#pragma clang fp contract(off)
+  n1 = fma_(w.a1, w.a1, fma_(w.w21, w.w21, w.w31 * w.w31));
+  n2 = fma_(w.a2, w.a2, fma_(w.w22, w.w22, w.w32 * w.w32));
+}
+
 // The dot product with the upwind neighbour by the sign of the speed s:
 // dotl = W . W(k-1), dotr = W . W(k+1).
 template <typename R>
@@ -196,7 +204,7 @@ __device__ __forceinline__ R upwind(R s, R dotl, R dotr) {
 //   M = amdq + fadd = sum_p (min(s_p,0) + c_p) W_p   (cell on the - side)
 // with c_p = g_p phi_p / 2 and g_p = |s_p| (1 - |s_p| dt/d).  A wave with s_p = 0 enters
 // neither fluctuation, as in the reference.
-// up_p = W_p . W_p of the upwind neighbour (upwind()).
+// n1, n2: norms(); up_p = W_p . W_p of the upwind neighbour (upwind()).
 // kL3Product: be_3 = L3 - al_3 from the product L3 = s2 rS with one rounding
 // (the x sweep, which has both factors at hand; the y sweep keeps L3 alone
 // in its window).
@@ -215,12 +223,11 @@ struct LimitT {         // per wave family
   R al[3];              // max(s, 0) - g h
 };
 template <bool kL3Product, typename R>
-__device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R up1, R up2, R up3, R dtd,
-                                             R P[3], R M[3], LimitT<R>& v) {
+__device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R n1, R n2, R up1, R up2, R up3,
+                                             R dtd, R P[3], R M[3], LimitT<R>& v) {
 #pragma clang fp contract(off)
   const WavesT<R>& w = f.w;
-  const R n[3] = {fma_(w.a1, w.a1, fma_(w.w21, w.w21, w.w31 * w.w31)),
-                  fma_(w.a2, w.a2, fma_(w.w22, w.w22, w.w32 * w.w32)), w.a3 * w.a3};
+  const R n[3] = {n1, n2, w.a3 * w.a3};
   const R up[3] = {up1, up2, up3}, L[3] = {f.L1, f.L2, f.L3};
 #pragma unroll
   for (int p = 0; p < 3; ++p) {
@@ -246,10 +253,10 @@ __device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R up1, R up2, R
   M[2] = fma_(be3, w.a3, fma_(be1, w.w31, be2 * w.w32));
 }
 template <bool kL3Product, typename R>
-__device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R up1, R up2, R up3, R dtd,
-                                             R P[3], R M[3]) {
+__device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R n1, R n2, R up1, R up2, R up3,
+                                             R dtd, R P[3], R M[3]) {
   LimitT<R> v;
-  limited_flux<kL3Product>(f, up1, up2, up3, dtd, P, M, v);
+  limited_flux<kL3Product>(f, n1, n2, up1, up2, up3, dtd, P, M, v);
 }
 
 }  // namespace fvna

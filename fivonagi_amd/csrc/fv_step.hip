@@ -129,22 +129,33 @@ __device__ __forceinline__ void masked_max(uint64_t mask, double& S, double a, d
 }
 
 // fvna::upwind of the x sweep: dl on the lanes with a positive speed, else the
-// right neighbour's dl, whose move folds into the select.
+// right neighbour's dl, whose move folds into the select; and fvna::norms, whose
+// multiply-adds fill the two wait states a select needs after the comparison
+// that writes its mask.
 __device__ __forceinline__ void upwind_x(const fvna::IfaceT<float>& f, float dl1, float dl2,
-                                         float dl3, float& up1, float& up2, float& up3) {
-  asm("s_nop 0\n\t"
-      "v_cmp_lt_f32_e32 vcc, 0, %3\n\t"
-      "v_cndmask_b32_dpp %0, %6, %6, vcc wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-      "v_cmp_lt_f32_e32 vcc, 0, %4\n\t"
-      "v_cndmask_b32_dpp %1, %7, %7, vcc wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-      "v_cmp_lt_f32_e32 vcc, 0, %5\n\t"
-      "v_cndmask_b32_dpp %2, %8, %8, vcc wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1"
-      : "=&v"(up1), "=&v"(up2), "=&v"(up3)
-      : "v"(f.L1), "v"(f.L2), "v"(f.L3), "v"(dl1), "v"(dl2), "v"(dl3)
+                                         float dl3, float& up1, float& up2, float& up3, float& n1,
+                                         float& n2) {
+  asm("v_cmp_lt_f32_e32 vcc, 0, %5\n\t"
+      "v_mul_f32_e32 %3, %13, %13\n\t"
+      "v_mul_f32_e32 %4, %16, %16\n\t"
+      "v_cndmask_b32_dpp %0, %8, %8, vcc wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "v_cmp_lt_f32_e32 vcc, 0, %6\n\t"
+      "v_fmac_f32_e32 %3, %12, %12\n\t"
+      "v_fmac_f32_e32 %4, %15, %15\n\t"
+      "v_cndmask_b32_dpp %1, %9, %9, vcc wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "v_cmp_lt_f32_e32 vcc, 0, %7\n\t"
+      "v_fmac_f32_e32 %3, %11, %11\n\t"
+      "v_fmac_f32_e32 %4, %14, %14\n\t"
+      "v_cndmask_b32_dpp %2, %10, %10, vcc wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+      : "=&v"(up1), "=&v"(up2), "=&v"(up3), "=&v"(n1), "=&v"(n2)
+      : "v"(f.L1), "v"(f.L2), "v"(f.L3), "v"(dl1), "v"(dl2), "v"(dl3), "v"(f.w.a1), "v"(f.w.w21),
+        "v"(f.w.w31), "v"(f.w.a2), "v"(f.w.w22), "v"(f.w.w32)
       : "vcc");
 }
 __device__ __forceinline__ void upwind_x(const fvna::IfaceT<double>& f, double dl1, double dl2,
-                                         double dl3, double& up1, double& up2, double& up3) {
+                                         double dl3, double& up1, double& up2, double& up3,
+                                         double& n1, double& n2) {
+  fvna::norms(f.w, n1, n2);
   up1 = fvna::upwind(f.L1, dl1, shl1(dl1));
   up2 = fvna::upwind(f.L2, dl2, shl1(dl2));
   up3 = fvna::upwind(f.L3, dl3, shl1(dl3));
@@ -869,7 +880,9 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
     // ---- y limiter at interface r-1 ----
     R M[3];
     if constexpr (kT <= 8) {
-      fvna::limited_flux<false>(fc.f, fvna::upwind(fc.f.L1, fc.dl[0], fn.dl[0]),
+      R nw1, nw2;
+      fvna::norms(fc.f.w, nw1, nw2);
+      fvna::limited_flux<false>(fc.f, nw1, nw2, fvna::upwind(fc.f.L1, fc.dl[0], fn.dl[0]),
                                 fvna::upwind(fc.f.L2, fc.dl[1], fn.dl[1]),
                                 fvna::upwind(fc.f.L3, fc.dl[2], fn.dl[2]), dty, fc.P, M);
     } else {
@@ -910,10 +923,10 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
     R dl1, dl2, dl3;
     dots_left(fx.w, dl1, dl2, dl3);
     // W(k).W(k+1) is the right neighbour's W(k+1).W(k)
-    R up1, up2, up3;
-    upwind_x(fx, dl1, dl2, dl3, up1, up2, up3);
+    R up1, up2, up3, nw1, nw2;
+    upwind_x(fx, dl1, dl2, dl3, up1, up2, up3, nw1, nw2);
     R PX[3], MX[3];
-    fvna::limited_flux<true>(fx, up1, up2, up3, dtx, PX, MX);
+    fvna::limited_flux<true>(fx, nw1, nw2, up1, up2, up3, dtx, PX, MX);
     const R mr0 = shl1(MX[0]), mr1 = shl1(MX[1]), mr2 = shl1(MX[2]);
     xn.q1 = fvna::sub_prod(y1q, dtxu, mr0 + PX[0]);
     xn.q2 = fvna::sub_prod(y2q, dtxu, mr1 + PX[1]);

@@ -21,8 +21,7 @@ import tempfile
 from .build import ARCH, HERE
 
 SRC = os.path.join(HERE, "csrc", "fv_step.hip")
-KERNEL = ("_ZN2fv14fv_step_kernelIfLb1ELb0EN4fvbc9EdgeDriveEEEvPKNS_8InstDescEPKNS_8WorkItem"
-          "EPKmiiPKNS_3CtlEPKNS_9SyncSlotsE")
+KERNEL = "_ZN2fv14fv_step_kernelIfLb1ELb0EN4fvbc9EdgeDriveEEE"   # (and the arguments' types)
 FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
          "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=16", "--cuda-device-only",
          "-S"]
@@ -39,10 +38,10 @@ _FIRST_ORDER = (
     "  {M}[0] = fvna::fma_(be1, w_.a1, be2 * w_.a2);\n"
     "  {M}[1] = fvna::fma_(be1, w_.w21, be2 * w_.w22);\n"
     "  {M}[2] = fvna::fma_(be3, w_.a3, fvna::fma_(be1, w_.w31, be2 * w_.w32)); }}")
-_Y_LIMITER = ("      fvna::limited_flux<false>(fc.f, fvna::upwind(fc.f.L1, fc.dl[0], fn.dl[0]),\n"
+_Y_LIMITER = ("      fvna::limited_flux<false>(fc.f, nw1, nw2, fvna::upwind(fc.f.L1, fc.dl[0], fn.dl[0]),\n"
               "                                fvna::upwind(fc.f.L2, fc.dl[1], fn.dl[1]),\n"
               "                                fvna::upwind(fc.f.L3, fc.dl[2], fn.dl[2]), dty, fc.P, M);")
-_X_LIMITER = "    fvna::limited_flux<true>(fx, up1, up2, up3, dtx, PX, MX);"
+_X_LIMITER = "    fvna::limited_flux<true>(fx, nw1, nw2, up1, up2, up3, dtx, PX, MX);"
 _X_START = "    const R ir = fvna::rcp(R(1) + y1q);\n    const R un = y2q * ir, ut = y3q * ir;"
 _Y_RIEMANN = ("      fvna::riemann(fvna::jump(bm.q1, bm.q3, bm.q2, bm.un, bm.ut, bn.q1, bn.q3, bn.q2, bn.un,\n"
               "                               bn.ut),\n"
@@ -70,7 +69,7 @@ def row_loop_counts(asm, kernel=KERNEL):
     """(VALU, transcendental, SALU) per row of the innermost loop holding the
     three unrolled rows' stores."""
     lines = asm.split("\n")
-    start = next(i for i, l in enumerate(lines) if l.startswith(kernel + ":"))
+    start = next(i for i, l in enumerate(lines) if l.startswith(kernel) and ":" in l)
     end = next(i for i in range(start, len(lines)) if lines[i].strip().startswith(".Lfunc_end"))
     body = lines[start:end]
     labels = {}
