@@ -1498,7 +1498,6 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
   // ---- reverse, segment by segment: recompute the segment's states with
   // the step kernel (each step from its logged control block) unless every
   // state was kept, then march the adjoint back over them ----
-  const bool one = ni == 1;
   int par = 0;
   for (int64_t seg = ncp - 1; seg >= 0; --seg) {
     const int64_t s0 = seg * K;
@@ -1525,8 +1524,8 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
       if (c->taylor_ring > 0)
         HIP_TRY(fv_launch_taylor_ghosts(di, ni, c->taylor_ring, 0, 0, c->stream));
       HIP_TRY(fv_launch_step(di, c->d_items, c->d_rowmask, c->n_groups(), 0, ni,
-                             one ? d_rctl + 2 * (size_t)s : nullptr, one ? d_rsync : nullptr,
-                             c->params[0].bc, c->ext_any ? 1 : 0, 0, 0, 0, c->stream));
+                             d_rctl + 2 * (size_t)s * ni, d_rsync, c->params[0].bc,
+                             c->ext_any ? 1 : 0, 0, 0, 0, c->stream));
     }
     for (int s = len - 1; s >= 0; --s) {
       // q_n as the step read it: the Taylor ghost ring of its T (a state the

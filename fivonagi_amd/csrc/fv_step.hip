@@ -539,11 +539,12 @@ using At = std::integral_constant<int, kT>;
 
 // One work item of attempt `phase` (mod 6) of an instance whose ghost cells
 // follow the boundary policy BC (apps/<app>/boundary.h).
-// kOne: the launch covers a single instance, whose control block and
-// reduction slots of this attempt are passed directly (ctl_in = its control
-// block of attempt a = ctl + a % 2, sync_in = the slots of attempt a-1 =
-// sync + (a + 2) % 3), so the fold's loads go out together with the work
-// item's instead of after the instance description's.
+// kOne: the launch covers a single instance.  The control blocks and reduction
+// slots of this attempt are passed directly (ctl_in = the first instance's
+// control block of attempt a = ctl + a % 2, sync_in = its slots of attempt a-1 =
+// sync + (a + 2) % 3; the next instance's follow two and three on), so the
+// fold's loads go out together with the work item's (kOne), or with the instance
+// description's rather than after it (16 uneven instances 53.1 -> 52.7 us).
 // kExt: some instance has a moving window or the HIFU boundary.
 //  - Moving window: the shift that follows an accepted step (moveDomain,
 //    common/main.cu:109-164) is folded into the stores: cell (i, j) of the new
@@ -582,8 +583,8 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
   double cfl_max = D.cfl_max;
   const double* dt_seq = D.dt_seq;
   fvbc::Tables tb{D.edge_c, D.edge_s, D.hifu_tab};
-  const FoldRaw<R> FR = fold_load<R>(kOne ? ctl_in : D.ctl + (phase & 1),
-                                     kOne ? sync_in : D.sync + (phase + 2) % 3);
+  const FoldRaw<R> FR = fold_load<R>(ctl_in + (kOne ? 0 : 2 * it.inst),
+                                     sync_in + (kOne ? 0 : 3 * it.inst));
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -1245,20 +1246,22 @@ void launch_step_r(bool one, bool ext, int bc, const fv::InstDesc* insts,
 }
 }  // namespace
 
-// One step attempt of every instance: n_groups workgroups, items[4 g ..] each.  ctl0/sync0: the control blocks and
-// slot sets of the only instance when n_inst == 1 (null otherwise), bc0 its
-// boundary kind; ext: some instance has a moving window, the HIFU boundary or
-// data collection; fp64: the instances are FP64; beside, collect: workgroups per
-// instance for beside_step, and how many of them collect the attempt before.
+// One step attempt of every instance: n_groups workgroups, items[4 g ..] each.
+// ctl0/sync0: the control blocks (two per instance) and slot sets (three) of the
+// instances, one instance after the other, where their descriptions point too;
+// bc0: the boundary kind of an only instance; ext: some instance has a moving
+// window, the HIFU boundary or data collection; fp64: the instances are FP64;
+// beside, collect: workgroups per instance for beside_step, and how many of them
+// collect the attempt before.
 extern "C" hipError_t fv_launch_step(const fv::InstDesc* insts, const fv::WorkItem* items,
                                      const uint64_t* rowmask, int n_groups, int phase,
                                      int n_inst, fv::Ctl* ctl0, fv::SyncSlots* sync0, int bc0,
                                      int ext, int fp64, int beside, int collect,
                                      hipStream_t stream) {
   if (n_groups <= 0) return hipSuccess;
-  const bool one = n_inst == 1 && ctl0 && sync0;
-  const fv::Ctl* c_in = one ? ctl0 + (phase & 1) : nullptr;
-  const fv::SyncSlots* s_in = one ? sync0 + (phase + 2) % 3 : nullptr;
+  const bool one = n_inst == 1;
+  const fv::Ctl* c_in = ctl0 + (phase & 1);
+  const fv::SyncSlots* s_in = sync0 + (phase + 2) % 3;
   const Beside bs{n_inst, beside, collect};
   if (fp64)
     launch_step_r<double>(one, ext != 0, bc0, insts, items, rowmask, n_groups, phase, c_in, s_in,
