@@ -57,7 +57,6 @@ __device__ __forceinline__ double rsq(double x) {
 __device__ __forceinline__ float fma_(float a, float b, float c) { return fmaf(a, b, c); }
 __device__ __forceinline__ double fma_(double a, double b, double c) { return fma(a, b, c); }
 __device__ __forceinline__ float min_(float a, float b) { return fminf(a, b); }
-__device__ __forceinline__ double min_(double a, double b) { return fmin(a, b); }
 
 // a + b never contracted with a product feeding it, so that when a is the
 // neighbouring lane's value its cross-lane move can fold into this add
@@ -81,10 +80,14 @@ __device__ __forceinline__ R sub_prod(R q, R d, R flux) {
 __device__ __forceinline__ float fmax2(float a, float b) {
   return __builtin_amdgcn_fmed3f(a, b, 3.4028234663852886e38f);
 }
-__device__ __forceinline__ double fmax2(double a, double b) { return fmax(a, b); }
+__device__ __forceinline__ double fmax2(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+// (the FP64 form is the bare instruction for the same reason)
 // clamp to [0, 1]; a NaN gives 0
 __device__ __forceinline__ float clamp01(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 1.0f); }
-__device__ __forceinline__ double clamp01(double x) { return fmin(fmax(x, 0.0), 1.0); }
 
 // Waves of one interface in (density, normal, tangential) component order.
 // W1 = a1*(1, L1, A1), W2 = a2*(1, L2, A2), W3 = (0, 0, a3).
@@ -183,6 +186,21 @@ __device__ __forceinline__ R dot2(const WavesT<R>& a, const WavesT<R>& b) {
   return fma_(b.a2, a.a2, fma_(b.w22, a.w22, b.w32 * a.w32));
 }
 
+// The limiter of a ratio r: t = (1+r)/4, mn = min(t, r), h = clamp(mn).  FP64
+// (h alone): 1/4 as a scalar operand of the multiply-add -- the compiler's form
+// adds into a register pair set to 1/4 first -- and the clamp as the minimum's
+// output modifier, without a canonicalising v_max before it.
+__device__ __forceinline__ void limit_half(float r, float& t, float& mn, float& h) {
+  t = fma_(0.25f, r, 0.25f);
+  mn = min_(t, r);
+  h = clamp01(mn);
+}
+__device__ __forceinline__ void limit_half(double r, double& t, double& mn, double& h) {
+  asm("v_fma_f64 %0, %2, %3, %3\n\tv_min_f64 %1, %0, %2 clamp"
+      : "=&v"(t), "=v"(h) : "v"(r), "s"(0.25));
+  mn = h;
+}
+
 // |W_1|^2, |W_2|^2
 template <typename R>
 __device__ __forceinline__ void norms(const WavesT<R>& w, R& n1, R& n2) {
@@ -233,9 +251,7 @@ __device__ __forceinline__ void limited_flux(const IfaceT<R>& f, R n1, R n2, R u
   for (int p = 0; p < 3; ++p) {
     v.rn[p] = rcp(n[p]);
     v.r[p] = up[p] * v.rn[p];
-    v.t[p] = fma_(R(0.25), v.r[p], R(0.25));
-    v.mn[p] = min_(v.t[p], v.r[p]);
-    v.h[p] = clamp01(v.mn[p]);
+    limit_half(v.r[p], v.t[p], v.mn[p], v.h[p]);
     const R s = fabs(L[p]);
     v.om[p] = fma_(-s, dtd, R(1));
     v.g[p] = s * v.om[p];
