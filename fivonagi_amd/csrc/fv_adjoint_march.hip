@@ -671,6 +671,26 @@ __global__ __launch_bounds__(64) void adj_segment_kernel(const AdjDesc* __restri
   for (int f = 0; f < 3; ++f) rdesc[e].q[0][f] = q + f * n;
 }
 
+// After a forward run that kept its state in the history alone: the last state
+// into the buffer the settled control block names.
+__global__ __launch_bounds__(256) void adj_back_kernel(const InstDesc* __restrict__ insts,
+                                                       int n_inst, int phase) {
+  for (int k = blockIdx.y; k < n_inst; k += gridDim.y) {
+    const InstDesc& D = insts[k];
+    const Ctl& P = D.ctl[(phase + 1) & 1];
+    const int64_t t = P.n_acc - D.log_base;
+    if (!D.hist_state || t < 1) continue;
+    const size_t n = (size_t)D.nx * (size_t)D.ny;
+    const float* s = D.hist + (size_t)t * 3 * n;
+    for (int f = 0; f < 3; ++f) {
+      float* q = D.q[P.cur][f];
+      for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
+           e += (size_t)gridDim.x * blockDim.x)
+        q[e] = s[f * n + e];
+    }
+  }
+}
+
 // After the forward run: steps the log does not hold (none, by then).
 __global__ __launch_bounds__(256) void adj_log_kernel(const AdjDesc* __restrict__ ds, int n_inst,
                                                       int nsteps) {
@@ -730,6 +750,13 @@ extern "C" hipError_t fv_adj_segment(const fv::AdjDesc* ds, int n_inst, int s0, 
                                      fv::Ctl* rctl, hipStream_t s) {
   hipLaunchKernelGGL(fv::adj_segment_kernel, dim3((len * n_inst + 63) / 64), dim3(64), 0, s, ds,
                      n_inst, s0, len, keep_all, first, rdesc, rctl);
+  return hipGetLastError();
+}
+
+extern "C" hipError_t fv_adj_back(const fv::InstDesc* insts, int n_inst, size_t max_cells,
+                                  int phase, hipStream_t s) {
+  hipLaunchKernelGGL(fv::adj_back_kernel, adj_grid(max_cells, n_inst), dim3(256), 0, s, insts,
+                     n_inst, phase);
   return hipGetLastError();
 }
 

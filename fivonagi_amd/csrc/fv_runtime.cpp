@@ -48,6 +48,8 @@ extern "C" hipError_t fv_adj_begin(const fv::AdjDesc* ds, int n_inst, size_t max
 extern "C" hipError_t fv_adj_segment(const fv::AdjDesc* ds, int n_inst, int s0, int len,
                                      int keep_all, fv::StateSlot kept0, fv::InstDesc* rdesc,
                                      fv::Ctl* rctl, hipStream_t s);
+extern "C" hipError_t fv_adj_back(const fv::InstDesc* insts, int n_inst, size_t max_cells,
+                                  int phase, hipStream_t s);
 extern "C" hipError_t fv_adj_log(const fv::AdjDesc* ds, int n_inst, int nsteps, hipStream_t s);
 extern "C" hipError_t fv_adj_end(const fv::AdjDesc* ds, int n_inst, size_t max_cells, int par,
                                  hipStream_t s);
@@ -1456,6 +1458,7 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
         d.dt_seq_len = 0;
         d.ctl_log = nullptr;
         d.hist = nullptr;
+        d.hist_state = 0;
         d.measure = nullptr;
         d.stage = nullptr;
         d.md_on = 0;
@@ -1470,12 +1473,16 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
   // ---- forward: log the control block of every accepted step and keep every
   // state, or one every K steps and the last (the extended step kernel also
   // stores its output into the history slot of its step) ----
+  bool back = false;                   // states to be put back where the context has them
   for (int k = 0; k < ni; ++k) {
     c->desc[k].ctl_log = ad[k].ctl_log;
     c->desc[k].log_base = ctl[k].n_acc;
     c->desc[k].log_len = nsteps;
     c->desc[k].hist = ad[k].kept;
     c->desc[k].hist_every = keep_all ? 1 : K;
+    // (a Taylor state has its ghost ring behind its fields)
+    c->desc[k].hist_state = keep_all && c->params[k].bc != FIVONAGI_BC_TAYLOR ? 1 : 0;
+    back = back || c->desc[k].hist_state;
   }
   int rc = upload_tables(c);
   c->keep_hist = true;
@@ -1486,13 +1493,22 @@ int fivonagi_step_adjoint(fivonagi_ctx* c, int64_t nsteps, const fivonagi_object
     rc = fivonagi_step(c, nsteps);
   }
   c->keep_hist = false;
+  int rc3 = 0;
+  if (back && (rc3 = read_ctls(c, ctl)) == 0) {
+    // also after a run that stopped with an error
+    const hipError_t e =
+        fv_adj_back(c->d_desc, ni, max_cells, (int)(c->attempts % 6), c->stream);
+    if (e != hipSuccess) rc3 = hip_fail(e, "state put back");
+  }
   for (int k = 0; k < ni; ++k) {
     c->desc[k].ctl_log = nullptr;
     c->desc[k].hist = nullptr;
+    c->desc[k].hist_state = 0;
   }
   int rc2 = upload_tables(c);
   if (rc) return rc;
   if (rc2) return rc2;
+  if (rc3) return rc3;
   HIP_TRY(fv_adj_log(d_ad, ni, (int)nsteps, c->stream));
 
   // ---- reverse, segment by segment: recompute the segment's states with

@@ -68,7 +68,8 @@ struct InstDesc {
   int64_t log_base, log_len;
   float* hist;          // when set (FP32): the state after accepted step t = n_acc - log_base,
                         // t in [1, log_len], every hist_every steps and after the last, slot
-                        // ceil(t / hist_every) = 3 grids (the extended step kernel)
+                        // ceil(t / hist_every) = 3 grids (the extended step kernel); slot 0
+                        // the state at log_base
   double dx, dy, delta, cfl_max, cfl_wish, omega;
   double inv_dx, inv_dy;     // 1/dx, 1/dy
   double dif_x, dif_y;       // delta/dx^2, delta/dy^2
@@ -105,7 +106,9 @@ struct InstDesc {
   double eta;           // cells per length unit
   int32_t mic[4];
   // taylor-angle-xy cut: i in [icenter - cut_half, icenter + cut_half]
-  int32_t cut_half, pad6;
+  int32_t cut_half;
+  int32_t hist_state;   // the history holds the state itself (every step kept, no ghost ring):
+                        // steps go from slot to slot and leave q alone
   double tan_theta;
   // FP64 instances (the reference's PRECISION=2): state, tables and the cfl
   // reduction in double

@@ -353,3 +353,23 @@ def test_item_heights_do_not_change_the_gradient(kind):
         assert abs(J - res[0][0]) <= 1e-13 * res[0][0]
         assert np.array_equal(ga, res[0][1]) and np.array_equal(gp, res[0][2])
         assert np.array_equal(lam, res[0][3])
+
+
+@pytest.mark.parametrize("K", [1, 4])
+def test_state_after_a_forward_run_that_stops(K):
+    """A prescribed dt sequence that ends inside the forward run fails the call;
+    the context then holds the state after the steps that were taken, bit for
+    bit that of plain steps (K = 1 keeps the running state in its history and
+    puts it back)."""
+    _, _, _, prob = case(5)
+    got = []
+    for adjoint in (True, False):
+        with fa.Context(prob) as ctx:
+            ctx.set_dt_sequence(0, np.full(7, 0.04))
+            with pytest.raises(RuntimeError):
+                if adjoint:
+                    ctx.step_adjoint(12, BOX, checkpoint_every=K)
+                else:
+                    ctx.step(12)
+            got.append(ctx.collect(0)[0])
+    assert np.array_equal(got[0], got[1]) and np.abs(got[0]).max() > 0
