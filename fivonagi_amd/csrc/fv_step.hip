@@ -1141,7 +1141,7 @@ __global__ __launch_bounds__(64) void fv_targets_kernel(const InstDesc* __restri
 
 // Data collection of the attempt of phase `phase` alone, run after its launch
 // (the last attempt of a run of launches; the others' comes with the launch
-// after them, ahead_of_step).  blockIdx.y = instance; threads cover the columns.
+// after them, beside_step).  blockIdx.y = instance; threads cover the columns.
 __global__ __launch_bounds__(256) void fv_collect_kernel(const InstDesc* __restrict__ insts,
                                                          int phase) {
   const InstDesc& D = insts[blockIdx.y];
