@@ -392,17 +392,26 @@ void build_work(const std::vector<fivonagi_params>& ps, const std::vector<int>& 
   out.rotate_used = rotate && skew > 0.0f;
   std::vector<Group> groups;
   if (running) {
-    // the least steps per wave whose groups are all resident at once (to 0.4%)
-    const long target = std::max(1L, cus * per_simd);
-    auto fits = [&](double c) {
-      return cut_running(strips, c, skew, levels, [](const Group&) {}) <= target;
+    // the least steps per wave whose groups are all resident at once (to 0.4%).
+    // A group holds four strips at most, so with very many strips no height
+    // makes them fit: then the least whose groups take as few rounds of
+    // residency as whole strips, one to a wave, do (from `whole` steps on even
+    // the lowest level holds any strip in one wave)
+    auto groups_at = [&](double c) {
+      return cut_running(strips, c, skew, levels, [](const Group&) {});
     };
+    int tallest = 0;
+    for (const auto& s : strips) tallest = std::max(tallest, s.rows);
+    const double whole = (tallest + kTail) / level_weight(levels - 1, levels, skew);
+    const long room = std::max(1L, cus * per_simd);
+    const long target = room * ((groups_at(whole) + room - 1) / room);
+    auto fits = [&](double c) { return c >= whole || groups_at(c) <= target; };
     double c = kSeamRows;
     if (asked > 0.0) {
       c = std::max<double>(kSeamRows, rows / asked);
     } else if (!fits(c)) {
       double lo = std::max(c, rows / (double)(target * fv::kGroupWaves)), hi = 1.05 * lo;
-      while (!fits(hi)) { lo = hi; hi *= 1.25; }
+      while (!fits(hi)) { lo = hi; hi = std::min(1.25 * hi, whole); }
       while (hi - lo > 0.004 * lo) {
         const double mid = 0.5 * (lo + hi);
         if (fits(mid)) hi = mid;
