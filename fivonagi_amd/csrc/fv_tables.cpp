@@ -362,12 +362,16 @@ void build_work(const std::vector<fivonagi_params>& ps, const std::vector<int>& 
   // the strips, with their lane masks
   std::vector<Piece> strips;
   long bytes = 0, waves = 0;               // waves: of the in-step cut
-  double rows = 0.0, asked = 0.0;
+  double rows = 0.0;
+  int asked = 0;                           // rows per wave all instances ask for
+  bool alike = true;
   for (int k = 0; k < (int)ps.size(); ++k) {
     const auto& p = ps[k];
     waves += strips_of(p) * in_step_items(p, auto_h);
     rows += (double)strips_of(p) * p.ny;
-    if (p.rows_per_wave > 0) asked += (double)strips_of(p) * p.ny / p.rows_per_wave;
+    const int a = std::max(0, p.rows_per_wave);
+    if (k == 0) asked = a;
+    alike = alike && a == asked;
     bytes += (long)cell_bytes * p.nx * p.ny;
     for (int s = 0; s < (int)strips_of(p); ++s) {
       const int x0 = s * fv::kStripCols;
@@ -388,6 +392,9 @@ void build_work(const std::vector<fivonagi_params>& ps, const std::vector<int>& 
     skew = (levels >= 4 && levels == per_simd) ? kAutoSkew : 0.0f;
     running = bytes <= kRunningBytes;
   }
+  // cut A marches every strip alike: where instances ask for different rows per
+  // wave, cut B gives each its own
+  running = running && alike;
   out.skew_used = skew;
   out.rotate_used = rotate && skew > 0.0f;
   std::vector<Group> groups;
@@ -407,8 +414,8 @@ void build_work(const std::vector<fivonagi_params>& ps, const std::vector<int>& 
     const long target = room * ((groups_at(whole) + room - 1) / room);
     auto fits = [&](double c) { return c >= whole || groups_at(c) <= target; };
     double c = kSeamRows;
-    if (asked > 0.0) {
-      c = std::max<double>(kSeamRows, rows / asked);
+    if (asked > 0) {
+      c = std::max(kSeamRows, asked);
     } else if (!fits(c)) {
       double lo = std::max(c, rows / (double)(target * fv::kGroupWaves)), hi = 1.05 * lo;
       while (!fits(hi)) { lo = hi; hi = std::min(1.25 * hi, whole); }
