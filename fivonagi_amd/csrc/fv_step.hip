@@ -1155,8 +1155,8 @@ __global__ __launch_bounds__(256) void fv_collect_kernel(const InstDesc* __restr
 // Ghost ring of the Taylor-shock instances for the attempt of phase `phase`
 // (the first attempt of a run of launches, or every one where a buffer has no
 // ring: then into the grid).  settle: instead, after that phase's last attempt:
-// where it was not accepted, the grid's ghost cells take the values it read, as
-// if they had been written there.  blockIdx.y = instance; the ring is
+// where the last attempt an instance ran was not accepted, the grid's ghost
+// cells take the values it read, as if they had been written there.  blockIdx.y = instance; the ring is
 // enumerated by a flat index.
 __global__ __launch_bounds__(256) void fv_taylor_ghost_kernel(const InstDesc* __restrict__ insts,
                                                              int phase, int settle) {
@@ -1176,7 +1176,9 @@ __global__ __launch_bounds__(256) void fv_taylor_ghost_kernel(const InstDesc* __
       state = F.state;
       P = F.p;
     }
-    if (state == kFoldReject || state == kFoldError)
+    // (an instance that an error stopped earlier in the run: still the ghost
+    // cells of the attempt that failed, whose control block it keeps)
+    if (state == kFoldReject || state == kFoldError || (state == kFoldIdle && P.err == 2))
       taylor_ring(D, P.T, P.cur, P.mdx, P.mdy, false, k0, dk);
     return;
   }
