@@ -378,7 +378,9 @@ int write_ctls(fivonagi_ctx* c, const std::vector<fv::Ctl>& in) {
 // the last of a run of launches.  What surrounds the step -- the Taylor ghost
 // ring the attempt reads, and its data collection -- is launched by itself only
 // there; between them each step launch collects the attempt before it and makes
-// the ring of the one after it (fv_step.hip, beside_step).
+// the ring of the one after it (fv_step.hip, beside_step).  Where a Taylor
+// instance has no ring its ghost cells go into the grid before each attempt, and
+// the attempt before must have been collected by then: by a launch of its own.
 hipError_t launch_phase(fivonagi_ctx* c, int phase, bool begin, bool end) {
   if (c->taylor_ring > 0 && (begin || !c->ring_all)) {
     hipError_t e =
@@ -386,13 +388,14 @@ hipError_t launch_phase(fivonagi_ctx* c, int phase, bool begin, bool end) {
     if (e != hipSuccess) return e;
   }
   const int threads = fv::kLanes * fv::kGroupWaves;
-  const int collect = begin ? 0 : (c->collect_nx + threads - 1) / threads;
+  const bool collect_alone = c->taylor_ring > 0 && !c->ring_all;
+  const int collect = begin || collect_alone ? 0 : (c->collect_nx + threads - 1) / threads;
   const int ring = end ? 0 : (c->taylor_ring + threads - 1) / threads;
   hipError_t e = fv_launch_step(c->d_desc, c->d_items, c->d_rowmask, c->n_groups(),
                                 phase, c->n_inst, c->d_ctl, c->d_sync, c->params[0].bc,
                                 c->ext_any || c->keep_hist ? 1 : 0, c->fp64 ? 1 : 0,
                                 collect + ring, collect, c->stream);
-  if (e == hipSuccess && end && c->collect_nx > 0)
+  if (e == hipSuccess && (end || collect_alone) && c->collect_nx > 0)
     e = fv_launch_collect(c->d_desc, c->n_inst, c->collect_nx, phase, c->stream);
   return e;
 }

@@ -1,0 +1,154 @@
+// runtime_check.cpp -- the host side of the runtime (fivonagi_amd/csrc/
+// fv_runtime.cpp) on a stand-in for the HIP runtime (hip/hip_runtime.h here),
+// one check per run (argv[1]).  The kernels are stand-ins too: a step attempt is
+// always accepted.  Prints "ok", or what was wrong.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <cstring>
+#include <string>
+
+#include "../../fivonagi_amd/csrc/fv_adjoint.h"
+#include "../../fivonagi_amd/csrc/fv_types.h"
+#include "../../include/fivonagi.h"
+
+namespace {
+std::string trace;                       // launches: s = step (and its collect), c = collection
+void note(char what, int phase, int collect) {
+  trace += what + std::to_string(phase) + (what == 's' && collect > 0 ? "+c " : " ");
+}
+}  // namespace
+
+extern "C" {
+hipError_t fv_launch_step(const fv::InstDesc* d, const fv::WorkItem*, const uint64_t*, int,
+                          int phase, int n, fv::Ctl*, fv::SyncSlots*, int, int, int, int,
+                          int collect, hipStream_t) {
+  fake::launch([=] {
+    note('s', phase, collect);
+    for (int k = 0; k < n; ++k) {
+      fv::Ctl& o = d[k].ctl[(phase + 1) & 1];
+      o = d[k].ctl[phase & 1];
+      if (o.n_acc >= o.target_acc || !(o.T < o.T_stop)) continue;
+      o.T += o.dt;
+      o.cur ^= 1;
+      ++o.n_acc;
+      ++o.n_att;
+    }
+  });
+  return hipSuccess;
+}
+hipError_t fv_launch_settle(const fv::InstDesc* d, int n, int phase, fv::Ctl* mirror, hipStream_t) {
+  fake::launch([=] {
+    for (int k = 0; k < n; ++k) {
+      d[k].ctl[(phase + 1) & 1] = d[k].ctl[phase & 1];
+      if (mirror) mirror[k] = d[k].ctl[phase & 1];
+    }
+  });
+  return hipSuccess;
+}
+hipError_t fv_launch_targets(const fv::InstDesc* d, int n, int phase, const int64_t* targets,
+                             int64_t target, double T_stop, hipStream_t) {
+  fake::launch([=] {
+    for (int k = 0; k < n; ++k) {
+      d[k].ctl[phase & 1].target_acc = targets ? targets[k] : target;
+      d[k].ctl[phase & 1].T_stop = T_stop;
+    }
+  });
+  return hipSuccess;
+}
+hipError_t fv_launch_collect(const fv::InstDesc*, int, int, int phase, hipStream_t) {
+  fake::launch([=] { note('c', phase, 0); });
+  return hipSuccess;
+}
+hipError_t fv_launch_taylor_ghosts(const fv::InstDesc*, int, int, int, int, hipStream_t) {
+  return hipSuccess;
+}
+hipError_t fv_step_waves_per_cu(int* w, int fp64) { *w = fp64 ? 8 : 16; return hipSuccess; }
+hipError_t fv_adj_occupancy(int* w) { *w = 8; return hipSuccess; }
+hipError_t fv_scratch_get(void**, size_t*) { return hipErrorInvalidValue; }
+// (no check runs the adjoint)
+hipError_t fv_adj_reverse(const fv::AdjDesc*, const fv::AdjItem*, const int32_t*, int, int,
+                          fv::StateSlot, fv::StateSlot, int, int, hipStream_t) { return 1; }
+hipError_t fv_adj_begin(const fv::AdjDesc*, int, size_t, int, int, fv::SyncSlots*, int,
+                        hipStream_t) { return 1; }
+hipError_t fv_adj_segment(const fv::AdjDesc*, int, int, int, int, fv::StateSlot, fv::InstDesc*,
+                          fv::Ctl*, hipStream_t) { return 1; }
+hipError_t fv_adj_back(const fv::InstDesc*, int, size_t, int, hipStream_t) { return 1; }
+hipError_t fv_adj_log(const fv::AdjDesc*, int, int, hipStream_t) { return 1; }
+hipError_t fv_adj_end(const fv::AdjDesc*, int, size_t, int, hipStream_t) { return 1; }
+}
+
+namespace {
+
+#define EXPECT(cond, ...)                                    \
+  do {                                                       \
+    if (!(cond)) {                                           \
+      std::printf("line %d: %s: ", __LINE__, #cond);         \
+      std::printf(__VA_ARGS__);                              \
+      std::printf("\n");                                     \
+      return 1;                                              \
+    }                                                        \
+  } while (0)
+
+fivonagi_params grid(int nx, int ny, int bc = FIVONAGI_BC_ZEROGRAD) {
+  fivonagi_params p;
+  std::memset(&p, 0, sizeof(p));
+  p.nx = nx; p.ny = ny;
+  p.dx = p.dy = 0.05;
+  p.beta = 3.5; p.delta = 1e-4;
+  p.cfl_max = 1.0; p.cfl_wish = 0.9;
+  p.dt0 = 0.005;
+  p.bc = bc;
+  p.cfl_mode = FIVONAGI_CFL_ALL;
+  return p;
+}
+
+fivonagi_ctx* context(const std::vector<fivonagi_params>& ps) {
+  static std::vector<float> q;                 // (of a large grid nothing is read)
+  size_t n = 0;
+  for (const auto& p : ps) n = std::max(n, (size_t)p.nx * p.ny);
+  if (4 * n < fake::kLarge) q.assign(n, 0.25f);
+  std::vector<const float*> host(3 * ps.size(), q.data());
+  static const float some = 0.f;
+  if (4 * n >= fake::kLarge) host.assign(3 * ps.size(), &some);
+  fivonagi_ctx* c = nullptr;
+  if (fivonagi_init(&c, ps.data(), (int)ps.size(), host.data()) != 0) {
+    std::printf("init: %s\n", fivonagi_last_error());
+    std::exit(1);
+  }
+  return c;
+}
+
+}  // namespace
+
+// A Taylor field that leaves no room for its ghost ring (4 GiB): the cells are
+// written into the grid before each attempt, so the attempt before it must have
+// been collected by then.
+static int check_collect_without_ring() {
+  for (int nx : {64, 32768}) {
+    fivonagi_ctx* c = context({grid(nx, nx, FIVONAGI_BC_TAYLOR)});
+    fivonagi_collect_opts o;
+    std::memset(&o, 0, sizeof(o));
+    o.eta = 1.0;
+    EXPECT(fivonagi_set_collect(c, 0, &o) == 0, "%s", fivonagi_last_error());
+    trace.clear();
+    EXPECT(fivonagi_enqueue(c, 6) == 0, "%s", fivonagi_last_error());
+    const char* want = nx == 64 ? "s0 s1+c s2+c s3+c s4+c s5+c c5 "
+                                : "s0 c0 s1 c1 s2 c2 s3 c3 s4 c4 s5 c5 ";
+    EXPECT(trace == want, "%d: %s", nx, trace.c_str());
+    fivonagi_destroy(c);
+  }
+  return 0;
+}
+
+int main(int argc, char** argv) {
+  const std::string name = argc > 1 ? argv[1] : "";
+  int rc = 1;
+  if (name == "collect_without_ring") rc = check_collect_without_ring();
+  if (rc == 0 && !fake::st().blocks.empty()) {
+    std::printf("%zu blocks not freed\n", fake::st().blocks.size());
+    rc = 1;
+  }
+  if (rc == 0) std::printf("ok\n");
+  return rc;
+}
