@@ -554,12 +554,16 @@ int download(fivonagi_ctx* c, const std::vector<Span>& spans) {
   }
   if (total <= kThreadBytes) {
     size_t off = 0;
+    hipError_t e = hipSuccess;
     for (const Span& s : spans) {
-      if (s.bytes)
-        HIP_TRY(hipMemcpyAsync(stage.p + off, s.src, s.bytes, hipMemcpyDeviceToHost, c->stream));
+      if (s.bytes && e == hipSuccess)
+        e = hipMemcpyAsync(stage.p + off, s.src, s.bytes, hipMemcpyDeviceToHost, c->stream);
       off += s.bytes;
     }
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    // waited for also after a refused copy: those before it write the buffer
+    const hipError_t es = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = es;
+    if (e != hipSuccess) return hip_fail(e, "download");
     c->targets_pending = false;
     off = 0;
     for (const Span& s : spans) {

@@ -33,6 +33,7 @@ struct State {
   std::recursive_mutex mu;
   int device = 0;
   Stream null_stream{0, {}};
+  std::vector<Stream*> streams;
   Stream* capturing = nullptr;                 // the stream under capture, by anyone
   Graph* into = nullptr;
   std::map<void*, size_t> blocks;
@@ -106,10 +107,19 @@ inline hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) {
 inline hipError_t hipMemset(void* d, int v, size_t n) { return hipMemsetAsync(d, v, n, nullptr); }
 
 inline hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  FAKE_LOCK;
   *s = new fake::Stream{fake::st().device, {}};
+  fake::st().streams.push_back(*s);
   return hipSuccess;
 }
-inline hipError_t hipStreamDestroy(hipStream_t s) { delete s; return hipSuccess; }
+inline hipError_t hipStreamDestroy(hipStream_t s) {
+  FAKE_LOCK;
+  auto& v = fake::st().streams;
+  for (size_t k = 0; k < v.size(); ++k)
+    if (v[k] == s) v.erase(v.begin() + k);
+  delete s;
+  return hipSuccess;
+}
 inline hipError_t hipStreamSynchronize(hipStream_t s) {
   FAKE_LOCK;
   if (!s) s = &fake::st().null_stream;

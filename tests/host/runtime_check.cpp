@@ -141,10 +141,32 @@ static int check_collect_without_ring() {
   return 0;
 }
 
+// A download whose second copy is refused: when the call returns, nothing of it
+// may still write the staging buffer, which another context may have by then.
+static int check_download_error() {
+  for (int nx : {100, 1500}) {                 // one wait; a ring of slots
+    fivonagi_ctx* c = context({grid(nx, nx)});
+    EXPECT(fivonagi_step(c, 1) == 0, "%s", fivonagi_last_error());
+    std::vector<float> q(3 * (size_t)nx * nx);
+    float* f[3] = {q.data(), q.data() + (size_t)nx * nx, q.data() + 2 * (size_t)nx * nx};
+    fake::st().fail_copy = 1;
+    EXPECT(fivonagi_collect(c, 0, f[0], f[1], f[2], nullptr, nullptr, nullptr, nullptr) != 0, "%d",
+           nx);
+    for (const auto* s : fake::st().streams)
+      EXPECT(s->queued.empty(), "%d: %zu copies in flight", nx, s->queued.size());
+    fake::st().fail_copy = -1;
+    EXPECT(fivonagi_collect(c, 0, f[0], f[1], f[2], nullptr, nullptr, nullptr, nullptr) == 0, "%s",
+           fivonagi_last_error());
+    fivonagi_destroy(c);
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   int rc = 1;
   if (name == "collect_without_ring") rc = check_collect_without_ring();
+  if (name == "download_error") rc = check_download_error();
   if (rc == 0 && !fake::st().blocks.empty()) {
     std::printf("%zu blocks not freed\n", fake::st().blocks.size());
     rc = 1;
