@@ -573,8 +573,18 @@ int download(fivonagi_ctx* c, const std::vector<Span>& spans) {
     return 0;
   }
   constexpr int kSlots = kStageSlots;
-  for (hipEvent_t& e : c->stage_ev)
-    if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  {
+    // events belong to the device that is current when they are made, and record
+    // only streams of theirs: the context's, whichever the caller's is now
+    int dev = c->device;
+    HIP_TRY(hipGetDevice(&dev));
+    if (dev != c->device) HIP_TRY(hipSetDevice(c->device));
+    hipError_t e = hipSuccess;
+    for (hipEvent_t& ev : c->stage_ev)
+      if (!ev && e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (dev != c->device) (void)hipSetDevice(dev);
+    if (e != hipSuccess) return hip_fail(e, "hipEventCreate (download)");
+  }
   constexpr size_t slot = kStageBytes / kSlots;
   std::vector<Span> chunks;
   for (const Span& s : spans)

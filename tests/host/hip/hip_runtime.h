@@ -31,7 +31,6 @@ struct Graph { std::vector<std::function<void()>> nodes; };
 constexpr size_t kLarge = 256u << 20;          // from this size on memory is never touched
 struct State {
   std::recursive_mutex mu;
-  int device = 0;
   Stream null_stream{0, {}};
   std::vector<Stream*> streams;
   Stream* capturing = nullptr;                 // the stream under capture, by anyone
@@ -41,6 +40,7 @@ struct State {
   std::vector<float> elapsed;                  // hipEventElapsedTime's answers, in turn
   size_t asked = 0;
 };
+inline int& device() { static thread_local int d = 0; return d; }
 inline State& st() { static State s; return s; }
 inline void launch(std::function<void()> f) {
   std::lock_guard<std::recursive_mutex> lk(st().mu);
@@ -61,8 +61,8 @@ enum hipStreamCaptureStatus { hipStreamCaptureStatusNone, hipStreamCaptureStatus
 
 inline const char* hipGetErrorString(hipError_t) { return "fake"; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
-inline hipError_t hipGetDevice(int* d) { *d = fake::st().device; return hipSuccess; }
-inline hipError_t hipSetDevice(int d) { FAKE_LOCK; fake::st().device = d; return hipSuccess; }
+inline hipError_t hipGetDevice(int* d) { *d = fake::device(); return hipSuccess; }
+inline hipError_t hipSetDevice(int d) { fake::device() = d; return hipSuccess; }
 inline hipError_t hipDeviceGetAttribute(int* v, int, int) { *v = 256; return hipSuccess; }
 inline hipError_t hipMemGetInfo(size_t* f, size_t* t) { *f = *t = (size_t)1 << 38; return hipSuccess; }
 
@@ -108,7 +108,7 @@ inline hipError_t hipMemset(void* d, int v, size_t n) { return hipMemsetAsync(d,
 
 inline hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
   FAKE_LOCK;
-  *s = new fake::Stream{fake::st().device, {}};
+  *s = new fake::Stream{fake::device(), {}};
   fake::st().streams.push_back(*s);
   return hipSuccess;
 }
@@ -158,7 +158,7 @@ inline hipError_t hipGraphDestroy(hipGraph_t g) { delete g; return hipSuccess; }
 inline hipError_t hipGraphExecDestroy(hipGraphExec_t e) { delete e; return hipSuccess; }
 
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
-  *e = new fake::Event{fake::st().device};
+  *e = new fake::Event{fake::device()};
   return hipSuccess;
 }
 inline hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }

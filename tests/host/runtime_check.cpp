@@ -162,11 +162,30 @@ static int check_download_error() {
   return 0;
 }
 
+// A download by a caller whose current device is another than the context's
+// (every launch before it done: only copies are left to do).
+static int check_download_device() {
+  for (int nx : {100, 1500}) {
+    fivonagi_ctx* c = context({grid(nx, nx)});
+    EXPECT(fivonagi_step(c, 1) == 0, "%s", fivonagi_last_error());
+    std::vector<float> q((size_t)nx * nx);
+    fake::device() = 1;
+    EXPECT(fivonagi_collect(c, 0, q.data(), q.data(), q.data(), nullptr, nullptr, nullptr,
+                            nullptr) == 0, "%d: %s", nx, fivonagi_last_error());
+    EXPECT(fake::device() == 1, "device %d", fake::device());
+    EXPECT(q[5] == 0.25f, "%g", (double)q[5]);
+    fake::device() = 0;
+    fivonagi_destroy(c);
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   int rc = 1;
   if (name == "collect_without_ring") rc = check_collect_without_ring();
   if (name == "download_error") rc = check_download_error();
+  if (name == "download_device") rc = check_download_device();
   if (rc == 0 && !fake::st().blocks.empty()) {
     std::printf("%zu blocks not freed\n", fake::st().blocks.size());
     rc = 1;
