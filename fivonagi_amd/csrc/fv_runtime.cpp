@@ -507,9 +507,14 @@ int check_ctx(fivonagi_ctx* c, int inst) {
 }
 
 // Stop conditions of the attempts launched from now on: an instance runs
-// while n_acc < tgt[k] and T < T_stop.  One launch, no host round trip.
+// while n_acc < tgt[k] and T < T_stop.  One launch, no host round trip.  Refused
+// on a stream under capture, whose replays would set them again.
 int write_targets(fivonagi_ctx* c, const std::vector<int64_t>& tgt,
                   double T_stop = std::numeric_limits<double>::infinity()) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(c->stream, &cap));
+  if (cap != hipStreamCaptureStatusNone)
+    return hip_fail(hipErrorStreamCaptureUnsupported, "stop conditions on a stream under capture");
   const int64_t* list = nullptr;
   if (c->n_inst > 1) {
     if (c->targets_pending) HIP_TRY(hipStreamSynchronize(c->stream));

@@ -180,12 +180,40 @@ static int check_download_device() {
   return 0;
 }
 
+// Attempts enqueued while the caller captures the stream: accepted where they
+// are launches alone; refused where the stop conditions have to be set first,
+// which the replays would set again, from host memory used for other targets by
+// then.
+static int check_enqueue_under_capture() {
+  for (int n : {1, 3}) {
+    fivonagi_ctx* c = context(std::vector<fivonagi_params>(n, grid(64, 64)));
+    hipStream_t s;
+    (void)hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+    EXPECT(fivonagi_set_stream(c, s) == 0, "%s", fivonagi_last_error());
+    for (bool first : {true, false}) {
+      hipGraph_t g;
+      (void)hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
+      const int rc = fivonagi_enqueue(c, 3);
+      (void)hipStreamEndCapture(s, &g);
+      EXPECT((rc != 0) == first, "%d instances, first %d: %d", n, first, rc);
+      EXPECT(g->nodes.size() == (first ? 0u : 3u), "%zu nodes", g->nodes.size());
+      (void)hipGraphDestroy(g);
+      if (first) EXPECT(fivonagi_enqueue(c, 3) == 0, "%s", fivonagi_last_error());
+    }
+    EXPECT(fivonagi_set_stream(c, nullptr) == 0, "%s", fivonagi_last_error());
+    (void)hipStreamDestroy(s);
+    fivonagi_destroy(c);
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   int rc = 1;
   if (name == "collect_without_ring") rc = check_collect_without_ring();
   if (name == "download_error") rc = check_download_error();
   if (name == "download_device") rc = check_download_device();
+  if (name == "enqueue_under_capture") rc = check_enqueue_under_capture();
   if (rc == 0 && !fake::st().blocks.empty()) {
     std::printf("%zu blocks not freed\n", fake::st().blocks.size());
     rc = 1;
