@@ -378,7 +378,8 @@ class Context:
         _check(load().fivonagi_set_skew(self._h, C.c_double(skew), int(bool(rotate))))
 
     def autotune(self, trial_steps=20):
-        """Pick the rows per wave with the fastest step; state is unchanged."""
+        """Pick the work split with the fastest step (its rows per wave are
+        returned); state is unchanged."""
         h = C.c_int32()
         _check(load().fivonagi_autotune(self._h, int(trial_steps), C.byref(h)))
         return h.value

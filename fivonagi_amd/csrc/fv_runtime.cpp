@@ -178,6 +178,7 @@ struct fivonagi_ctx {
   hipStream_t stream = nullptr;
   int n_inst = 0;
   std::vector<fivonagi_params> params;
+  std::vector<int32_t> rows_asked;         // rows_per_wave the instances came with
   std::vector<fv::InstDesc> desc;          // host copy of the instance table
   std::vector<fv::WorkItem> items;         // kGroupWaves places per workgroup
   std::vector<uint64_t> rowmask;           // CFL lane mask per strip row (fv::WorkItem::mrow)
@@ -451,6 +452,15 @@ int graph_for(fivonagi_ctx* c, int G, hipGraphExec_t* out) {
   return 0;
 }
 
+// Mean rows per work item of an instance (heights differ when the split is
+// skewed).
+int mean_rows(const fivonagi_ctx* c, int inst) {
+  const auto& p = c->params[inst];
+  const int strips = (p.nx + fv::kStripCols - 1) / fv::kStripCols;
+  const int chunks = std::max(1, c->desc[inst].n_items / strips);
+  return (int)std::lround((double)p.ny / chunks);
+}
+
 // n attempts: single launches up to a phase-0 boundary, then graph replays
 // (graph_for: the exact length of a request up to kGraphChunk, else chunks
 // and the rest); fewer than 6 attempts run as single launches.
@@ -695,6 +705,7 @@ static int init_impl(fivonagi_ctx** out, const fivonagi_params* p, int n_inst,
   const size_t es = f64 ? sizeof(double) : sizeof(float);
   constexpr size_t kFieldFromHost = 1u << 20;
   c->params.assign(p, p + n_inst);
+  for (int k = 0; k < n_inst; ++k) c->rows_asked.push_back(p[k].rows_per_wave);
   c->desc.resize(n_inst);
   c->dt_seq_dev.assign(n_inst, nullptr);
   c->dt_seq_cap.assign(n_inst, 0);
@@ -902,73 +913,83 @@ int fivonagi_autotune(fivonagi_ctx* c, int trial_steps, int32_t* rows_out) {
   }
   c->collect_nx = 0;
   const int auto_h = auto_rows(c->params, c->cus * c->per_cu);
-  std::vector<int> cands = {auto_h, 8, 12, 16, 20, 24, 32, 40, 48, 64, 96, 128};
+  // (0 twice: the first trial of all also brings the device to its clock)
+  const std::vector<int> cands = {0, 0, auto_h, 8, 12, 16, 20, 24, 32, 40, 48, 64, 96, 128};
   hipEvent_t e0 = nullptr, e1 = nullptr;
   (void)hipEventCreate(&e0);
   (void)hipEventCreate(&e1);
+  // A split: the same rows per wave for every instance, or (rows 0) what each
+  // came with -- with the automatic skew that is the split a context starts
+  // with, whose height is found, not asked for -- and skew and cut.
+  struct Split { int rows; float skew; bool rotate; };
+  auto take = [&](const Split& s) {
+    for (int k = 0; k < c->n_inst; ++k)
+      c->params[k].rows_per_wave = s.rows > 0 ? s.rows : c->rows_asked[k];
+    c->skew = s.skew;
+    c->rotate = s.rotate;
+    build_items(c, s.rows > 0 ? s.rows : auto_h, s.skew, s.rotate);
+    return upload_items(c);
+  };
+  // the saved state in the saved buffer, and its counters
+  auto restore = [&]() -> int {
+    for (int k = 0; k < c->n_inst; ++k) {
+      const size_t n = (size_t)c->params[k].nx * c->params[k].ny;
+      for (int f = 0; f < 3; ++f)
+        HIP_TRY(hipMemcpyAsync(c->desc[k].q[saved[k].cur][f],
+                               (char*)keep[k] + (c->fp64 ? 8 : 4) * (size_t)f * n,
+                               (c->fp64 ? 8 : 4) * n, hipMemcpyDeviceToDevice, c->stream));
+    }
+    return write_ctls(c, saved);
+  };
   float best_ms = 1e30f;
-  int best_h = auto_h;
-  float best_skew = c->skew;
-  bool best_rot = c->rotate;
+  Split best{0, -1.0f, false};
   int rc = 0;
-  std::vector<fivonagi_params> orig = c->params;
-  // one candidate split: trial_steps attempts after 2 warm-up attempts
-  auto trial = [&](int h, float skew, bool rot) -> int {
-    for (auto& p : c->params) p.rows_per_wave = h;
-    build_items(c, h, skew, rot);
-    if (int r = upload_items(c)) return r;
+  // one split: trial_steps attempts from the saved state on (the time of a step
+  // depends on the state by some %), timed behind as many that are not (they
+  // capture the graphs the timed ones replay and keep the device busy before
+  // them: after an idle moment it runs slower for some ms) and those to phase 0
+  auto trial = [&](const Split& s) -> int {
+    if (int r = take(s)) return r;
+    if (int r = restore()) return r;
     std::vector<int64_t> tgt(c->n_inst, INT64_MAX);
     if (int r = write_targets(c, tgt)) return r;
-    if (int r = launch_attempts(c, 2)) return r;
+    if (int r = launch_attempts(c, (6 - c->attempts % 6) % 6)) return r;
+    if (int r = launch_attempts(c, trial_steps)) return r;
+    if (int r = launch_attempts(c, (6 - c->attempts % 6) % 6)) return r;
     (void)hipEventRecord(e0, c->stream);
     if (int r = launch_attempts(c, trial_steps)) return r;
     (void)hipEventRecord(e1, c->stream);
     (void)hipEventSynchronize(e1);
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, e0, e1);
-    if (ms < best_ms) { best_ms = ms; best_h = h; best_skew = skew; best_rot = rot; }
+    if (ms < best_ms) { best_ms = ms; best = s; }
     return 0;
   };
-  // heights with the automatic skew, then skews and level layouts at the
-  // best height
+  // the heights with the automatic skew, then skews and cuts at the best one
   for (int h : cands)
-    if ((rc = trial(h, -1.0f, false))) break;
+    if ((rc = trial({h, -1.0f, false}))) break;
   if (!rc) {
-    const int h = best_h;
+    const int h = best.rows;
     for (float sk : {0.0f, 0.25f, 0.5f, 0.75f})
       for (bool rot : {false, true}) {
         if (sk == 0.0f && rot) continue;
-        if (!rc) rc = trial(h, sk, rot);
+        if (!rc) rc = trial({h, sk, rot});
       }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  // restore: chosen work split, the saved state in the saved buffer, counters,
-  // data collection and dt sequences (build_items sets n_items afresh)
-  c->params = orig;
-  for (auto& p : c->params) p.rows_per_wave = best_h;
-  c->skew = best_skew;
-  c->rotate = best_rot;
+  // restore: chosen work split, data collection and dt sequences (build_items
+  // sets n_items afresh), state and counters; also after a trial that failed
   c->desc = desc_saved;
   c->collect_nx = collect_nx_saved;
-  build_items(c, best_h, c->skew, c->rotate);
-  int rc2 = upload_items(c);
-  for (int k = 0; k < c->n_inst; ++k) {
-    const size_t n = (size_t)c->params[k].nx * c->params[k].ny;
-    for (int f = 0; f < 3; ++f)
-      (void)hipMemcpyAsync(c->desc[k].q[saved[k].cur][f],
-                           (char*)keep[k] + (c->fp64 ? 8 : 4) * (size_t)f * n,
-                           (c->fp64 ? 8 : 4) * n, hipMemcpyDeviceToDevice, c->stream);
-  }
-  hipError_t es = hipStreamSynchronize(c->stream);
-  int rc3 = (rc || rc2 || es != hipSuccess) ? 0 : write_ctls(c, saved);
+  const int rc2 = take(best);
+  const int rc3 = restore();
   release();
   c->unlimited = false;
   if (rc) return rc;
   if (rc2) return rc2;
-  if (es != hipSuccess) return hip_fail(es, "hipStreamSynchronize (autotune)");
   if (rc3) return rc3;
-  if (rows_out) *rows_out = best_h;
+  if (rows_out) *rows_out = best.rows > 0 ? best.rows : mean_rows(c, 0);
   return 0;
 }
 
@@ -1261,11 +1282,7 @@ int fivonagi_info(fivonagi_ctx* c, int inst, fivonagi_info_t* info) {
   info->md_x = t.mdx;
   info->md_y = t.mdy;
   info->fp64 = c->fp64 ? 1 : 0;
-  // mean rows per work item (heights differ when the split is skewed)
-  const auto& p = c->params[inst];
-  const int strips = (p.nx + fv::kStripCols - 1) / fv::kStripCols;
-  const int chunks = std::max(1, c->desc[inst].n_items / strips);
-  info->rows_per_wave = (int)std::lround((double)p.ny / chunks);
+  info->rows_per_wave = mean_rows(c, inst);
   return 0;
 }
 

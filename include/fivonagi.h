@@ -135,12 +135,12 @@ int fivonagi_enqueue(fivonagi_ctx *ctx, int64_t nattempts);
 int fivonagi_sync(fivonagi_ctx *ctx);
 
 /* Autotuner (no counterpart in the reference): time trial_steps step
-   attempts for each candidate height of the work items (rows per wave), then
-   for each height skew at the best height, keep the fastest, and restore the
-   state and counters as they were.  The trials run with data collection and
+   attempts of the split the context was made with, of each candidate height of
+   the work items (rows per wave), then of each height skew and cut at the best
+   of them, keep the fastest, and restore the state and counters as they were.  The trials run with data collection and
    prescribed dt sequences switched off (both are restored, untouched).
-   rows_per_wave_out (may be NULL) receives the height; fivonagi_info reports
-   the skew. */
+   rows_per_wave_out (may be NULL) receives the height (of the split the
+   context was made with: its mean); fivonagi_info reports the skew. */
 int fivonagi_autotune(fivonagi_ctx *ctx, int trial_steps, int32_t *rows_per_wave_out);
 
 /* Work split (no counterpart in the reference): skew of the work-item

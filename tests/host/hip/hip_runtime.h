@@ -1,7 +1,7 @@
 // A stand-in for the HIP runtime on the host, for checks of what
 // fivonagi_amd/csrc/fv_runtime.cpp asks of it (tests/host/runtime_check.cpp).
 // Device memory is host memory (large blocks are address space alone, and copies
-// of that size move nothing); work on streams is done when they are waited
+// from and to them move nothing); work on streams is done when they are waited
 // for, launches and captured launches at once; a call can be made to fail.
 #ifndef FAKE_HIP_RUNTIME_H
 #define FAKE_HIP_RUNTIME_H
@@ -42,6 +42,12 @@ struct State {
 };
 inline int& device() { static thread_local int d = 0; return d; }
 inline State& st() { static State s; return s; }
+inline bool real(const void* p) {              // not in a large block
+  auto it = st().blocks.upper_bound((void*)p);
+  if (it == st().blocks.begin()) return true;
+  --it;
+  return it->second < kLarge || (const char*)p >= (const char*)it->first + it->second;
+}
 inline void launch(std::function<void()> f) {
   std::lock_guard<std::recursive_mutex> lk(st().mu);
   if (st().into) st().into->nodes.push_back(f);
@@ -89,19 +95,20 @@ inline hipError_t hipHostFree(void* p) { return hipFree(p); }
 
 inline hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
   FAKE_LOCK;
-  if (n < fake::kLarge) std::memmove(d, s, n);
+  if (fake::real(d) && fake::real(s)) std::memmove(d, s, n);
   return hipSuccess;
 }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t st) {
   FAKE_LOCK;
   auto& g = fake::st();
   if (g.fail_copy >= 0 && g.fail_copy-- == 0) return hipErrorInvalidValue;
-  if (n < fake::kLarge)
+  if (fake::real(d) && fake::real(s))
     (st ? st : &g.null_stream)->queued.push_back([=] { std::memmove(d, s, n); });
   return hipSuccess;
 }
 inline hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) {
-  if (n < fake::kLarge) std::memset(d, v, n);
+  FAKE_LOCK;
+  if (fake::real(d)) std::memset(d, v, n);
   return hipSuccess;
 }
 inline hipError_t hipMemset(void* d, int v, size_t n) { return hipMemsetAsync(d, v, n, nullptr); }

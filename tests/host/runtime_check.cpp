@@ -207,6 +207,37 @@ static int check_enqueue_under_capture() {
   return 0;
 }
 
+// The autotuner keeps the fastest of its trials: the split the context started
+// with where that is it -- also when another was chosen meanwhile -- and one of
+// the others where those are.
+static int check_autotune() {
+  std::vector<std::vector<fivonagi_params>> all = {
+      {grid(400, 400)}, {grid(1024, 1024)}, {grid(4096, 1024)}, {grid(8192, 2048)},
+      std::vector<fivonagi_params>(16, grid(512, 512)), {grid(200, 300), grid(700, 100)}};
+  all.back()[0].rows_per_wave = 21;
+  for (const auto& ps : all) {
+    fivonagi_ctx* c = context(ps);
+    fivonagi_info_t a, b;
+    int32_t rows = 0;
+    EXPECT(fivonagi_info(c, 0, &a) == 0, "%s", fivonagi_last_error());
+    for (int fastest : {0, 3, 0, 15, 0}) {
+      auto& g = fake::st();
+      g.elapsed.assign(100, 2.0f);
+      g.elapsed[fastest] = 1.0f;
+      g.asked = 0;
+      EXPECT(fivonagi_autotune(c, 20, &rows) == 0, "%s", fivonagi_last_error());
+      EXPECT(fivonagi_info(c, 0, &b) == 0, "%s", fivonagi_last_error());
+      const bool same = a.n_items == b.n_items && a.skew == b.skew && a.rotate == b.rotate;
+      EXPECT(fastest != 0 || same, "%dx%d: %d items skew %g, had %d skew %g", ps[0].nx, ps[0].ny,
+             b.n_items, b.skew, a.n_items, a.skew);
+      EXPECT(fastest != 3 || !same, "%dx%d: %d items", ps[0].nx, ps[0].ny, b.n_items);
+      EXPECT(rows > 0 && (fastest != 0 || rows == a.rows_per_wave), "%d rows", rows);
+    }
+    fivonagi_destroy(c);
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   int rc = 1;
@@ -214,6 +245,7 @@ int main(int argc, char** argv) {
   if (name == "download_error") rc = check_download_error();
   if (name == "download_device") rc = check_download_device();
   if (name == "enqueue_under_capture") rc = check_enqueue_under_capture();
+  if (name == "autotune") rc = check_autotune();
   if (rc == 0 && !fake::st().blocks.empty()) {
     std::printf("%zu blocks not freed\n", fake::st().blocks.size());
     rc = 1;
