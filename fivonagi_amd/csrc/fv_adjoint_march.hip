@@ -108,16 +108,18 @@ struct Vec2 {          // momentum parts
 // ga += kp[p] times family p of the waves of the interface to the left (kR
 // false) or right: the lane move is the operand of the multiply-add (which
 // the compiler forms only where a moved value has a single use).  The s_nop
-// covers the two wait states between a write of W and its read across lanes.
+// covers the two wait states between a write of W and its read across lanes;
+// g[6], which the Riemann transpose passes on to a lane move as it is, is written
+// first, so that it has its two as well.
 #define FV_FMAC7(dir)                                                                  \
   asm("s_nop 1\n\t"                                                                    \
+      "v_fmac_f32_dpp %6, %13, %16 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
       "v_fmac_f32_dpp %0, %7, %14 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"  \
       "v_fmac_f32_dpp %1, %8, %14 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"  \
       "v_fmac_f32_dpp %2, %9, %14 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"  \
       "v_fmac_f32_dpp %3, %10, %15 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
       "v_fmac_f32_dpp %4, %11, %15 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
-      "v_fmac_f32_dpp %5, %12, %15 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
-      "v_fmac_f32_dpp %6, %13, %16 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1"      \
+      "v_fmac_f32_dpp %5, %12, %15 " dir " row_mask:0xf bank_mask:0xf bound_ctrl:1"     \
       : "+&v"(ga.g[0]), "+&v"(ga.g[1]), "+&v"(ga.g[2]), "+&v"(ga.g[3]), "+&v"(ga.g[4]),     \
         "+&v"(ga.g[5]), "+&v"(ga.g[6])                                                   \
       : "v"(W.a1), "v"(W.w21), "v"(W.w31), "v"(W.a2), "v"(W.w22), "v"(W.w32), "v"(W.a3), \
@@ -341,7 +343,7 @@ __device__ __forceinline__ void reverse_item(const AdjDesc& D, const AdjItem& it
                                      y2q, y3q, un, ut);
     fvna::riemann(jx, hbeta, fx, vx);
     float dlx1, dlx2, dlx3;
-    dots_left(fx.w, dlx1, dlx2, dlx3);
+    dots_left<true>(fx.w, dlx1, dlx2, dlx3);
     const float drx1 = shl1(dlx1), drx2 = shl1(dlx2), drx3 = shl1(dlx3);
     float PX[3], MX[3];
     fvad::LimT limx;

@@ -37,20 +37,31 @@ __device__ __forceinline__ double shl1(double v) { return dpp64(v, 0); }
 // (a, shr1(a)), each multiply-add taking its neighbour operand by DPP.  The
 // compiler folds a cross-lane move only into two-operand forms it has before
 // register allocation, never into a multiply-add, so these are written out;
-// s_nop covers the two wait states between a VALU write and a DPP read.
+// s_nop covers the two wait states between a VALU write and a DPP read: before
+// and, where the products are moved between lanes by what the compiler makes of
+// the code behind (kMoved), behind.  (The step's only lane moves of them stand in
+// upwind_x, behind three instructions of its own.)
+#define FV_DOTS_LEFT(tail)                                                                        \
+  asm("s_nop 1\n\t"                                                                               \
+      "v_mul_f32_dpp %0, %5, %5 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"           \
+      "v_mul_f32_dpp %1, %8, %8 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"           \
+      "v_mul_f32_dpp %2, %9, %9 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"           \
+      "v_fmac_f32_dpp %0, %4, %4 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"          \
+      "v_fmac_f32_dpp %1, %7, %7 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"          \
+      "v_fmac_f32_dpp %0, %3, %3 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"          \
+      "v_fmac_f32_dpp %1, %6, %6 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1" tail         \
+      : "=&v"(d1), "=&v"(d2), "=&v"(d3)                                                           \
+      : "v"(w.a1), "v"(w.w21), "v"(w.w31), "v"(w.a2), "v"(w.w22), "v"(w.w32), "v"(w.a3))
+template <bool kMoved>
 __device__ __forceinline__ void dots_left(const fvna::WavesT<float>& w, float& d1, float& d2,
                                           float& d3) {
-  asm("s_nop 1\n\t"
-      "v_mul_f32_dpp %0, %5, %5 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-      "v_mul_f32_dpp %1, %8, %8 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-      "v_mul_f32_dpp %2, %9, %9 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-      "v_fmac_f32_dpp %0, %4, %4 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-      "v_fmac_f32_dpp %1, %7, %7 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-      "v_fmac_f32_dpp %0, %3, %3 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-      "v_fmac_f32_dpp %1, %6, %6 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1"
-      : "=&v"(d1), "=&v"(d2), "=&v"(d3)
-      : "v"(w.a1), "v"(w.w21), "v"(w.w31), "v"(w.a2), "v"(w.w22), "v"(w.w32), "v"(w.a3));
+  if constexpr (kMoved)
+    FV_DOTS_LEFT("\n\ts_nop 1");
+  else
+    FV_DOTS_LEFT("");
 }
+#undef FV_DOTS_LEFT
+template <bool kMoved>
 __device__ __forceinline__ void dots_left(const fvna::WavesT<double>& w, double& d1, double& d2,
                                           double& d3) {
   fvna::WavesT<double> l;

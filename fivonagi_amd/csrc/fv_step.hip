@@ -972,7 +972,7 @@ __device__ __forceinline__ void step_impl(const InstDesc* __restrict__ insts, co
     masked_max(mX, Sx, fx.L1, fx.L2);
     // W(k).W(k-1), with the waves of the interface to the left
     R dl1, dl2, dl3;
-    dots_left(fx.w, dl1, dl2, dl3);
+    dots_left<false>(fx.w, dl1, dl2, dl3);
     // W(k).W(k+1) is the right neighbour's W(k+1).W(k)
     R up1, up2, up3, nw1, nw2;
     upwind_x(fx, dl1, dl2, dl3, up1, up2, up3, nw1, nw2);
