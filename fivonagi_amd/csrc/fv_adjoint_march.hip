@@ -26,8 +26,9 @@
 // A wave runs one or more work items (row ranges of a strip) in turn; the
 // host groups them into waves of about equal cost.
 //
-// Bound by VALU issue: two waves per SIMD (255 registers each) keep it busy,
-// and HBM is a third used.  So the row is kept short: the limiter's transpose
+// Bound by VALU issue: two waves per SIMD (255 registers each) keep it busy 86%
+// of the step (counters, 2048x1024: 32.5 M issue quad-cycles, 61.4 us), and memory
+// moves 1.85 TB/s, 39% of what a copy reaches.  So the row is kept short: the limiter's transpose
 // takes factors formed with the forward values, neighbours' waves enter the
 // multiply-adds by DPP, rules of single rows and columns stand in branches,
 // and four rows per round leave no window moves: 872 -> about 680 VALU

@@ -227,9 +227,8 @@ std::vector<int> group_heights(int R, int max_waves) {
 // Row boundaries of one strip cut into `chunks` work items.  With skew > 0
 // the items get `levels` height levels (item j: level (j + rot) % levels)
 // with weights falling linearly from 1 + skew to 1 - skew (mean 1), so the
-// strip keeps its number of items, some taller and some shorter.  rot (the
-// strip index) spreads the levels a strip has one more item of evenly over
-// the strips, so every level has the same number of items.
+// strip keeps its number of items, some taller and some shorter.  (The in-step
+// cut takes rot = 0: the same rows in every strip.)
 std::vector<int> chunk_bounds(int ny, int chunks, float skew, int levels, int rot) {
   const int L = std::max(1, std::min(levels, chunks));
   std::vector<double> cum(chunks + 1, 0.0);

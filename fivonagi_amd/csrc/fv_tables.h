@@ -43,7 +43,8 @@ void host_inst(const fivonagi_params& q, bool f64, HostInst& h);
 void table_bytes(const std::vector<double>& v, bool f64, char* out);
 
 // Is cell (i, j) one the CFL reduction counts, for an instance's mask kind
-// (fv::CflMask) and bitmap?
+// (fv::CflMask) and bitmap?  (The lane masks are formed word by word; this is
+// what they are checked against.)
 bool cfl_counted(int cfl_mask, const std::vector<uint32_t>& fold_bits, int nx, int i, int j);
 
 // Rows per item of the in-step cut (see build_work): the smallest height
@@ -55,7 +56,7 @@ int auto_rows(const std::vector<fivonagi_params>& ps, long target_waves);
 std::vector<int> group_heights(int R, int max_waves);
 
 // Row boundaries of one strip cut into `chunks` work items (skewed heights,
-// `levels` levels, pattern rotated by rot).
+// `levels` levels, the first item at level rot; the in-step cut takes 0).
 std::vector<int> chunk_bounds(int ny, int chunks, float skew, int levels, int rot);
 
 // The work list of the step kernel.
@@ -75,7 +76,8 @@ struct WorkList {
 //   in step     one wave per item, every strip of an instance cut at the same
 //               rows, auto_h (or the instance's rows_per_wave) rows each.
 // cus, per_cu: the device's CUs and resident step waves per CU; skew < 0:
-// automatic, as the choice of the cut then is; else rotate picks running on.
+// automatic, as the choice of the cut then is; else rotate picks running on
+// (instances that ask for different rows_per_wave are always cut in step).
 // cell_bytes: bytes of state, in and out, per cell.
 void build_work(const std::vector<fivonagi_params>& ps, const std::vector<int>& cfl_mask,
                 const std::vector<std::vector<uint32_t>>& fold_bits, long cus, int per_cu,

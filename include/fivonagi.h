@@ -150,8 +150,9 @@ int fivonagi_autotune(fivonagi_ctx *ctx, int trial_steps, int32_t *rows_per_wave
    a SIMD finish; < 0 = automatic (0.5 when every SIMD starts its full
    complement of step waves, else 0).  With skew >= 0, rotate != 0 cuts the
    strips running on, one after another, into workgroups whose waves share
-   their seam rows; rotate = 0 cuts every strip of an instance at the same rows,
-   one wave per item.  Automatic: running on up to 256 MiB of state (in and
+   their seam rows; rotate = 0, or instances that ask for different
+   rows_per_wave, cuts every strip of an instance at the same rows, one wave per
+   item.  Automatic: running on up to 256 MiB of state (in and
    out), which the memory-side cache holds.  Which is fastest depends on the
    grid: fivonagi_autotune tries them.  Results do not depend on it. */
 int fivonagi_set_skew(fivonagi_ctx *ctx, double skew, int rotate);
