@@ -233,9 +233,11 @@ struct fivonagi_ctx {
   std::vector<fv::Ctl> ctl_cache;
   bool ctl_cache_ok = false;
   // pinned host memory: the control blocks as the settle kernel leaves them,
-  // then the targets the targets kernel reads
+  // then the targets the targets kernel reads.  Where there is none (h_ctl null)
+  // both are copied, the targets through d_targets
   fv::Ctl* h_ctl = nullptr;
   int64_t* h_targets = nullptr;
+  int64_t* d_targets = nullptr;
   bool targets_pending = false;            // a launch may still have to read h_targets
   hipEvent_t stage_ev[kStageSlots] = {};   // downloads: a slot of the staging buffer is full
 
@@ -352,7 +354,15 @@ int read_ctls(fivonagi_ctx* c, std::vector<fv::Ctl>& out) {
   HIP_TRY(fv_launch_settle(c->d_desc, c->n_inst, phase, c->h_ctl, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->targets_pending = false;
-  out.assign(c->h_ctl, c->h_ctl + c->n_inst);
+  if (c->h_ctl) {
+    out.assign(c->h_ctl, c->h_ctl + c->n_inst);
+  } else {
+    std::vector<fv::Ctl> both(2 * (size_t)c->n_inst);
+    HIP_TRY(hipMemcpy(both.data(), c->d_ctl, sizeof(fv::Ctl) * both.size(),
+                      hipMemcpyDeviceToHost));
+    out.resize(c->n_inst);
+    for (int k = 0; k < c->n_inst; ++k) out[k] = both[2 * (size_t)k + ((phase + 1) & 1)];
+  }
   c->ctl_cache = out;
   c->ctl_cache_ok = true;
   return 0;
@@ -526,7 +536,12 @@ int write_targets(fivonagi_ctx* c, const std::vector<int64_t>& tgt,
   if (cap != hipStreamCaptureStatusNone)
     return hip_fail(hipErrorStreamCaptureUnsupported, "stop conditions on a stream under capture");
   const int64_t* list = nullptr;
-  if (c->n_inst > 1) {
+  if (c->n_inst > 1 && !c->h_ctl) {
+    HIP_TRY(hipStreamSynchronize(c->stream));    // (the launch before may still read them)
+    HIP_TRY(hipMemcpy(c->d_targets, tgt.data(), sizeof(int64_t) * c->n_inst,
+                      hipMemcpyHostToDevice));
+    list = c->d_targets;
+  } else if (c->n_inst > 1) {
     if (c->targets_pending) HIP_TRY(hipStreamSynchronize(c->stream));
     std::copy(tgt.begin(), tgt.end(), c->h_targets);
     c->targets_pending = true;
@@ -740,11 +755,17 @@ static int init_impl(fivonagi_ctx** out, const fivonagi_params* p, int n_inst,
     c->h_ctl = (fv::Ctl*)pinned_pool().take_mirror();
     c->mirror_pooled = c->h_ctl != nullptr;
   }
-  if (!c->h_ctl) {
-    e = hipHostMalloc((void**)&c->h_ctl, mirror, hipHostMallocDefault);
-    if (e != hipSuccess) { delete c; return hip_fail(e, "hipHostMalloc"); }
+  if (!c->h_ctl &&
+      hipHostMalloc((void**)&c->h_ctl, mirror, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    c->h_ctl = nullptr;
   }
-  c->h_targets = (int64_t*)(c->h_ctl + n_inst);
+  if (c->h_ctl) {
+    c->h_targets = (int64_t*)(c->h_ctl + n_inst);
+  } else {
+    c->d_targets = (int64_t*)c->dalloc(sizeof(int64_t) * n_inst, &e);
+    if (e != hipSuccess) { delete c; return hip_fail(e, "hipMalloc targets"); }
+  }
   c->d_ctl = (fv::Ctl*)c->dalloc(sizeof(fv::Ctl) * 2 * n_inst, &e);
   if (e != hipSuccess) { delete c; return hip_fail(e, "hipMalloc ctl"); }
   c->d_sync = (fv::SyncSlots*)c->dalloc(sizeof(fv::SyncSlots) * 3 * n_inst, &e);

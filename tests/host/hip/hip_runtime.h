@@ -18,7 +18,8 @@
 #include <vector>
 
 typedef int hipError_t;
-constexpr hipError_t hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorInvalidHandle = 400,
+constexpr hipError_t hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2,
+                     hipErrorInvalidHandle = 400,
                      hipErrorStreamCaptureUnsupported = 900;
 
 namespace fake {
@@ -36,6 +37,7 @@ struct State {
   Stream* capturing = nullptr;                 // the stream under capture, by anyone
   Graph* into = nullptr;
   std::map<void*, size_t> blocks;
+  bool no_pinned = false;                      // hipHostMalloc fails
   int fail_copy = -1;                          // asynchronous copies until one fails (< 0: none)
   std::vector<float> elapsed;                  // hipEventElapsedTime's answers, in turn
   size_t asked = 0;
@@ -90,7 +92,9 @@ inline hipError_t hipFree(void* p) {
   return hipSuccess;
 }
 template <class T> hipError_t hipMalloc(T** p, size_t n) { return fake_alloc((void**)p, n); }
-inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return fake_alloc(p, n); }
+inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  return fake::st().no_pinned ? hipErrorOutOfMemory : fake_alloc(p, n);
+}
 inline hipError_t hipHostFree(void* p) { return hipFree(p); }
 
 inline hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {

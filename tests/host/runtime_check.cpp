@@ -4,6 +4,7 @@
 // always accepted.  Prints "ok", or what was wrong.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <string>
@@ -238,6 +239,28 @@ static int check_autotune() {
   return 0;
 }
 
+// A process with no pinned memory left: contexts are made, step (also when their
+// instances have different targets) and are read as with it.
+static int check_no_pinned_memory() {
+  fake::st().no_pinned = true;
+  for (int n : {1, 3, 50}) {
+    fivonagi_ctx* c = context(std::vector<fivonagi_params>(n, grid(64, 40)));
+    EXPECT(fivonagi_step(c, 5) == 0, "%s", fivonagi_last_error());
+    EXPECT(fivonagi_enqueue(c, 2) == 0, "%s", fivonagi_last_error());
+    EXPECT(fivonagi_step(c, 4) == 0, "%s", fivonagi_last_error());
+    std::vector<float> q(64 * 40);
+    for (int k = 0; k < n; ++k) {
+      int64_t acc = 0;
+      double T = 0.0;
+      EXPECT(fivonagi_collect(c, k, q.data(), nullptr, nullptr, &T, nullptr, &acc, nullptr) == 0,
+             "%s", fivonagi_last_error());
+      EXPECT(acc == 11 && std::abs(T - 11 * 0.005) < 1e-12, "%lld steps, T %g", (long long)acc, T);
+    }
+    fivonagi_destroy(c);
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   int rc = 1;
@@ -246,6 +269,7 @@ int main(int argc, char** argv) {
   if (name == "download_device") rc = check_download_device();
   if (name == "enqueue_under_capture") rc = check_enqueue_under_capture();
   if (name == "autotune") rc = check_autotune();
+  if (name == "no_pinned_memory") rc = check_no_pinned_memory();
   if (rc == 0 && !fake::st().blocks.empty()) {
     std::printf("%zu blocks not freed\n", fake::st().blocks.size());
     rc = 1;

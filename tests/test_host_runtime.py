@@ -24,7 +24,7 @@ def check(tmp_path_factory):
 
 @pytest.mark.parametrize("name", [
     "collect_without_ring", "download_error", "download_device",
-    "enqueue_under_capture", "autotune",
+    "enqueue_under_capture", "autotune", "no_pinned_memory",
 ])
 def test_runtime(check, name):
     r = subprocess.run([check, name], capture_output=True, text=True, timeout=120)
